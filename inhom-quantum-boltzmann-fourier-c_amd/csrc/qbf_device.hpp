@@ -21,6 +21,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 namespace qbf {
 
@@ -234,26 +235,21 @@ struct TwTab {
 	static constexpr int SIZE = 2 * P + T / P;
 };
 
-// Layout of the per-lane twiddle table w^(p u): float grids interleave it by lane, [u][p], so
-// that the G distinct addresses of one read fall into distinct banks; double grids keep it
-// [p][u] (their N = 64 kernels are register-bound, and the interleaved addressing costs them
-// registers).
-template <typename R, int G, int E>
-__device__ __forceinline__ constexpr int tw_lane(int p) { return sizeof(R) == 4 ? p : p * E; }
-template <typename R, int G>
-__device__ __forceinline__ constexpr int tw_step() { return sizeof(R) == 4 ? G : 1; }
+// The per-lane twiddle table w^(p u) is interleaved by lane, [u][p], so that the G distinct addresses
+// of one read fall into distinct banks: entry u of lane p at G u + p.  (FP64, [p][u]: a fifth of the
+// I3 kernel's LDS cycles were conflicts.)
 
 // Forward FFT of one line: interleaved layout in, blocked layout out.
 // twP[j] = (cos, sin)(2 pi j / P), j < P; the per-lane table (cos, sin)(2 pi p u / P) follows it
-// (in LDS, laid out as tw_lane / tw_step below).
+// (in LDS).
 template <typename R, int P, int G, int E>
 __device__ __forceinline__ void line_fwd(cx<R>* v, int p, const cx<R>* twP)
 {
 	dft<R, E, -1>(v);
 	if constexpr (G > 1) {
-		const cx<R>* tl = twP + P + tw_lane<R, G, E>(p) + opaque_zero();
+		const cx<R>* tl = twP + P + p + opaque_zero();
 #pragma unroll
-		for (int u = 1; u < E; u++) v[u] = cmulc<R>(v[u], tl[tw_step<R, G>() * u]);
+		for (int u = 1; u < E; u++) v[u] = cmulc<R>(v[u], tl[G * u]);
 #pragma unroll
 		for (int h = G / 2; h >= 1; h >>= 1) {
 			// DIF butterfly across lanes p, p^h:  lo: a + b,  hi: (a - b) * conj(w)
@@ -326,9 +322,9 @@ __device__ __forceinline__ void line_bwd(cx<R>* v, int p, const cx<R>* twP)
 				}
 			}
 		}
-		const cx<R>* tl = twP + P + tw_lane<R, G, E>(p) + opaque_zero();
+		const cx<R>* tl = twP + P + p + opaque_zero();
 #pragma unroll
-		for (int u = 1; u < E; u++) v[u] = cmul<R>(v[u], tl[tw_step<R, G>() * u]);
+		for (int u = 1; u < E; u++) v[u] = cmul<R>(v[u], tl[G * u]);
 	}
 	dft<R, E, +1>(v);
 }
@@ -342,63 +338,94 @@ __device__ __forceinline__ void line_bwd(cx<R>* v, int p, const cx<R>* twP)
 // rows times G consecutive columns: distinct because the pitch is G modulo LANES.  Writes /
 // reads of columns (C_b) hit LANES/G consecutive columns in G row blocks E rows apart: E*pitch
 // is a multiple of LANES, and the per-block skew LANES/G separates the blocks.
-template <typename R, class GE>
+//
+// SPLIT: a grid that does not fit in the 160 KiB of LDS whole (FP64 128 x 128: 256 KiB) goes through
+// it in two halves, real parts then imaginary parts: each half is the same grid of 8-byte elements,
+// and a thread's real parts are free to take the transposed ones while its imaginary parts wait, so no
+// staging registers are needed (two barriers more per exchange).  Against an exchange through a
+// per-workgroup slot in global memory (35 GB of HBM traffic per 16,384 K applications): FP64 Strang
+// step at N = 64, 16 cells, J = 32, M = 16, 110.8 -> 62.5 ms.
+template <typename R, class GE, bool SPLIT = false>
 struct Xpose {
-	static constexpr int LANES = 128 / (int)sizeof(cx<R>);
+	using El = typename std::conditional<SPLIT, R, cx<R>>::type;
+	static constexpr int LANES = 128 / (int)sizeof(El);
 	static constexpr int SKEW = LANES / GE::G;
 	static constexpr int SIZE = GE::P * GE::PITCH + GE::G * SKEW;
-	cx<R>* g0;
-	__device__ __forceinline__ cx<R>* gp() const { return g0 + opaque_zero(); }
+	El* g0;
+	__device__ __forceinline__ El* gp() const { return g0 + opaque_zero(); }
 	__device__ __forceinline__ int a(int row, int col) const { return row * GE::PITCH + col + (row / GE::E) * SKEW; }
-	// R_i (line = row) -> LDS
-	__device__ __forceinline__ void put_Ri(const cx<R>* v, int line, int p) const
+	static __device__ __forceinline__ void out(El& e, cx<R> v, int c)
 	{
-		cx<R>* g = gp();
-#pragma unroll
-		for (int s = 0; s < GE::E; s++) g[a(line, p + GE::G * s)] = v[s];
+		if constexpr (SPLIT) e = c ? v.y : v.x;
+		else e = v;
 	}
-	// LDS -> C_b (line = column)
-	__device__ __forceinline__ void get_Cb(cx<R>* v, int line, int p) const
+	static __device__ __forceinline__ void in(cx<R>& v, El e, int c)
 	{
-		const cx<R>* g = gp();
+		if constexpr (SPLIT) (c ? v.y : v.x) = e;
+		else v = e;
+	}
+	// put(g, c), get(g, c): this thread's writes and reads of half c (c = 0 only without SPLIT); the
+	// first barrier waits for the reads of the previous exchange
+	template <class Put, class Get>
+	__device__ __forceinline__ void pass(Put put, Get get) const
+	{
+#pragma unroll
+		for (int c = 0; c < (SPLIT ? 2 : 1); c++) {
+			__syncthreads();
+			put(gp(), c);
+			__syncthreads();
+			get((const El*)gp(), c);
+		}
+	}
+	// one thread's share of a line in the four layouts, NZ: without the padding zeros (the elements s
+	// with E/4 <= s < 3E/4, see padded_nonzero; read as zeros)
+	__device__ __forceinline__ void put_Ri(El* g, const cx<R>* v, int line, int p, int c) const
+	{
+#pragma unroll
+		for (int s = 0; s < GE::E; s++) out(g[a(line, p + GE::G * s)], v[s], c);
+	}
+	__device__ __forceinline__ void put_Cb(El* g, const cx<R>* v, int line, int p, int c) const
+	{
 		const int r0 = GE::E * brev<GE::G>(p);
 #pragma unroll
-		for (int u = 0; u < GE::E; u++) v[u] = g[a(r0 + u, line)];
+		for (int u = 0; u < GE::E; u++) out(g[a(r0 + u, line)], v[u], c);
 	}
-	// C_b (line = column) -> LDS
-	__device__ __forceinline__ void put_Cb(const cx<R>* v, int line, int p) const
+	__device__ __forceinline__ void get_Cb(const El* g, cx<R>* v, int line, int p, int c) const
 	{
-		cx<R>* g = gp();
 		const int r0 = GE::E * brev<GE::G>(p);
 #pragma unroll
-		for (int u = 0; u < GE::E; u++) g[a(r0 + u, line)] = v[u];
+		for (int u = 0; u < GE::E; u++) in(v[u], g[a(r0 + u, line)], c);
 	}
-	// one element of row `row`
-	__device__ __forceinline__ cx<R> get(int row, int col) const { return gp()[a(row, col)]; }
-	// LDS -> R_i (line = row)
-	__device__ __forceinline__ void get_Ri(cx<R>* v, int line, int p) const
+	__device__ __forceinline__ void get_Ri(const El* g, cx<R>* v, int line, int p, int c) const
 	{
-		const cx<R>* g = gp();
 #pragma unroll
-		for (int s = 0; s < GE::E; s++) v[s] = g[a(line, p + GE::G * s)];
+		for (int s = 0; s < GE::E; s++) in(v[s], g[a(line, p + GE::G * s)], c);
+	}
+	// R_i -> C_b and C_b -> R_i of the whole grid
+	__device__ __forceinline__ void RiCb(cx<R>* v, int line, int p) const
+	{
+		pass([&](El* g, int c) { put_Ri(g, v, line, p, c); }, [&](const El* g, int c) { get_Cb(g, v, line, p, c); });
+	}
+	__device__ __forceinline__ void CbRi(cx<R>* v, int line, int p) const
+	{
+		pass([&](El* g, int c) { put_Cb(g, v, line, p, c); }, [&](const El* g, int c) { get_Ri(g, v, line, p, c); });
 	}
 };
 
 // Fill the LDS twiddle tables from a global table of (cos, sin)(2 pi j / 256) in double:
-// twP[j] = w^j for j < P, the per-lane table w^(p*u) at twP[P + tw_lane(p) + tw_step * u], and the
+// twP[j] = w^j for j < P, the per-lane table w^(p*u) at twP[P + G u + p], and the
 // twiddles of the cross-lane stages at twP[2P + h + m] = w^(m P / 2h), m < h < G, kept apart so
 // that the lanes of one stage read consecutive entries; w = exp(2 pi i / P).
 // (load_twiddles_g: G lanes per line, filled by the NT threads of the workgroup)
 template <typename R, int P, int G, int NT>
 __device__ __forceinline__ void load_twiddles_g(cx<R>* twP, const double2* tw256)
 {
-	constexpr int E = P / G;
 	for (int j = threadIdx.x; j < 2 * P + G; j += NT) {
 		int k;
 		if (j < P) {
 			k = j;
 		} else if (j < 2 * P) {
-			k = sizeof(R) == 4 ? ((j - P) % G) * ((j - P) / G) : ((j - P) / E) * ((j - P) % E);
+			k = ((j - P) % G) * ((j - P) / G);
 		} else {
 			const int i = j - 2 * P;
 			int h = 1;

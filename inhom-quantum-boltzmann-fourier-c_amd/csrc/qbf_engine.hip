@@ -88,28 +88,28 @@ static int scratch_for_current_device(int* devOut, void** ptrOut)
 }
 
 // threads per workgroup for a padded P x P grid (P = 2N), and for an unpadded N x N grid
-// XG: exchange rows and columns through a per-workgroup global scratch slot instead of LDS
-// (an FP64 128 x 128 grid is 256 KiB, more than the 160 KiB of LDS of a CU)
+// SP: exchange rows and columns through LDS in two halves, real and imaginary parts (an FP64
+// 128 x 128 grid is 256 KiB, more than the 160 KiB of LDS of a CU)
 template <typename R, int N> struct Cfg;
-template <> struct Cfg<double, 16> { static constexpr int T = 128; static constexpr bool XG = false; };
-template <> struct Cfg<double, 32> { static constexpr int T = 256; static constexpr bool XG = false; };
-template <> struct Cfg<double, 64> { static constexpr int T = 1024; static constexpr bool XG = true; };
-template <> struct Cfg<float, 16> { static constexpr int T = 128; static constexpr bool XG = false; };
-template <> struct Cfg<float, 32> { static constexpr int T = 256; static constexpr bool XG = false; };
+template <> struct Cfg<double, 16> { static constexpr int T = 128; static constexpr bool SP = false; };
+template <> struct Cfg<double, 32> { static constexpr int T = 256; static constexpr bool SP = false; };
+template <> struct Cfg<double, 64> { static constexpr int T = 1024; static constexpr bool SP = true; };
+template <> struct Cfg<float, 16> { static constexpr int T = 128; static constexpr bool SP = false; };
+template <> struct Cfg<float, 32> { static constexpr int T = 256; static constexpr bool SP = false; };
 #ifndef QBF_F32_N64_THREADS
 #define QBF_F32_N64_THREADS 1024   // 512 also fits in registers (G = 4, E = 32)
 #endif
-template <> struct Cfg<float, 64> { static constexpr int T = QBF_F32_N64_THREADS; static constexpr bool XG = false; };
+template <> struct Cfg<float, 64> { static constexpr int T = QBF_F32_N64_THREADS; static constexpr bool SP = false; };
 // N = 128: the padded grids stay in global memory (qbf_big.hip: one workgroup of 512 threads per
-// grid, line sweeps; T must match big::TB, XG sizes the scratch per grid)
-template <> struct Cfg<double, 128> { static constexpr int T = 512; static constexpr bool XG = true; };
-template <> struct Cfg<float, 128> { static constexpr int T = 512; static constexpr bool XG = true; };
+// grid, line sweeps; T must match big::TB)
+template <> struct Cfg<double, 128> { static constexpr int T = 512; static constexpr bool SP = true; };
+template <> struct Cfg<float, 128> { static constexpr int T = 512; static constexpr bool SP = true; };
 template <int N> struct CfgNN;
-template <> struct CfgNN<16> { static constexpr int T = 64; static constexpr bool XG = false; };
-template <> struct CfgNN<32> { static constexpr int T = 128; static constexpr bool XG = false; };
-template <> struct CfgNN<64> { static constexpr int T = 256; static constexpr bool XG = false; };
-// an FP64 128 x 128 state grid (256 KiB) exchanges through global memory as well
-template <> struct CfgNN<128> { static constexpr int T = 1024; static constexpr bool XG = true; };
+template <> struct CfgNN<16> { static constexpr int T = 64; static constexpr bool SP = false; };
+template <> struct CfgNN<32> { static constexpr int T = 128; static constexpr bool SP = false; };
+template <> struct CfgNN<64> { static constexpr int T = 256; static constexpr bool SP = false; };
+// (a 128 x 128 FP64 state grid)
+template <> struct CfgNN<128> { static constexpr int T = 1024; static constexpr bool SP = true; };
 
 struct qbf_graph {
 	hipGraph_t graph = nullptr;
@@ -286,7 +286,7 @@ struct EngineT final : public qbf_engine {
 	static constexpr int P = 2 * N, NN = N * N, PP = P * P;
 	static constexpr int T = Cfg<R, N>::T;
 	static constexpr int TN = CfgNN<N>::T;
-	static constexpr bool XG = Cfg<R, N>::XG;
+	static constexpr bool SP = Cfg<R, N>::SP;
 	static constexpr bool BIG = N == 128;        // P = 256 kernels of qbf_big.hip, natural grid order
 	static_assert(!BIG || T == big::TB<R>, "launch size of the N = 128 kernels");
 	using GE = Geo<P, T>;
@@ -324,7 +324,7 @@ struct EngineT final : public qbf_engine {
 	{
 		for (DevBuf* b : {&i1[0].phi, &i1[0].psi1n, &i1[1].phi, &i1[1].psi1n, &i2p1, &i2p2, &i2pc, &i3p1, &i3p2n,
 			     &What, &Ahat, &Bhat, &Sbuf, &acc3, &Fscr, &xscr, &Wmid, &WF, &WF2, &Wt1, &Wt2, &src3, &Wpk,
-			     &WhatP, &reim, &Ipk, &xscrN, &Cf})
+			     &WhatP, &reim, &Ipk, &Cf})
 			b->lock = &liveGraphs;
 		return ensure_twiddles();
 	}
@@ -444,13 +444,12 @@ struct EngineT final : public qbf_engine {
 	}
 
 	// --------------------------------------------------------------- launches
-	// exchange scratch for nblocks workgroups (only for configurations that exchange through global memory)
+	// scratch grids of nblocks workgroups (N = 128, whose grids live in global memory)
 	int xs_for(int nblocks, void** xs, int gridsPerBlock = 1)
 	{
 		*xs = nullptr;
-		if (!XG) return 0;
-		const size_t per = BIG ? (size_t)PP * gridsPerBlock : (size_t)Xpose<R, GE>::SIZE;
-		int r = xscr.ensure((size_t)nblocks * per * sizeof(C));
+		if (!BIG) return 0;
+		int r = xscr.ensure((size_t)nblocks * PP * gridsPerBlock * sizeof(C));
 		if (r) return r;
 		*xs = xscr.p;
 		return 0;
@@ -469,13 +468,13 @@ struct EngineT final : public qbf_engine {
 		if (r) return r;
 		if constexpr (BIG) {
 			hipLaunchKernelGGL((k_padfft_big<R>), dim3(nb), dim3(T), 0, stream, a);
-		} else if constexpr (!XG && N == 64 && std::is_same<R, float>::value) {
+		} else if constexpr (N == 64 && std::is_same<R, float>::value) {
 			// one workgroup per CU, each looping over pairs of grids (measured: FP32 step 354 -> 335 ms at
 			// Nx = 512; 256 and 512 workgroups alike)
 			constexpr int WG = 256;
 			hipLaunchKernelGGL((k_padfft_loop<R, N, T>), dim3(nb < WG ? nb : WG), dim3(T), 0, stream, a);
 		} else {
-			hipLaunchKernelGGL((k_padfft<R, N, T, XG>), dim3(nb), dim3(T), 0, stream, a);
+			hipLaunchKernelGGL((k_padfft<R, N, T, SP>), dim3(nb), dim3(T), 0, stream, a);
 		}
 		HIPCHK(hipGetLastError());
 		return 0;
@@ -510,7 +509,7 @@ struct EngineT final : public qbf_engine {
 		if constexpr (BIG)
 			hipLaunchKernelGGL((k_i1acc_big<R>), dim3(ncell * ninst * nch), dim3(T), 0, stream, a);
 		else
-			hipLaunchKernelGGL((k_i1acc<R, N, T, XG>), dim3(ncell * ninst * nch), dim3(T), 0, stream, a);
+			hipLaunchKernelGGL((k_i1acc<R, N, T, SP>), dim3(ncell * ninst * nch), dim3(T), 0, stream, a);
 		HIPCHK(hipGetLastError());
 		*nchunk = nch;
 		return 0;
@@ -540,9 +539,9 @@ struct EngineT final : public qbf_engine {
 		if constexpr (BIG)
 			hipLaunchKernelGGL((k_i2acc_big<R>), dim3(ncell * ninst * nch), dim3(T), 0, stream, a);
 		else if (pair)
-			hipLaunchKernelGGL((k_i2acc<R, N, T, XG, true>), dim3(ncell * ninst * nch), dim3(T), 0, stream, a);
+			hipLaunchKernelGGL((k_i2acc<R, N, T, SP, true>), dim3(ncell * ninst * nch), dim3(T), 0, stream, a);
 		else
-			hipLaunchKernelGGL((k_i2acc<R, N, T, XG, false>), dim3(ncell * ninst * nch), dim3(T), 0, stream, a);
+			hipLaunchKernelGGL((k_i2acc<R, N, T, SP, false>), dim3(ncell * ninst * nch), dim3(T), 0, stream, a);
 		HIPCHK(hipGetLastError());
 		*nchunk = nch;
 		return 0;
@@ -561,7 +560,7 @@ struct EngineT final : public qbf_engine {
 		while (nchunk * ncell * nout < 1024) nchunk *= 2;
 		if (nchunk > nq) nchunk = nq;
 		if (nchunk < 1) nchunk = 1;
-		const size_t perQ = (size_t)ncell * nF * GB * (XG ? 2 : 1);
+		const size_t perQ = (size_t)ncell * nF * GB * (BIG || SP ? 2 : 1);
 		int qr = (int)(fBudget / perQ);
 		if (qr < 1) qr = 1;
 		if (qr > nq) qr = nq;
@@ -605,9 +604,9 @@ struct EngineT final : public qbf_engine {
 					return set_err(-1, "the BF16 split path exists for N = 64 only");
 				}
 			} else if (pair)
-				hipLaunchKernelGGL((k_i3acc<R, N, T, XG, true>), dim3(ncell * nout * nchunk), dim3(T), 0, stream, a);
+				hipLaunchKernelGGL((k_i3acc<R, N, T, SP, true>), dim3(ncell * nout * nchunk), dim3(T), 0, stream, a);
 			else
-				hipLaunchKernelGGL((k_i3acc<R, N, T, XG, false>), dim3(ncell * nout * nchunk), dim3(T), 0, stream, a);
+				hipLaunchKernelGGL((k_i3acc<R, N, T, SP, false>), dim3(ncell * nout * nchunk), dim3(T), 0, stream, a);
 			HIPCHK(hipGetLastError());
 			if (ee) {
 				HIPCHK(hipEventRecord(ee, stream));
@@ -713,7 +712,7 @@ struct EngineT final : public qbf_engine {
 		if constexpr (BIG)
 			hipLaunchKernelGGL((k_combine_big<R>), dim3(ncell * nout), dim3(T), 0, stream, a);
 		else
-			hipLaunchKernelGGL((k_combine<R, N, T, XG>), dim3(ncell * nout), dim3(T), 0, stream, a);
+			hipLaunchKernelGGL((k_combine<R, N, T, SP>), dim3(ncell * nout), dim3(T), 0, stream, a);
 		HIPCHK(hipGetLastError());
 		return 0;
 	}
@@ -986,41 +985,19 @@ struct EngineT final : public qbf_engine {
 	}
 
 	// --------------------------------------------------------------- state transforms and transport
-	// N x N state transforms; with XGN the exchange goes through xscrN, at most NB_XN grids a launch
-	static constexpr bool XGN = CfgNN<N>::XG;
-	static constexpr int NB_XN = 2048;
-	DevBuf xscrN;
+	// N x N state transforms
+	static constexpr bool SPN = CfgNN<N>::SP;
 	int phys2fourier(const double* in, int ngrid, double2* out) override
 	{
-		for (int g0 = 0; g0 < ngrid; g0 += NB_XN) {
-			const int ng = ngrid - g0 < NB_XN ? ngrid - g0 : NB_XN;
-			double2* xs = nullptr;
-			if (XGN) {
-				int r = xscrN.ensure(sizeof(double2) * (size_t)NB_XN * Xpose<double, Geo<N, TN>>::SIZE);
-				if (r) return r;
-				xs = xscrN.template as<double2>();
-			}
-			hipLaunchKernelGGL((k_phys2fourier<N, TN, XGN>), dim3(ng), dim3(TN), 0, stream, in + (size_t)g0 * NN,
-				out + (size_t)g0 * NN, g_tw256, ng, xs);
-			HIPCHK(hipGetLastError());
-		}
+		hipLaunchKernelGGL((k_phys2fourier<N, TN, SPN>), dim3(ngrid), dim3(TN), 0, stream, in, out, g_tw256, ngrid);
+		HIPCHK(hipGetLastError());
 		return 0;
 	}
 
 	int fourier2phys(const double2* in, int ngrid, double* out) override
 	{
-		for (int g0 = 0; g0 < ngrid; g0 += NB_XN) {
-			const int ng = ngrid - g0 < NB_XN ? ngrid - g0 : NB_XN;
-			double2* xs = nullptr;
-			if (XGN) {
-				int r = xscrN.ensure(sizeof(double2) * (size_t)NB_XN * Xpose<double, Geo<N, TN>>::SIZE);
-				if (r) return r;
-				xs = xscrN.template as<double2>();
-			}
-			hipLaunchKernelGGL((k_fourier2phys<N, TN, XGN>), dim3(ng), dim3(TN), 0, stream, in + (size_t)g0 * NN,
-				out + (size_t)g0 * NN, g_tw256, ng, xs);
-			HIPCHK(hipGetLastError());
-		}
+		hipLaunchKernelGGL((k_fourier2phys<N, TN, SPN>), dim3(ngrid), dim3(TN), 0, stream, in, out, g_tw256, ngrid);
+		HIPCHK(hipGetLastError());
 		return 0;
 	}
 

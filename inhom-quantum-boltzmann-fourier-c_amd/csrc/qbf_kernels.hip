@@ -28,11 +28,12 @@ __device__ __forceinline__ int unpad(int x)
 template <int E>
 __device__ __forceinline__ constexpr bool padded_nonzero(int s) { return s < E / 4 || s >= 3 * E / 4; }
 
-template <typename R, int N, class GE>
+template <typename R, int N, class GE, class XP>
 __device__ __forceinline__ void padfft_reg(cx<R>* v, const double2* __restrict__ src, const void* pre, int preKind,
-	const Xpose<R, GE>& X, const cx<R>* tw, int line, int p)
+	const XP& X, const cx<R>* tw, int line, int p)
 {
 	constexpr int G = GE::G, E = GE::E, P = GE::P;
+	using El = typename XP::El;
 	static_assert(2 * N == G * E, "padded line of 2N = G E elements");
 	const int kn = unpad<N>(line);
 	// base pointers formed here (opaque SGPRs): in a loop over terms the per-element 64-bit
@@ -62,42 +63,40 @@ __device__ __forceinline__ void padfft_reg(cx<R>* v, const double2* __restrict__
 		}
 		line_fwd<R, P, G, E>(v, p, tw);
 	}
-	__syncthreads();
-	if (kn >= 0) X.put_Cb(v, line, p);
-	__syncthreads();
+	X.pass([&](El* g, int c) { if (kn >= 0) X.put_Cb(g, v, line, p, c); },
+		[&](const El* g, int c) {
 #pragma unroll
-	for (int s = 0; s < E; s++) v[s] = padded_nonzero<E>(s) ? X.get(line, p + G * s) : czero<R>();
+			for (int s = 0; s < E; s++)
+				if (padded_nonzero<E>(s)) XP::in(v[s], g[X.a(line, p + G * s)], c);
+		});
+#pragma unroll
+	for (int s = 0; s < E; s++)
+		if (!padded_nonzero<E>(s)) v[s] = czero<R>();
 	line_fwd<R, P, G, E>(v, p, tw);
 }
 
 // R_b (physical) -> IFFT2 -> C_i (frequency)
-template <typename R, class GE>
-__device__ __forceinline__ void ifft2_reg(cx<R>* v, const Xpose<R, GE>& X, const cx<R>* tw, int line, int p)
+template <typename R, class GE, class XP>
+__device__ __forceinline__ void ifft2_reg(cx<R>* v, const XP& X, const cx<R>* tw, int line, int p)
 {
 	constexpr int G = GE::G, E = GE::E, P = GE::P;
 	line_bwd<R, P, G, E>(v, p, tw);
-	__syncthreads();
-	X.put_Ri(v, line, p);
-	__syncthreads();
-	X.get_Cb(v, line, p);
+	X.RiCb(v, line, p);
 	line_bwd<R, P, G, E>(v, p, tw);
 }
 
 // C_i (frequency) -> FFT2 -> R_b (physical)
-template <typename R, class GE>
-__device__ __forceinline__ void fft2_reg(cx<R>* v, const Xpose<R, GE>& X, const cx<R>* tw, int line, int p)
+template <typename R, class GE, class XP>
+__device__ __forceinline__ void fft2_reg(cx<R>* v, const XP& X, const cx<R>* tw, int line, int p)
 {
 	constexpr int G = GE::G, E = GE::E, P = GE::P;
 	line_fwd<R, P, G, E>(v, p, tw);
-	__syncthreads();
-	X.put_Cb(v, line, p);
-	__syncthreads();
-	X.get_Ri(v, line, p);
+	X.CbRi(v, line, p);
 	line_fwd<R, P, G, E>(v, p, tw);
 }
 
 // ---------------------------------------------------------------------------------------------
-template <typename R, int N, int T, bool XG>
+template <typename R, int N, int T, bool SP>
 __global__ __launch_bounds__(T) void k_padfft(PadFFTArgs a)
 {
 	// Two grids per workgroup: the N non-zero columns of grid 2b on lines 0..N-1 and those of grid
@@ -105,14 +104,14 @@ __global__ __launch_bounds__(T) void k_padfft(PadFFTArgs a)
 	// the LDS grid, columns 0..N-1 and N..2N-1; then a row pass per grid.
 	using GE = Geo<2 * N, T>;
 	constexpr int P = GE::P, E = GE::E, G = GE::G;
-	__shared__ cx<R> lds[XG ? 1 : Xpose<R, GE>::SIZE];
+	using XP = Xpose<R, GE, SP>;
+	__shared__ typename XP::El lds[XP::SIZE];
 	__shared__ cx<R> tw[TwTab<P, T>::SIZE];
 	load_twiddles<R, P, T>(tw, a.tw256);
-	cx<R>* xbuf = XG ? (cx<R>*)a.xs + (size_t)blockIdx.x * Xpose<R, GE>::SIZE : lds;
 	const int o0 = 2 * blockIdx.x;
 	const int line = threadIdx.x / G, p = threadIdx.x % G;
 	const int o = o0 + line / N, kn = line % N;
-	Xpose<R, GE> X{xbuf};
+	XP X{lds};
 	cx<R> v[E];
 	__syncthreads();
 	if (o < a.ngrid) {
@@ -140,28 +139,37 @@ __global__ __launch_bounds__(T) void k_padfft(PadFFTArgs a)
 			}
 		}
 		line_fwd<R, P, G, E>(v, p, tw);
-		X.put_Cb(v, line, p);
 	}
-	__syncthreads();
-	for (int g = 0; g < 2 && o0 + g < a.ngrid; g++) {
+	// the non-zero elements of this line's row of either grid
+	using El = typename XP::El;
+	cx<R> r[2][E / 2];
+	X.pass([&](El* g, int c) { if (o < a.ngrid) X.put_Cb(g, v, line, p, c); },
+		[&](const El* g, int c) {
 #pragma unroll
-		for (int s = 0; s < E; s++)
-			v[s] = padded_nonzero<E>(s) ? X.get(line, g * N + p + G * s - (s >= E / 4 ? N : 0)) : czero<R>();
+			for (int k = 0; k < 2; k++)
+#pragma unroll
+				for (int j = 0; j < E / 2; j++) XP::in(r[k][j], g[X.a(line, k * N + p + G * j)], c);
+		});
+#pragma unroll
+	for (int k = 0; k < 2; k++) {
+		if (o0 + k >= a.ngrid) break;
+#pragma unroll
+		for (int s = 0; s < E; s++) v[s] = padded_nonzero<E>(s) ? r[k][s < E / 4 ? s : s - E / 2] : czero<R>();
 		line_fwd<R, P, G, E>(v, p, tw);
-		store_native<R, GE>((cx<R>*)a.out + (size_t)(o0 + g) * (P * P), v);
+		store_native<R, GE>((cx<R>*)a.out + (size_t)(o0 + k) * (P * P), v);
 	}
 }
 
 // ---------------------------------------------------------------------------------------------
-template <typename R, int N, int T, bool XG>
+template <typename R, int N, int T, bool SP>
 __global__ __launch_bounds__(T) void k_i1acc(I1Args a)
 {
 	using GE = Geo<2 * N, T>;
 	constexpr int P = GE::P, E = GE::E;
-	__shared__ cx<R> lds[XG ? 1 : Xpose<R, GE>::SIZE];
+	using XP = Xpose<R, GE, SP>;
+	__shared__ typename XP::El lds[XP::SIZE];
 	__shared__ cx<R> tw[TwTab<P, T>::SIZE];
 	load_twiddles<R, P, T>(tw, a.tw256);
-	cx<R>* xbuf = XG ? (cx<R>*)a.xs + (size_t)blockIdx.x * Xpose<R, GE>::SIZE : lds;
 	const int lb = xcd_block();
 	const int chunk = lb % a.nchunk;
 	const int inst = (lb / a.nchunk) % a.ninst;
@@ -172,7 +180,7 @@ __global__ __launch_bounds__(T) void k_i1acc(I1Args a)
 	const double2* g = a.src + ((size_t)cell * a.nsrc + a.instSrc[inst]) * (N * N);
 	const cx<R>* Fh = (const cx<R>*)a.Fhat + ((size_t)cell * a.nFh + a.instFh[inst]) * (P * P);
 	const R fa = (R)a.fa, fb = (R)a.fb;
-	Xpose<R, GE> X{xbuf};
+	XP X{lds};
 	cx<R> acc[E], v[E];
 #pragma unroll
 	for (int s = 0; s < E; s++) acc[s] = czero<R>();
@@ -202,15 +210,15 @@ __global__ __launch_bounds__(T) void k_i1acc(I1Args a)
 // PAIR (f = g, real grids): FFT2(pad(psi1 f)) and FFT2(pad(psi2 f)) are the real and imaginary
 // parts of FFT2(pad((psi1 + i psi2) f)) when both are real (psi1, psi2 even, f the spectrum of a
 // real state with empty Nyquist lines), so one transform per term gives the product re * im.
-template <typename R, int N, int T, bool XG, bool PAIR>
+template <typename R, int N, int T, bool SP, bool PAIR>
 __global__ __launch_bounds__(T) void k_i2acc(I2Args a)
 {
 	using GE = Geo<2 * N, T>;
 	constexpr int P = GE::P, E = GE::E;
-	__shared__ cx<R> lds[XG ? 1 : Xpose<R, GE>::SIZE];
+	using XP = Xpose<R, GE, SP>;
+	__shared__ typename XP::El lds[XP::SIZE];
 	__shared__ cx<R> tw[TwTab<P, T>::SIZE];
 	load_twiddles<R, P, T>(tw, a.tw256);
-	cx<R>* xbuf = XG ? (cx<R>*)a.xs + (size_t)blockIdx.x * Xpose<R, GE>::SIZE : lds;
 	const int lb = xcd_block();
 	const int chunk = lb % a.nchunk;
 	const int inst = (lb / a.nchunk) % a.ninst;
@@ -220,7 +228,7 @@ __global__ __launch_bounds__(T) void k_i2acc(I2Args a)
 	const int line = threadIdx.x / GE::G, p = threadIdx.x % GE::G;
 	const double2* f = a.src + ((size_t)cell * a.nsrc + a.instF[inst]) * (N * N);
 	const double2* g = a.src + ((size_t)cell * a.nsrc + a.instG[inst]) * (N * N);
-	Xpose<R, GE> X{xbuf};
+	XP X{lds};
 	cx<R> acc[E], x1[E], v[E];
 #pragma unroll
 	for (int u = 0; u < E; u++) acc[u] = czero<R>();
@@ -251,15 +259,15 @@ __global__ __launch_bounds__(T) void k_i2acc(I2Args a)
 // application carries the two instances (S_2p H, S_2p+1 H) and acc += w_2p F_2p Y_2p + w_2p+1 F_2p+1 Y_2p+1
 // (instW[out][2 in], [2 in + 1]).  Exact for spectra of real states whose Nyquist lines vanish;
 // otherwise off by the dropped imaginary parts, which the host bounds before choosing it.
-template <typename R, int N, int T, bool XG, bool PAIR>
+template <typename R, int N, int T, bool SP, bool PAIR>
 __global__ __launch_bounds__(T) void k_i3acc(I3Args a)
 {
 	using GE = Geo<2 * N, T>;
 	constexpr int P = GE::P, E = GE::E;
-	__shared__ cx<R> lds[XG ? 1 : Xpose<R, GE>::SIZE];
+	using XP = Xpose<R, GE, SP>;
+	__shared__ typename XP::El lds[XP::SIZE];
 	__shared__ cx<R> tw[TwTab<P, T>::SIZE];
 	load_twiddles<R, P, T>(tw, a.tw256);
-	cx<R>* xbuf = XG ? (cx<R>*)a.xs + (size_t)blockIdx.x * Xpose<R, GE>::SIZE : lds;
 	const int lb = xcd_block();
 	const int chunk = lb % a.nchunk;
 	const int out = (lb / a.nchunk) % a.nout;
@@ -269,7 +277,7 @@ __global__ __launch_bounds__(T) void k_i3acc(I3Args a)
 	const int qa = (int)(((long long)chunk * a.nq) / a.nchunk);
 	const int qb = (int)(((long long)(chunk + 1) * a.nq) / a.nchunk);
 	cx<R>* accp = (cx<R>*)a.acc + (((size_t)cell * a.nout + out) * a.nchunk + chunk) * (P * P);
-	Xpose<R, GE> X{xbuf};
+	XP X{lds};
 	cx<R> acc[E], v[E];
 	if (a.accumulate) {
 		load_native<R, GE>(acc, accp);
@@ -346,13 +354,14 @@ __global__ __launch_bounds__(T) void k_padfft_loop(PadFFTArgs a)
 	using GE = Geo<2 * N, T>;
 	constexpr int P = GE::P, E = GE::E, G = GE::G;
 	constexpr int NZ = E / 2;                      // non-zero elements per lane in the column pass
-	__shared__ cx<R> lds[Xpose<R, GE>::SIZE];
+	using XP = Xpose<R, GE>;
+	__shared__ typename XP::El lds[XP::SIZE];
 	__shared__ cx<R> tw[TwTab<P, T>::SIZE];
 	load_twiddles<R, P, T>(tw, a.tw256);
 	const int line = threadIdx.x / G, p = threadIdx.x % G;
 	const int kn = line % N;
 	const int npair = (a.ngrid + 1) / 2;
-	Xpose<R, GE> X{lds};
+	XP X{lds};
 	cx<R> v[E];
 	double2 raw[NZ];
 	// the state values of pair b for this lane (the grid o = 2 b + line / N, if it exists)
@@ -398,14 +407,14 @@ __global__ __launch_bounds__(T) void k_padfft_loop(PadFFTArgs a)
 				}
 			}
 			line_fwd<R, P, G, E>(v, p, tw);
-			X.put_Cb(v, line, p);
+			X.put_Cb(X.gp(), v, line, p, 0);
 		}
 		__syncthreads();
 		if (b + (int)gridDim.x < npair) load(b + gridDim.x);
 		for (int g = 0; g < 2 && o0 + g < a.ngrid; g++) {
 #pragma unroll
 			for (int s = 0; s < E; s++)
-				v[s] = padded_nonzero<E>(s) ? X.get(line, g * N + p + G * s - (s >= E / 4 ? N : 0)) : czero<R>();
+				v[s] = padded_nonzero<E>(s) ? X.gp()[X.a(line, g * N + p + G * s - (s >= E / 4 ? N : 0))] : czero<R>();
 			line_fwd<R, P, G, E>(v, p, tw);
 			// non-temporal stores: the F grids of a launch (GiBs) are read back from HBM by the I3
 			// kernel, so they need not displace other lines from L2 (FP32 step 329 -> 327 ms)
@@ -421,20 +430,20 @@ __global__ __launch_bounds__(T) void k_padfft_loop(PadFFTArgs a)
 }
 
 // ---------------------------------------------------------------------------------------------
-template <typename R, int N, int T, bool XG>
+template <typename R, int N, int T, bool SP>
 __global__ __launch_bounds__(T) void k_combine(CombineArgs a)
 {
 	using GE = Geo<2 * N, T>;
 	constexpr int P = GE::P, E = GE::E, G = GE::G;
-	__shared__ cx<R> lds[XG ? 1 : Xpose<R, GE>::SIZE];
+	using XP = Xpose<R, GE, SP>;
+	__shared__ typename XP::El lds[XP::SIZE];
 	__shared__ cx<R> tw[TwTab<P, T>::SIZE];
 	load_twiddles<R, P, T>(tw, a.tw256);
-	cx<R>* xbuf = XG ? (cx<R>*)a.xs + (size_t)blockIdx.x * Xpose<R, GE>::SIZE : lds;
 	const int o = blockIdx.x % a.nout;
 	const int cell = blockIdx.x / a.nout;
 	const int line = threadIdx.x / G, p = threadIdx.x % G;
 	const int t = threadIdx.x;
-	Xpose<R, GE> X{xbuf};
+	XP X{lds};
 	cx<R> v[E];
 #pragma unroll
 	for (int u = 0; u < E; u++) v[u] = czero<R>();
@@ -524,21 +533,22 @@ __global__ void k_scaled_diff(const double2* __restrict__ a, const double2* __re
 // ---------------------------------------------------------------------------------------------
 // N x N transforms of the state (src/simulation.c:224-283): physical real -> Fourier / N^2
 // (full complex FFT of the real data), and Fourier -> unnormalised backward FFT -> real part.
-// XG: exchange through the per-workgroup slot xs + blockIdx.x * Xpose::SIZE (N = 128)
-template <int N, int T, bool XG>
+// SP: the grid goes through LDS in two halves (N = 128)
+template <int N, int T, bool SP>
 __global__ __launch_bounds__(T) void k_phys2fourier(const double* __restrict__ in, double2* __restrict__ out,
-	const double2* tw256, int ngrid, double2* xs)
+	const double2* tw256, int ngrid)
 {
 	using GE = Geo<N, T>;
 	constexpr int E = GE::E, G = GE::G;
-	__shared__ cx<double> lds[XG ? 1 : Xpose<double, GE>::SIZE];
+	using XP = Xpose<double, GE, SP>;
+	__shared__ typename XP::El lds[XP::SIZE];
 	__shared__ cx<double> tw[TwTab<N, T>::SIZE];
 	load_twiddles<double, N, T>(tw, tw256);
 	const int gi = blockIdx.x;
 	if (gi >= ngrid) return;
 	const int line = threadIdx.x / G, p = threadIdx.x % G;
 	const double* src = in + (size_t)gi * (N * N);
-	Xpose<double, GE> X{XG ? xs + (size_t)blockIdx.x * Xpose<double, GE>::SIZE : lds};
+	XP X{lds};
 	cx<double> v[E];
 #pragma unroll
 	for (int s = 0; s < E; s++) v[s] = make_double2(src[(p + G * s) * N + line], 0.0);
@@ -551,20 +561,21 @@ __global__ __launch_bounds__(T) void k_phys2fourier(const double* __restrict__ i
 	for (int u = 0; u < E; u++) dst[line * N + k0 + u] = make_double2(v[u].x * sc, v[u].y * sc);
 }
 
-template <int N, int T, bool XG>
+template <int N, int T, bool SP>
 __global__ __launch_bounds__(T) void k_fourier2phys(const double2* __restrict__ in, double* __restrict__ out,
-	const double2* tw256, int ngrid, double2* xs)
+	const double2* tw256, int ngrid)
 {
 	using GE = Geo<N, T>;
 	constexpr int E = GE::E, G = GE::G;
-	__shared__ cx<double> lds[XG ? 1 : Xpose<double, GE>::SIZE];
+	using XP = Xpose<double, GE, SP>;
+	__shared__ typename XP::El lds[XP::SIZE];
 	__shared__ cx<double> tw[TwTab<N, T>::SIZE];
 	load_twiddles<double, N, T>(tw, tw256);
 	const int gi = blockIdx.x;
 	if (gi >= ngrid) return;
 	const int line = threadIdx.x / G, p = threadIdx.x % G;
 	const double2* src = in + (size_t)gi * (N * N);
-	Xpose<double, GE> X{XG ? xs + (size_t)blockIdx.x * Xpose<double, GE>::SIZE : lds};
+	XP X{lds};
 	cx<double> v[E];
 	const int k0 = E * brev<G>(p);
 #pragma unroll
