@@ -12,7 +12,7 @@
 // The kernels take the argument blocks of the register-resident kernels of smaller N
 // (qbf_kernels.hip) with the same meaning; all their P x P grids (spectra, tables, partial sums)
 // are in natural order instead of the register-native order.
-#include "qbf_kernels.hip"
+#include "qbf_i3fold.hip"
 
 namespace qbf {
 namespace big {
@@ -401,6 +401,208 @@ __global__ __launch_bounds__(big::TB<R>) void k_i3acc_big(I3Args a)
 }
 
 // ---------------------------------------------------------------------------------------------
+// I3 part of CdInt over mirrored quadrature terms (I3FoldArgs; the identity and the sums are
+// k_i3fold's with one output, or one packed pair, per workgroup).  The four products of an output
+// with the components i go through the first two passes of k_i3acc_big together; the third forms
+// F_i Y_i and the mirror's b_i = S_j Y_i and takes the latter back through a row IFFT in the same
+// registers (packed pairs: b_2p + i b_2p+1), so that a mirrored term pair costs the scratch grids'
+// traffic of four products plus half a column pass over the box.
+template <typename R, bool PAIR>
+__global__ __launch_bounds__(big::TB<R>) void k_i3fold_big(I3FoldArgs a)
+{
+	using namespace big;
+	constexpr int T = TB<R>, L = T / G;         // L: lines per sweep
+	constexpr int NO = PAIR ? 2 : 4;            // outputs (packed pairs), grids of a cell
+	constexpr int NB = PAIR ? 2 : 4;            // mirror grids
+	// FP64: the sums are formed where they are written (sunk below the mirror's branch they would spill
+	// their operands; FP32 has the registers, and is faster with the loads free to move: 48.2 ms for the
+	// step of 32 cells against 54.1)
+	auto form = [](cx<R> x) { return sizeof(R) == 8 ? pin<R>(x) : x; };
+	__shared__ cx<R> tw[TW];
+	load_twiddles_g<R, P, G, T>(tw, a.tw256);
+	const int lb = xcd_block();
+	const int chunk = lb % a.nchunk;
+	const int j = (lb / a.nchunk) % NO;
+	const int cell = lb / (a.nchunk * NO);
+	const int qa = (int)(((long long)chunk * a.nq) / a.nchunk);
+	const int qb = (int)(((long long)(chunk + 1) * a.nq) / a.nchunk);
+	const int lt = threadIdx.x / G, p = threadIdx.x % G;
+	cx<R>* xs = (cx<R>*)a.xs + (size_t)blockIdx.x * (I3_NI * PP);
+	cx<R>* accp = (cx<R>*)a.acc + (((size_t)cell * NO + j) * a.nchunk + chunk) * PP;
+	using MB = MirrorBox<N, G, E, PAIR>;
+	constexpr int DN = MB::DL * MB::DL;
+	const long long dstep = (long long)NO * a.nchunk * a.nblk * DN;
+	cx<R>* Dp = (cx<R>*)a.D + NO * cell * dstep + (long long)((j * a.nchunk + chunk) * a.nblk + a.blk0 - 1) * DN;
+	const cx<R>* Sh = (const cx<R>*)a.Shat + (size_t)cell * NO * PP;
+	const cx<R>* Sj = Sh + (size_t)j * PP;
+	const int r0 = blk(p);
+	// columns of the mirror sums: the N of the box, and +N/2 with packed pairs (a last sweep in which
+	// one line is active)
+	constexpr int NSW = N / L + (PAIR ? 1 : 0);
+	auto mcol = [&](int sw) { return sw < N / L ? padrow(sw * L + lt) : (lt == 0 ? N / 2 : -1); };
+	int nb = 0;                                 // blocks begun
+	auto next_block = [&]() {
+		Dp += DN;
+		nb++;
+		for (int g = 0; g < NB; g++)
+			for (int e = threadIdx.x; e < DN; e += T) Dp[g * dstep + e] = czero<R>();
+	};
+	if (!a.accumulate) {
+#pragma unroll 1
+		for (int sw = 0; sw < P / L; sw++) {
+			cx<R>* row = accp + (sw * L + lt) * P + r0;
+#pragma unroll
+			for (int u = 0; u < E; u++) row[u] = czero<R>();
+		}
+	}
+	__syncthreads();
+#pragma unroll 1
+	for (int qq = qa; qq < qb; qq++) {
+		const cx<R>* Fq = (const cx<R>*)a.F + ((size_t)cell * a.nq + qq) * NO * PP;
+		const R* ps = (const R*)a.psi2n + (size_t)(a.q0 + qq) * PP;
+		const bool mir = a.q0 + qq < a.nmir;
+		if ((qq - qa) % DBLOCK<R> == 0 && (qq > qa || !a.resumeD)) {
+			// (barriers follow before D is read)
+			next_block();
+		}
+#pragma unroll 1
+		for (int sw = 0; sw < P / L; sw++) {
+			const int rb = (sw * L + lt) * P;
+#pragma unroll 1
+			for (int in = 0; in < 4; in++) {
+				const cx<R>* Sg = uni(Sh, (long long)(PAIR ? in >> 1 : in) * PP) + rb + r0;
+				const cx<R>* Fh = uni(Fq, (long long)j * PP) + rb + r0;
+				cx<R> v[E];
+				if constexpr (PAIR) {
+					const bool hi = in & 1;
+#pragma unroll
+					for (int u = 0; u < E; u++) v[u] = cscale<R>(Fh[u], hi ? Sg[u].y : Sg[u].x);
+				} else {
+#pragma unroll
+					for (int u = 0; u < E; u++) v[u] = cmul<R>(Sg[u], Fh[u]);
+				}
+				line_bwd<R, P, G, E>(v, p, tw);
+				cx<R>* x = uni(xs, (long long)in * PP) + rb + p;
+#pragma unroll
+				for (int s = 0; s < E; s++) x[G * s] = v[s];
+			}
+		}
+		__syncthreads();
+#pragma unroll 1
+		for (int sw = 0; sw < P / L; sw++) {
+			const int c = sw * L + lt;
+			R m[E];
+#pragma unroll
+			for (int s = 0; s < E; s++) m[s] = ps[(p + G * s) * P + c];
+#pragma unroll 1
+			for (int in = 0; in < 4; in++) {
+				cx<R>* x = uni(xs, (long long)in * PP) + r0 * P + c;
+				cx<R> v[E];
+#pragma unroll
+				for (int u = 0; u < E; u++) v[u] = x[u * P];
+				line_bwd<R, P, G, E>(v, p, tw);
+#pragma unroll
+				for (int s = 0; s < E; s++) {
+					v[s].x *= m[s];
+					v[s].y *= m[s];
+				}
+				line_fwd<R, P, G, E>(v, p, tw);
+#pragma unroll
+				for (int u = 0; u < E; u++) x[u * P] = v[u];
+			}
+		}
+		__syncthreads();
+#pragma unroll 1
+		for (int sw = 0; sw < P / L; sw++) {
+			const int rb = (sw * L + lt) * P;
+			cx<R> sum[E];
+			R bx[PAIR ? E : 1];
+#pragma unroll
+			for (int u = 0; u < E; u++) sum[u] = czero<R>();
+#pragma unroll 1
+			for (int in = 0; in < 4; in++) {
+				const cx<R>* x = uni((const cx<R>*)xs, (long long)in * PP) + rb + p;
+				cx<R> v[E];
+#pragma unroll
+				for (int s = 0; s < E; s++) v[s] = x[G * s];
+				line_fwd<R, P, G, E>(v, p, tw);
+				const R ei = eta_sgn<R>(in);
+				const cx<R>* Ff = uni(Fq, (long long)(PAIR ? in >> 1 : in) * PP) + rb + r0;
+				const cx<R>* Sg = uni(Sj, 0) + rb + r0;
+				const bool hi = in & 1;
+				if constexpr (PAIR) {
+					const R ea = eta_sgn<R>(2 * j);
+#pragma unroll
+					for (int u = 0; u < E; u++) {
+						const cx<R> f = Ff[u];
+						const R fv = ei * (hi ? f.y : f.x);
+						sum[u] = form(mk<R>(sum[u].x + fv * v[u].x, sum[u].y + fv * v[u].y));
+					}
+					if (!mir) continue;
+#pragma unroll
+					for (int u = 0; u < E; u++) {
+						const cx<R> s = Sg[u];
+						const R b = (ea * s.x) * v[u].x - s.y * v[u].y;
+						if (hi) v[u] = mk<R>(bx[u], b);
+						else bx[u] = b;
+					}
+					if (!hi) continue;
+				} else {
+					const R ej = eta_sgn<R>(j);
+#pragma unroll
+					for (int u = 0; u < E; u++) {
+						const cx<R> y = cmul<R>(Ff[u], v[u]);
+						sum[u] = form(mk<R>(sum[u].x + ei * y.x, sum[u].y + ei * y.y));
+					}
+					if (!mir) continue;
+#pragma unroll
+					for (int u = 0; u < E; u++) v[u] = cscale<R>(cmul<R>(Sg[u], v[u]), ej);
+				}
+				// row IFFT of the mirror grid into a scratch row that this line has read already
+				line_bwd<R, P, G, E>(v, p, tw);
+				cx<R>* y = uni(xs, (long long)(PAIR ? in >> 1 : in) * PP) + rb + p;
+#pragma unroll
+				for (int s = 0; s < E; s++)
+					if (padded_nonzero<E>(s) || (PAIR && s == E / 4)) y[G * s] = v[s];
+			}
+			cx<R>* row = accp + rb + r0;
+#pragma unroll
+			for (int u = 0; u < E; u++) row[u] = cadd<R>(row[u], sum[u]);
+		}
+		__syncthreads();
+		if (!mir) continue;
+		// columns of the box: IFFT along l, times conj(E(r)), into D
+		const cx<R>* ph = (const cx<R>*)a.phase + (size_t)(a.q0 + qq) * (2 * (N + 1));
+#pragma unroll 1
+		for (int sw = 0; sw < NSW; sw++) {
+			const int c = mcol(sw);
+			if (c < 0) continue;
+#pragma unroll 1
+			for (int g = 0; g < NB; g++) {
+				const cx<R>* x = uni((const cx<R>*)xs, (long long)g * PP) + r0 * P + c;
+				cx<R> v[E];
+#pragma unroll
+				for (int u = 0; u < E; u++) v[u] = x[u * P];
+				line_bwd<R, P, G, E>(v, p, tw);
+				cx<R>* d = uni(Dp, g * dstep) + MB::idx(c);
+				const cx<R> pk = ph[N + 1 + phase_idx<N>(c)];
+#pragma unroll
+				for (int s = 0; s < E; s++) {
+					if (!padded_nonzero<E>(s) && !(PAIR && s == E / 4)) continue;
+					const int l = p + G * s;
+					if (!padded_nonzero<E>(s) && l != N / 2) continue;
+					const cx<R> e = cmul<R>(ph[phase_idx<N>(l)], pk);
+					const int i = MB::idx(l) * MB::DL;
+					d[i] = cadd<R>(d[i], cmul<R>(v[s], e));
+				}
+			}
+		}
+		__syncthreads();
+	}
+	while (nb < a.nper) next_block();
+}
+
+// ---------------------------------------------------------------------------------------------
 // Combination, IFFT2, Extract and epilogue (CombineArgs as k_combine)
 template <typename R>
 __global__ __launch_bounds__(big::TB<R>) void k_combine_big(CombineArgs a)
@@ -450,6 +652,8 @@ __global__ __launch_bounds__(big::TB<R>) void k_combine_big(CombineArgs a)
 	// the N columns that the Extract keeps (src/grid.c:195-210)
 	const int comp = a.outComp[o];
 	const size_t cb = (size_t)cell * 4 * (N * N);
+	const double2* Dg = a.D ? a.D + (size_t)cell * a.Dcell + (a.Dpair ? comp >> 1 : comp) * a.Dstep : nullptr;
+	const double dc = a.Dcoef[o];
 #pragma unroll 1
 	for (int sw = 0; sw < N / L; sw++) {
 		const int kn = sw * L + lt;
@@ -464,6 +668,21 @@ __global__ __launch_bounds__(big::TB<R>) void k_combine_big(CombineArgs a)
 			if (ln < 0) continue;
 			const int e = ln * N + kn;
 			double vr = a.outScale * (double)v[s].x, vi = a.outScale * (double)v[s].y;
+			if (Dg) {
+				const int l = p + G * s;
+				double2 z;
+				if (a.Dpair) {
+					using MB = MirrorBox<N, G, E, true>;
+					const int i1 = MB::idx(l) * MB::DL + MB::idx(c);
+					const int i2 = MB::idx((P - l) % P) * MB::DL + MB::idx((P - c) % P);
+					z = unpack_hermitian<double>(Dg[i1], Dg[i2], comp & 1);
+				} else {
+					using MB = MirrorBox<N, G, E, false>;
+					z = Dg[MB::idx(l) * MB::DL + MB::idx(c)];
+				}
+				vr += dc * z.x;
+				vi += dc * z.y;
+			}
 			if (a.Wcb && comp > 0) {
 				// magnetic rotation 2 (B x w) (src/simulation.c:74-98)
 				const double* B = a.Bext + 3 * cell;

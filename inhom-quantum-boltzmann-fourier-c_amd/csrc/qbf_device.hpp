@@ -31,7 +31,7 @@ template <> struct cplx_sel<double> { using type = double2; };
 template <typename R> using cx = typename cplx_sel<R>::type;
 
 template <typename R>
-__device__ __forceinline__ cx<R> mk(R a, R b)
+__host__ __device__ __forceinline__ cx<R> mk(R a, R b)
 {
 	cx<R> r;
 	r.x = a;
@@ -217,6 +217,14 @@ __device__ __forceinline__ X* uni(X* p, long long off)
 	unsigned long long a = (unsigned long long)(p + off);
 	asm volatile("" : "+s"(a));
 	return (X*)(gX*)a;
+}
+
+// A VGPR copy of a lane index that the compiler cannot trace: addresses formed from it are not
+// hoisted out of the enclosing loop into (spilled) registers.
+__device__ __forceinline__ int opaque_lane(int x)
+{
+	asm volatile("" : "+v"(x));
+	return x;
 }
 
 // Materialise a value in VGPRs here: keeps a load unconditional (not sunk into a branch
@@ -456,5 +464,62 @@ __device__ __forceinline__ void load_native(cx<R>* v, const cx<R>* src)
 #pragma unroll
 	for (int u = 0; u < GE::E; u++) v[u] = uni(src, (long long)u * GE::T)[threadIdx.x];
 }
+
+// One array in global memory through a buffer descriptor: element t + u * T (u a compile-time
+// constant after unrolling) is a load with the lane's byte offset in a VGPR and u * T in a scalar
+// offset, so that many loads in flight need no 64-bit scalar address each (with uni() the kernels
+// that read five grids per term spilled about 60 SGPRs).  The base is opaque: loads through different
+// BufRefs of one array are not merged, and none is hoisted out of a loop that constructs it (kept in
+// registers from one use to the next, they spilled the accumulators).  n: elements of the array;
+// accesses beyond it read zero and are not written.
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+template <typename X>
+struct BufRef {
+	X* base;
+	__amdgpu_buffer_rsrc_t rs;
+	__device__ __forceinline__ BufRef(const X* p, int n)
+		: base((X*)p), rs(__builtin_amdgcn_make_buffer_rsrc((void*)uni(p, 0), 0, n * (int)sizeof(X), 0x00020000)) {}
+	// element voff + soff: voff per lane, soff uniform
+	__device__ __forceinline__ X get(int voff, int soff) const
+	{
+		const int vb = voff * (int)sizeof(X), sb = soff * (int)sizeof(X);
+		if constexpr (sizeof(X) == 4) return __builtin_bit_cast(X, __builtin_amdgcn_raw_buffer_load_b32(rs, vb, sb, 0));
+		else if constexpr (sizeof(X) == 8) return __builtin_bit_cast(X, __builtin_amdgcn_raw_buffer_load_b64(rs, vb, sb, 0));
+		else return __builtin_bit_cast(X, __builtin_amdgcn_raw_buffer_load_b128(rs, vb, sb, 0));
+	}
+	// 16-byte values go through a global store: a buffer_store_dwordx4 with a scalar offset reads its
+	// last data lanes late, and the compiler lets the next instruction overwrite the data registers
+	// (measured: lanes 12-15 of each 16 then stored the new values)
+	__device__ __forceinline__ void put(int voff, int soff, X x) const
+	{
+		const int vb = voff * (int)sizeof(X), sb = soff * (int)sizeof(X);
+		if constexpr (sizeof(X) == 4) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, x), rs, vb, sb, 0);
+		else if constexpr (sizeof(X) == 8) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, x), rs, vb, sb, 0);
+		else uni(base, soff)[voff] = x;
+	}
+};
+
+// fn(u, ld(u)) for u < E, the loads ld issued in batches of B with the next batch in flight while one
+// is used.  (Left to itself the compiler issued one load at a time in the kernels that are close to
+// their register limit, each waited for before the next: FP32 step at N = 64 244 ms against 206.)
+template <int E, int B, class Ld, class Fn>
+__device__ __forceinline__ void batched(Ld ld, Fn fn)
+{
+	static_assert(E % B == 0, "whole batches");
+	decltype(ld(0)) x[E];
+#pragma unroll
+	for (int k = 0; k < B; k++) x[k] = ld(k);
+#pragma unroll
+	for (int b = 0; b < E; b += B) {
+		if (b + B < E)
+#pragma unroll
+			for (int k = 0; k < B; k++) x[b + B + k] = ld(b + B + k);
+		__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+		for (int k = 0; k < B; k++) fn(b + k, x[b + k]);
+		__builtin_amdgcn_sched_barrier(0);
+	}
+}
+template <typename X, typename Y> struct Two { X a; Y b; };
 
 } // namespace qbf

@@ -20,9 +20,13 @@
 #include <stdio.h>
 #include <stdarg.h>
 #include <string.h>
+#include <algorithm>
+#include <atomic>
 #include <deque>
+#include <memory>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <unordered_map>
 #include <vector>
 #include <type_traits>
@@ -269,6 +273,24 @@ struct DevBuf {
 	template <typename X> X* as() const { return (X*)p; }
 };
 
+// fn(0 .. n-1), each over nel elements, on a few host threads (table checks and conversions); on the
+// calling thread alone where there is little to do or no thread can be started
+template <class F>
+void on_threads(unsigned n, int nel, F fn)
+{
+	std::atomic<unsigned> next{0};
+	auto work = [&]() { for (unsigned k; (k = next.fetch_add(1)) < n;) fn(k); };
+	std::vector<std::thread> th;
+	try {
+		const unsigned want = std::min({8u, std::max(1u, std::thread::hardware_concurrency()),
+			(unsigned)((unsigned long long)n * nel >> 19)});
+		for (unsigned t = 1; t < want; t++) th.emplace_back(work);
+	} catch (const std::exception&) {
+	}
+	work();
+	for (auto& t : th) t.join();
+}
+
 double2* g_tw256 = nullptr;
 
 int ensure_twiddles()
@@ -292,17 +314,21 @@ struct EngineT final : public qbf_engine {
 	using GE = Geo<P, T>;
 	using C = cx<R>;
 	static constexpr size_t GB = sizeof(C) * PP;    // bytes of one padded grid
+		// workgroups of the fold kernels resident at once: 16 waves a CU, 8 at FP64 N = 32 (registers)
+	static constexpr int FOLD_RES = BIG ? 512 : 256 * (16 * 64 / T) * FOLD_WPE<R, N> / 4;
 
 	struct I1Tab { int n = 0; DevBuf phi, psi1n; };
 	I1Tab i1[2];
 	int n2 = 0; DevBuf i2p1, i2p2, i2pc;
-	int n3 = 0; DevBuf i3p1, i3p2n;
+	// I3 terms in the order: one of each mirrored pair (n3m of them), terms without a mirror (up to
+	// n3f), the other ones of the pairs (see mirror_order and k_i3fold)
+	int n3 = 0, n3m = 0, n3f = 0; DevBuf i3p1, i3p2n, i3ph;
 	// BF16 hi/lo split path (precision QBF_BF16X3, N = 64): the I3 K-operator runs k_i3acc_mfma,
 	// whose psi2 table has its own order (i3p2m)
 	bool mfmaI3 = false;
 	DevBuf i3p2m;
 
-	DevBuf What, Ahat, Bhat, Sbuf, acc3, Fscr, xscr;
+	DevBuf What, Ahat, Bhat, Sbuf, acc3, Dmir, Dsum, Vsum, Fscr, xscr;
 	// Combination-term tables: each distinct table is uploaded once and its device copy reused, so
 	// that evaluations after the first of a configuration issue no host copy and no synchronisation
 	// (which makes the step capturable in a HIP graph).  At most TERM_CACHE tables are kept.
@@ -313,8 +339,7 @@ struct EngineT final : public qbf_engine {
 	static constexpr size_t TERM_CACHE = 64;
 	std::deque<TermTab> termCache;
 	DevBuf Wmid, WF, WF2, Wt1, Wt2, src3;
-	DevBuf Wpk, WhatP, reim, Ipk;     // paired path: packed spectra, their padded transforms, realness,
-	                                  // packed I1-type results
+	DevBuf Wpk, WhatP, reim;          // paired path: packed spectra, their padded transforms, realness
 	// device memory for the F grids of one I3 launch (it sets the quadrature terms per launch; the
 	// accumulators cross HBM once per launch).  Measured at N = 64 on 512 cells: FP32 8 GiB (64 terms
 	// per launch) 329 ms per step against 336 ms with 2 GiB; FP64 16 GiB no faster than 2 GiB.
@@ -322,9 +347,9 @@ struct EngineT final : public qbf_engine {
 
 	int init()
 	{
-		for (DevBuf* b : {&i1[0].phi, &i1[0].psi1n, &i1[1].phi, &i1[1].psi1n, &i2p1, &i2p2, &i2pc, &i3p1, &i3p2n,
-			     &What, &Ahat, &Bhat, &Sbuf, &acc3, &Fscr, &xscr, &Wmid, &WF, &WF2, &Wt1, &Wt2, &src3, &Wpk,
-			     &WhatP, &reim, &Ipk, &Cf})
+		for (DevBuf* b : {&i1[0].phi, &i1[0].psi1n, &i1[1].phi, &i1[1].psi1n, &i2p1, &i2p2, &i2pc, &i3p1, &i3p2n, &i3ph,
+			     &What, &Ahat, &Bhat, &Sbuf, &acc3, &Dmir, &Dsum, &Vsum, &Fscr, &xscr, &Wmid, &WF, &WF2, &Wt1, &Wt2, &src3, &Wpk,
+			     &WhatP, &reim, &Cf})
 			b->lock = &liveGraphs;
 		return ensure_twiddles();
 	}
@@ -415,12 +440,120 @@ struct EngineT final : public qbf_engine {
 		return 0;
 	}
 
+	// psi1 of one term is a translation phase: psi1(l, k) = psi1(l, 0) psi1(0, k), each factor
+	// multiplicative over the signed frequencies and conjugate under their reversal
+	static bool is_phase(const double* g, double tol)
+	{
+		struct Z { double x, y; };
+		auto at = [&](int l, int k) { const double* z = g + 2 * ((k & (N - 1)) + (size_t)N * (l & (N - 1))); return Z{z[0], z[1]}; };
+		auto mul = [](Z a, Z b) { return Z{a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x}; };
+		auto near = [&](Z a, Z b) { return fabs(a.x - b.x) <= tol && fabs(a.y - b.y) <= tol; };
+		if (!near(at(0, 0), Z{1, 0})) return false;
+		const Z el = at(1, 0), ek = at(0, 1);
+		for (int x = -N / 2; x < N / 2 - 1; x++)
+			if (!near(mul(at(x, 0), el), at(x + 1, 0)) || !near(mul(at(0, x), ek), at(0, x + 1))) return false;
+		for (int x = 1; x < N / 2; x++)
+			if (!near(at(-x, 0), Z{at(x, 0).x, -at(x, 0).y}) || !near(at(0, -x), Z{at(0, x).x, -at(0, x).y})) return false;
+		for (int l = 0; l < N; l++) {
+			const Z a = at(l, 0);
+			double worst = 0;
+			for (int k = 0; k < N; k++) {
+				const Z z = mul(a, at(0, k)), w = at(l, k);
+				const double d = fabs(z.x - w.x) + fabs(z.y - w.y);
+				worst = d <= worst ? worst : d;              // (a NaN stays)
+			}
+			if (!(worst <= 2 * tol)) return false;
+		}
+		return true;
+	}
+
+	// Order of the I3 terms: first a representative of every mirrored pair (psi1 a translation phase,
+	// its partner's psi1 the conjugate, psi2 equal; both to MIRROR_TOL, about ten times what the rounding of
+	// the tables' angles and weights leaves), then the terms without a partner, then the partners.
+	static constexpr double MIRROR_TOL = 4e-13;
+	static bool is_mirror(const double* a1, const double* a2, const double* b1, const double* b2)
+	{
+		const double scale = fabs(a2[0]) > 0 ? fabs(a2[0]) : 1.0;     // psi2's value at the origin sets its scale
+		auto near = [](const double* a, const double* b, int n, double sgn, double tol) {
+			double worst = 0;
+			for (int i = 0; i < n; i++) {
+				const double d = fabs(a[i] - ((i & 1) ? sgn : 1.0) * b[i]);
+				worst = d <= worst ? worst : d;                       // (a NaN stays)
+			}
+			return worst <= tol;
+		};
+		for (int l = 0; l < N; l++)
+			if (!near(a1 + 2 * N * l, b1 + 2 * N * l, 2 * N, -1.0, MIRROR_TOL)) return false;
+		for (int l = 0; l < P; l++)
+			if (!near(a2 + P * l, b2 + P * l, P, 1.0, MIRROR_TOL * scale)) return false;
+		return is_phase(a1, MIRROR_TOL);
+	}
+	static void mirror_order(unsigned num, const double* p1, const double* p2, std::vector<unsigned>& order, int* nmir,
+		int* nfold)
+	{
+		// candidates by psi1(1, 0), psi1(0, 1) and two values of psi2, then each pair in full
+		std::vector<std::pair<unsigned, unsigned>> cand;
+		std::vector<char> used(num, 0);
+		for (unsigned q = 0; q < num; q++) {
+			if (used[q]) continue;
+			const double *a1 = p1 + (size_t)q * 2 * NN, *a2 = p2 + (size_t)q * PP;
+			for (unsigned r = q + 1; r < num; r++) {
+				const double *b1 = p1 + (size_t)r * 2 * NN, *b2 = p2 + (size_t)r * PP;
+				if (used[r] || !(fabs(a1[2 * N + 1] + b1[2 * N + 1]) <= MIRROR_TOL) || !(fabs(a1[3] + b1[3]) <= MIRROR_TOL) ||
+					!(fabs(a2[1] - b2[1]) <= MIRROR_TOL * fabs(a2[0])) || !(fabs(a2[P] - b2[P]) <= MIRROR_TOL * fabs(a2[0])))
+					continue;
+				cand.push_back({q, r});
+				used[q] = used[r] = 1;
+				break;
+			}
+		}
+		std::vector<char> ok(cand.size(), 0);
+		on_threads((unsigned)cand.size(), PP, [&](unsigned k) {
+			const unsigned q = cand[k].first, r = cand[k].second;
+			ok[k] = is_mirror(p1 + (size_t)q * 2 * NN, p2 + (size_t)q * PP, p1 + (size_t)r * 2 * NN, p2 + (size_t)r * PP);
+		});
+		std::vector<unsigned> self, mir;
+		order.clear();
+		std::fill(used.begin(), used.end(), 0);
+		for (size_t k = 0; k < cand.size(); k++)
+			if (ok[k]) {
+				order.push_back(cand[k].first);
+				mir.push_back(cand[k].second);
+				used[cand[k].first] = used[cand[k].second] = 1;
+			}
+		*nmir = (int)order.size();
+		for (unsigned q = 0; q < num; q++)
+			if (!used[q]) self.push_back(q);
+		order.insert(order.end(), self.begin(), self.end());
+		*nfold = (int)order.size();
+		order.insert(order.end(), mir.begin(), mir.end());
+	}
+
 	int set_i3(unsigned num, const double* p1, const double* p2) override
 	{
+		std::vector<unsigned> order;
+		int nmir = 0, nfold = 0;
+		mirror_order(num, p1, p2, order, &nmir, &nfold);
 		std::vector<R> p2n((size_t)num * PP);
-		for (unsigned q = 0; q < num; q++) to_Ci_native(p2 + (size_t)q * PP, &p2n[(size_t)q * PP]);
-		int r = upload(i3p1, p1, sizeof(double2) * NN * (size_t)num);
+		std::unique_ptr<double[]> s1(new double[(size_t)num * 2 * NN]);
+		on_threads(num, PP, [&](unsigned q) {
+			memcpy(&s1[(size_t)q * 2 * NN], p1 + (size_t)order[q] * 2 * NN, sizeof(double) * 2 * NN);
+			to_Ci_native(p2 + (size_t)order[q] * PP, &p2n[(size_t)q * PP]);
+		});
+		int r = upload(i3p1, s1.get(), sizeof(double2) * NN * (size_t)num);
 		if (!r) r = upload(i3p2n, p2n.data(), sizeof(R) * p2n.size());
+		// conj(psi1) of the representatives along l and along k, frequencies 0 .. N/2, -N/2 .. -1 (+N/2: the
+		// conjugate of -N/2)
+		std::vector<C> ph;
+		ph.reserve((size_t)nmir * 2 * (N + 1));
+		for (int q = 0; q < nmir; q++)
+			for (int axis = 0; axis < 2; axis++)
+				for (int x = 0; x <= N; x++) {
+					const int f = x <= N / 2 ? x : x - 1;       // index on the N grid
+					const double* z = p1 + 2 * ((size_t)order[q] * NN + (size_t)f * (axis == 0 ? N : 1));
+					ph.push_back(mk<R>((R)z[0], (R)(x == N / 2 ? z[1] : -z[1])));
+				}
+		if (!r && nmir) r = upload(i3ph, ph.data(), sizeof(C) * ph.size());
 		if (r) return r;
 		if (mfmaI3) {
 			// k_i3acc_mfma's order: psi2 of row 16 w + i16, column 4 kq + r + 16 t at
@@ -434,12 +567,14 @@ struct EngineT final : public qbf_engine {
 							for (int ln = 0; ln < 64; ln++) {
 								const int l = 16 * w + (ln & 15), k = 4 * (ln >> 4) + rr + 16 * t;
 								p2m[(size_t)q * PP + ((w * 8 + t) * 4 + rr) * 64 + ln] =
-									(float)p2[(size_t)q * PP + k + (size_t)P * l];
+									(float)p2[(size_t)order[q] * PP + k + (size_t)P * l];
 							}
 			r = upload(i3p2m, p2m.data(), sizeof(float) * p2m.size());
 			if (r) return r;
 		}
 		n3 = (int)num;
+		n3m = nmir;
+		n3f = nfold;
 		return 0;
 	}
 
@@ -653,21 +788,6 @@ struct EngineT final : public qbf_engine {
 		return 0;
 	}
 
-	// Real parts and imaginary parts of packed I1-type results [ncell][npk][nch] into the slots
-	// dst[k][0], dst[k][1] of out [ncell][nout][nch] (imaginary part zero); -1: not used.
-	int unpack_real(const DevBuf& packed, int npk, DevBuf& out, int nout, int nch, const int (*dst)[2], int ncell)
-	{
-		int r = out.ensure((size_t)ncell * nout * nch * GB);
-		if (r) return r;
-		UnpackArgs a{};
-		a.in = packed.p; a.out = out.p; a.npk = npk; a.nout = nout; a.nch = nch;
-		for (int k = 0; k < npk; k++) { a.dst[k][0] = dst[k][0]; a.dst[k][1] = dst[k][1]; }
-		const long long n = (long long)ncell * npk * nch * PP;
-		hipLaunchKernelGGL((k_unpack_real<R>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, a, n, (long long)PP);
-		HIPCHK(hipGetLastError());
-		return 0;
-	}
-
 	// I3 part of CdInt on packed component pairs (see k_i3acc, PAIR); Wpk from pack_sources
 	int run_i3_pairs(int ncell, int* nchunk)
 	{
@@ -691,8 +811,91 @@ struct EngineT final : public qbf_engine {
 		return run_i3(Wpk.template as<double2>(), 3, 2, two, WhatP.p, 2, 4, ni, iF, iS, iH, iW, ncell, nchunk, true);
 	}
 
+	// elements of a mirror sum
+	static constexpr long long mirror_size(bool pair)
+	{
+		return BIG ? (long long)(N + pair) * (N + pair) : pair ? MirrorBox<N, GE::G, GE::E, true>::SIZE : MirrorBox<N, GE::G, GE::E, false>::SIZE;
+	}
+
+	// Term ranges of a fold launch over nq terms with wg workgroups per range: the fewest rounds of
+	// resident workgroups times terms per workgroup (a workgroup's start and end cost about half a term);
+	// the fewest ranges where that is equal.  10 cells, N = 64, FP32, 256 terms: 32 ranges, 5 full rounds
+	// of 8 terms; 8 ranges would be two rounds of 32, the second one a quarter full.
+	static int fold_chunks(int wg, int nq)
+	{
+		int best = 1;
+		double cost = INFINITY;
+		for (int c = 1; c <= nq && (c == 1 || (long long)wg * (c - 1) < 8LL * FOLD_RES); c++) {
+			const long long rounds = ((long long)wg * c + FOLD_RES - 1) / FOLD_RES;
+			const double x = (double)rounds * ((nq + c - 1) / c + 0.5);
+			if (x < cost * (1 - 1e-9)) {
+				cost = x;
+				best = c;
+			}
+		}
+		return best;
+	}
+
+	// I3 part of CdInt with one pass per mirrored pair of terms (see k_i3fold): acc3 [cell][no][*na] and
+	// Dmir [cell][no][*nd] partial sums, no = 4 outputs or (PAIR) 2 packed pairs.  F and S as run_i3 (src
+	// with nsrc grids per cell, the first no of them).
+	template <bool PAIR>
+	int run_i3_fold(const double2* src, int nsrc, const void* Shat, int ncell, int* na, int* nd)
+	{
+		// four workgroups per cell and term range: outputs, or (output pair, instance pair), of which the
+		// pair kernel at N = 128 takes both instance pairs
+		constexpr int NO = PAIR ? 2 : 4, NI = PAIR && !BIG ? 2 : 1;
+		const int nq = n3f;
+		const int wg = ncell * NO * NI;
+		const size_t perQ = (size_t)ncell * NO * GB * (BIG || SP ? 2 : 1);
+		int qr = (int)(fBudget / perQ);
+		if (qr < 1) qr = 1;
+		if (qr > nq) qr = nq;
+		const int nchunk = fold_chunks(wg, qr);
+		int r = Fscr.ensure((size_t)ncell * NO * GB * qr);
+		if (!r) r = acc3.ensure((size_t)ncell * NO * NI * nchunk * GB);
+		// blocks of mirror sums per workgroup (FP64: one over all launches)
+		const bool blocks = DBLOCK<R> < nq;
+		const int perLaunch = blocks ? ((qr + nchunk - 1) / nchunk + DBLOCK<R> - 1) / DBLOCK<R> : 0;
+		const int nblk = blocks ? perLaunch * ((nq + qr - 1) / qr) : 1;
+		if (!r) r = Dmir.ensure(sizeof(C) * (size_t)ncell * NO * NO * nchunk * nblk * mirror_size(PAIR));
+		if (r) return r;
+		const int slots[4] = {0, 1, 2, 3};
+		for (int q0 = 0; q0 < nq; q0 += qr) {
+			const int nqr = (nq - q0) < qr ? (nq - q0) : qr;
+			r = launch_padfft(src, nsrc, i3p1.p, 2, q0, nqr, NO, slots, Fscr.p, ncell);
+			if (r) return r;
+			I3FoldArgs a{};
+			a.Shat = Shat; a.F = Fscr.p; a.nq = nqr; a.q0 = q0; a.nmir = n3m;
+			a.psi2n = i3p2n.p; a.phase = i3ph.p;
+			a.nchunk = nchunk; a.accumulate = q0 > 0; a.acc = acc3.p; a.D = Dmir.p; a.nblk = nblk;
+			a.blk0 = blocks ? (q0 / qr) * perLaunch : (q0 > 0); a.resumeD = !blocks && q0 > 0;
+			a.nper = blocks ? perLaunch : (q0 == 0); a.tw256 = g_tw256;
+			r = xs_for(wg * nchunk, &a.xs, BIG ? big::I3_NI : 1);
+			if (r) return r;
+			hipEvent_t eb = nullptr, ee = nullptr;
+			if (prof && !tl_capturing && prof_begin(&eb, &ee) == 0) HIPCHK(hipEventRecord(eb, stream));
+			if constexpr (BIG)
+				hipLaunchKernelGGL((k_i3fold_big<R, PAIR>), dim3(wg * nchunk), dim3(T), 0, stream, a);
+			else if constexpr (PAIR)
+				hipLaunchKernelGGL((k_i3fold_pair<R, N, T, SP>), dim3(wg * nchunk), dim3(T), 0, stream, a);
+			else
+				hipLaunchKernelGGL((k_i3fold<R, N, T, SP>), dim3(wg * nchunk), dim3(T), 0, stream, a);
+			HIPCHK(hipGetLastError());
+			if (ee) {
+				HIPCHK(hipEventRecord(ee, stream));
+				profK += (PAIR ? 8.0 : 16.0) * ncell * nqr;
+			}
+		}
+		*na = NI * nchunk;
+		*nd = NO * nchunk * nblk;
+		return 0;
+	}
+
+	// Dm: the mirrored terms' sums (sum_mirror; null: none), added with the factors Dcoef
 	int launch_combine(std::vector<CTerm> (&tl)[4], int nout, const int* outComp, int ncell, double2* out,
-		const double2* base, const double2* Wcb, const double* Bext, double cf)
+		const double2* base, const double2* Wcb, const double* Bext, double cf, const double2* Dm = nullptr,
+		bool Dpair = false, const double* Dcoef = nullptr)
 	{
 		int maxT = 1;
 		for (int o = 0; o < nout; o++) maxT = (int)tl[o].size() > maxT ? (int)tl[o].size() : maxT;
@@ -706,6 +909,10 @@ struct EngineT final : public qbf_engine {
 		a.terms = dterms; a.maxTerms = maxT; a.nout = nout;
 		for (int o = 0; o < nout; o++) { a.nterm[o] = (int)tl[o].size(); a.outComp[o] = outComp[o]; }
 		a.outScale = 1.0; a.out = out; a.base = base; a.Wcb = Bext ? Wcb : nullptr; a.Bext = Bext; a.cf = cf;
+		a.D = Dm; a.Dpair = Dpair;
+		a.Dstep = mirror_size(Dpair);
+		a.Dcell = (Dpair ? 2 : 4) * a.Dstep;
+		for (int o = 0; o < nout; o++) a.Dcoef[o] = Dcoef ? Dcoef[o] : 0.0;
 		a.tw256 = g_tw256;
 		r = xs_for(ncell * nout, &a.xs);
 		if (r) return r;
@@ -761,13 +968,32 @@ struct EngineT final : public qbf_engine {
 		return 0;
 	}
 
-	// buf[o][c] (+)= ..., o < nouter, c < nch grids: buf[o][0] = sum_c buf[o][c]
-	int sum_chunks(void* buf, long long nouter, int nch)
+	// Dsum = the mirror sums from their nd parts per grid
+	int sum_mirror(bool pair, int ncell, int nd)
 	{
-		if (nch <= 1) return 0;
-		const long long n = nouter * PP;
-		hipLaunchKernelGGL((k_sum_chunks<R>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, (C*)buf, nch,
-			nouter, (long long)PP);
+		const long long nel = mirror_size(pair), n = nel * ncell * (pair ? 2 : 4);
+		int r = Dsum.ensure(sizeof(double2) * n);
+		if (r) return r;
+		const int ne = 256 / SUM_CL;
+		hipLaunchKernelGGL((k_sum_mirror<R>), dim3((unsigned)((n + ne - 1) / ne)), dim3(256), 0, stream, (const C*)Dmir.p,
+			Dsum.template as<double2>(), nd, n, nel);
+		HIPCHK(hipGetLastError());
+		return 0;
+	}
+
+	int assemble(AssembleArgs& a, int ncell)
+	{
+		int r = Vsum.ensure((size_t)ncell * 4 * GB);
+		if (r) return r;
+		const double p2 = 1.0 / ((double)P * P);
+		a.c2 = p2; a.c4 = p2 * p2; a.V = Vsum.p; a.PP = PP; a.n = (long long)ncell * PP;
+		int most = 1;
+		for (int n : {a.A ? a.nchA : 1, a.B ? a.nchB : 1, a.B ? a.nchS : 1, a.B ? a.nchAcc : 1}) most = n > most ? n : most;
+		// parts shared by 8 threads where there are more than 4 of them (few cells)
+		if (most > 4)
+			hipLaunchKernelGGL((k_assemble<R, 8>), dim3((unsigned)((a.n + 31) / 32)), dim3(256), 0, stream, a);
+		else
+			hipLaunchKernelGGL((k_assemble<R, 1>), dim3((unsigned)((a.n + 255) / 256)), dim3(256), 0, stream, a);
 		HIPCHK(hipGetLastError());
 		return 0;
 	}
@@ -812,35 +1038,33 @@ struct EngineT final : public qbf_engine {
 		}
 		if (cc) {
 			// -2 (2 w_tr - 1) ... : Fhat = FFT2(pad(-4 W0 + 2 delta)) = -4 What_0 + 2 (src/collision.c:220-227)
-			if (pair) {
-				// packed sources W2 + i W3 and W1 -> Ahat slots (1, 2) and (0, -)
-				const int srcs[2] = {1, 2}, dst[2][2] = {{1, 2}, {0, -1}};
-				r = launch_i1(QBF_TAB_I1, Wpk.template as<double2>(), 3, What.p, 4, -4.0, 2.0, 2, srcs, zero4, Ipk,
-					ncell, &nchA);
-				if (!r) r = unpack_real(Ipk, 2, Ahat, 3, nchA, dst, ncell);
-			} else {
-				const int g3[3] = {1, 2, 3};
-				r = launch_i1(QBF_TAB_I1, W, 4, What.p, 4, -4.0, 2.0, 3, g3, zero4, Ahat, ncell, &nchA);
-			}
+			// packed sources W2 + i W3 and W1, or components 1..3
+			const int srcs[2] = {1, 2}, g3[3] = {1, 2, 3};
+			r = pair ? launch_i1(QBF_TAB_I1, Wpk.template as<double2>(), 3, What.p, 4, -4.0, 2.0, 2, srcs, zero4, Ahat, ncell, &nchA)
+				: launch_i1(QBF_TAB_I1, W, 4, What.p, 4, -4.0, 2.0, 3, g3, zero4, Ahat, ncell, &nchA);
 			if (r) return r;
 		}
-		int nchunk = 1;
+		int nchAcc = 1, nD = 1;
+		// one pass per mirrored pair of I3 terms where the table has any (k_i3acc_mfma has no such form)
+		const bool fold = cd && n3m > 0 && !mfmaI3;
 		if (cd) {
-			// I4 with Fhat = FFT2(pad(2 W0 - delta)) = 2 What_0 - 1 (src/collision.c:127-134)
-			if (pair) {
-				// packed sources W0 + i W1 and W2 + i W3 -> Bhat slots (0, 1) and (2, 3)
-				const int srcs[2] = {0, 1}, dst[2][2] = {{0, 1}, {2, 3}};
-				r = launch_i1(QBF_TAB_I4, Wpk.template as<double2>(), 3, What.p, 4, 2.0, -1.0, 2, srcs, zero4, Ipk,
-					ncell, &nchB);
-				if (!r) r = unpack_real(Ipk, 2, Bhat, 4, nchB, dst, ncell);
-			} else {
-				r = launch_i1(QBF_TAB_I4, W, 4, What.p, 4, 2.0, -1.0, 4, all4, zero4, Bhat, ncell, &nchB);
-			}
+			// I4 with Fhat = FFT2(pad(2 W0 - delta)) = 2 What_0 - 1 (src/collision.c:127-134); packed sources
+			// W0 + i W1 and W2 + i W3, or the components
+			const int srcs[2] = {0, 1};
+			r = pair ? launch_i1(QBF_TAB_I4, Wpk.template as<double2>(), 3, What.p, 4, 2.0, -1.0, 2, srcs, zero4, Bhat, ncell, &nchB)
+				: launch_i1(QBF_TAB_I4, W, 4, What.p, 4, 2.0, -1.0, 4, all4, zero4, Bhat, ncell, &nchB);
 			// (no paired I2 kernel at N = 128: its I2 runs on the complex sources)
 			if (!r) r = launch_i2(W, 4, 4, all4, all4, Sbuf, ncell, &nchS, pair && !BIG);
 			if (r) return r;
-			if (pair) {
-				r = run_i3_pairs(ncell, &nchunk);
+			if (fold && pair) {
+				r = WhatP.ensure((size_t)ncell * 2 * GB);
+				const int two[2] = {0, 1};
+				if (!r) r = launch_padfft(Wpk.template as<double2>(), 3, nullptr, 0, 0, 1, 2, two, WhatP.p, ncell);
+				if (!r) r = run_i3_fold<true>(Wpk.template as<double2>(), 3, WhatP.p, ncell, &nchAcc, &nD);
+			} else if (fold) {
+				r = run_i3_fold<false>(W, 4, What.p, ncell, &nchAcc, &nD);
+			} else if (pair) {
+				r = run_i3_pairs(ncell, &nchAcc);
 			} else {
 				static const double eta[4] = {1, -1, -1, -1};
 				int ni[4] = {4, 4, 4, 4};
@@ -848,58 +1072,26 @@ struct EngineT final : public qbf_engine {
 				double iW[4][4];
 				for (int j = 0; j < 4; j++)
 					for (int i = 0; i < 4; i++) { iF[j][i] = i; iS[j][i] = i; iH[j][i] = j; iW[j][i] = eta[i]; }
-				r = run_i3(W, 4, 4, all4, What.p, 4, 4, ni, iF, iS, iH, iW, ncell, &nchunk);
+				r = run_i3(W, 4, 4, all4, What.p, 4, 4, ni, iF, iS, iH, iW, ncell, &nchAcc);
 			}
 			if (r) return r;
 		}
-		// the partial sums over term ranges are added here over the whole grid, so that k_combine
-		// reads one grid per term (added in the order k_combine used: the result is unchanged)
-		if (cc) r = sum_chunks(Ahat.p, 3LL * ncell, nchA);
-		if (!r && cd) r = sum_chunks(Bhat.p, 4LL * ncell, nchB);
-		if (!r && cd) r = sum_chunks(Sbuf.p, 4LL * ncell, nchS);
-		if (!r && cd) r = sum_chunks(acc3.p, 4LL * ncell, nchunk);
+		const bool pairAcc = fold && pair;
+		AssembleArgs a{};
+		a.What = What.p; a.A = cc ? Ahat.p : nullptr; a.B = cd ? Bhat.p : nullptr; a.S = Sbuf.p; a.acc = acc3.p;
+		a.nchA = nchA; a.nchB = nchB; a.nchS = nchS; a.nchAcc = nchAcc; a.pairAB = pair; a.pairAcc = pairAcc;
+		r = assemble(a, ncell);
+		if (!r && fold) r = sum_mirror(pairAcc, ncell, nD);
 		if (r) return r;
-		const double p2 = 1.0 / ((double)P * P), p4 = p2 * p2;
-		const double eta2[4] = {2, -2, -2, -2};
-		const C* Wh = What.template as<C>();
-		auto Wslot = [&](int c) { return (const void*)(Wh + (size_t)c * PP); };
 		std::vector<CTerm> tl[4];
-		if (cc) {
-			const C* A = Ahat.template as<C>();
-			const long long a3 = 3LL * nchA * PP;
-			auto As = [&](int s) { return (const void*)(A + (size_t)s * nchA * PP); };
-			// Cc_1 = I1(f,W2,W3) - I1(f,W3,W2), cyclic (src/collision.c:231-253); Ahat slot s <-> g = s+1
-			// (each slot: nchA partial sums over term ranges, added into the first)
-			tl[1].push_back(term(Wslot(3), c4, As(1), a3, p4, 1, 0, 1, PP));
-			tl[1].push_back(term(Wslot(2), c4, As(2), a3, -p4, 1, 0, 1, PP));
-			tl[2].push_back(term(Wslot(1), c4, As(2), a3, p4, 1, 0, 1, PP));
-			tl[2].push_back(term(Wslot(3), c4, As(0), a3, -p4, 1, 0, 1, PP));
-			tl[3].push_back(term(Wslot(2), c4, As(0), a3, p4, 1, 0, 1, PP));
-			tl[3].push_back(term(Wslot(1), c4, As(1), a3, -p4, 1, 0, 1, PP));
+		double Dcoef[4];
+		const double p2 = 1.0 / ((double)P * P), eta2[4] = {2, -2, -2, -2};
+		for (int j = 0; j < 4; j++) {
+			tl[j].push_back(term(nullptr, 0, Vsum.template as<C>() + (size_t)j * PP, 4LL * PP, 1.0));
+			Dcoef[j] = -eta2[j] * p2 * p2;
 		}
-		if (cd) {
-			const C* B = Bhat.template as<C>();
-			const C* S = Sbuf.template as<C>();
-			const C* A3 = acc3.template as<C>();
-			const long long b4 = 4LL * nchB * PP, s4 = 4LL * nchS * PP;
-			auto Bs = [&](int s) { return (const void*)(B + (size_t)s * nchB * PP); };
-			for (int j = 0; j < 4; j++) {
-				// I4 terms (src/collision.c:137-167)
-				tl[j].push_back(term(Wslot(0), c4, Bs(j), b4, eta2[j] * p4, 1, 0, 1, PP));
-				tl[j].push_back(term(Wslot(j), c4, Bs(0), b4, 2 * p4, 1, 0, 1, PP));
-				if (j == 0)
-					for (int jj = 0; jj < 4; jj++)
-						tl[j].push_back(term(Wslot(jj), c4, Bs(jj), b4, -2 * p4, 1, 0, 1, PP));
-				// I3 terms: -eta2_j / P^4 * sum_chunks acc_j (src/collision.c:110-121)
-				tl[j].push_back(term(nullptr, 0, A3 + (size_t)j * nchunk * PP, 4LL * nchunk * PP, -eta2[j] * p4,
-					1, 0, 1, PP));
-				// I2 terms: eta2_i / P^2 * (delta_j0 - What_j) .* S_i (src/collision.c:82-106)
-				for (int i = 0; i < 4; i++)
-					tl[j].push_back(term(Wslot(j), c4, S + (size_t)i * nchS * PP, s4, eta2[i] * p2, -1.0,
-						j == 0 ? 1.0 : 0.0, 1, PP));
-			}
-		}
-		return launch_combine(tl, 4, all4, ncell, out, base, Wcb, Bext, cf);
+		return launch_combine(tl, 4, all4, ncell, out, base, Wcb, Bext, cf, fold ? Dsum.template as<double2>() : nullptr,
+			pairAcc, Dcoef);
 	}
 
 	int collision_step(const double2* W, int ncell, double dt, const double* Bext, double2* Wnext) override

@@ -430,6 +430,27 @@ __global__ __launch_bounds__(T) void k_padfft_loop(PadFFTArgs a)
 }
 
 // ---------------------------------------------------------------------------------------------
+// Layout of a mirror sum D: the N x N box of the padded frequency grid (EDGE: and its +N/2 row and
+// column), in the C_i native order of the lines and elements that lie in it: line' (element s' of it)
+// at (s' * DL + line') * G + p.  N = 128 (k_i3fold_big): row' * DL + column'.
+template <int N, int G, int E, bool EDGE>
+struct MirrorBox {
+	static constexpr int DL = N + EDGE, DS = E / 2 + EDGE;
+	static constexpr int SIZE = DS * DL * G;
+	// padded line / row / column index 0 .. N/2 - 1 (EDGE: N/2), 3N/2 .. 2N - 1
+	static __device__ __forceinline__ constexpr int idx(int x) { return x < N / 2 + EDGE ? x : x - N + EDGE; }
+	static __device__ __forceinline__ constexpr int elem(int s) { return s < E / 4 + EDGE ? s : s - E / 2 + EDGE; }
+	// element (l, k) of the padded grid
+	static __device__ __forceinline__ int at(int l, int k) { return (elem(l / G) * DL + idx(k)) * G + l % G; }
+};
+
+// One of two Hermitian spectra a, b from their packed sum z = a + i b at r and w = (a + i b)(-r)
+template <typename R>
+__device__ __forceinline__ cx<R> unpack_hermitian(cx<R> z, cx<R> w, int second)
+{
+	return second ? mk<R>(R(0.5) * (z.y + w.y), R(0.5) * (w.x - z.x)) : mk<R>(R(0.5) * (z.x + w.x), R(0.5) * (z.y - w.y));
+}
+
 template <typename R, int N, int T, bool SP>
 __global__ __launch_bounds__(T) void k_combine(CombineArgs a)
 {
@@ -475,12 +496,27 @@ __global__ __launch_bounds__(T) void k_combine(CombineArgs a)
 	if (kn < 0) return;
 	const int comp = a.outComp[o];
 	const size_t cb = (size_t)cell * 4 * (N * N);
+	const double2* Dg = a.D ? a.D + (size_t)cell * a.Dcell + (a.Dpair ? comp >> 1 : comp) * a.Dstep : nullptr;
+	const double dc = a.Dcoef[o];
 #pragma unroll
 	for (int s = 0; s < E; s++) {
 		const int ln = unpad<N>(p + G * s);
 		if (ln < 0) continue;
 		const int e = ln * N + kn;
 		double vr = a.outScale * (double)v[s].x, vi = a.outScale * (double)v[s].y;
+		if (Dg) {
+			const int l = p + G * s;
+			double2 z;
+			if (a.Dpair) {
+				using MB = MirrorBox<N, G, E, true>;
+				z = unpack_hermitian<double>(Dg[MB::at(l, line)], Dg[MB::at((P - l) % P, (P - line) % P)], comp & 1);
+			} else {
+				using MB = MirrorBox<N, G, E, false>;
+				z = Dg[MB::at(l, line)];
+			}
+			vr += dc * z.x;
+			vi += dc * z.y;
+		}
 		if (a.Wcb && comp > 0) {
 			// magnetic rotation 2 (B x w) (src/simulation.c:74-98)
 			const double* B = a.Bext + 3 * cell;
@@ -504,18 +540,128 @@ __global__ __launch_bounds__(T) void k_combine(CombineArgs a)
 }
 
 // ---------------------------------------------------------------------------------------------
-// Partial sums over term ranges, buf[o][c][e] (c < nch): buf[o][0][e] = sum_c buf[o][c][e], added in
-// chunk order (the order k_combine adds them in when it is given the chunks)
+// Mirror sums of the I3 terms from their parts in[o][c][e] (c < nch, e < nel): out[o][e] = sum_c in[o][c][e]
+// in FP64.  SUM_CL threads share an element: thread c adds the parts c, c + SUM_CL, ..., and the sums
+// are added in order.
+constexpr int SUM_CL = 8;
 template <typename R>
-__global__ void k_sum_chunks(cx<R>* __restrict__ buf, int nch, long long nouter, long long PPe)
+__global__ __launch_bounds__(256) void k_sum_mirror(const cx<R>* __restrict__ in, double2* __restrict__ out, int nch,
+	long long n, long long nel)
 {
-	const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= nouter * PPe) return;
-	const long long o = i / PPe, e = i % PPe;
-	cx<R>* p = buf + o * nch * PPe + e;
-	cx<R> s = p[0];
-	for (int c = 1; c < nch; c++) s = cadd<R>(s, p[(long long)c * PPe]);
-	p[0] = s;
+	constexpr int CL = SUM_CL, NE = 256 / CL;
+	__shared__ double2 sh[CL][NE];
+	const int c = threadIdx.x / NE, x = threadIdx.x % NE;
+	const long long i = (long long)blockIdx.x * NE + x;
+	double2 s = make_double2(0, 0);
+	const cx<R>* p = in + (i / nel) * nch * nel + i % nel;
+	if (i < n)
+		for (int k = c; k < nch; k += CL) {
+			const cx<R> y = p[k * nel];
+			s = make_double2(s.x + (double)y.x, s.y + (double)y.y);
+		}
+	sh[c][x] = s;
+	__syncthreads();
+	if (c || i >= n) return;
+	for (int k = 1; k < CL; k++) s = make_double2(s.x + sh[k][x].x, s.y + sh[k][x].y);
+	out[i] = s;
+}
+
+// The physical-domain sum of a collision evaluation, per cell and grid element, V [cell][4][PP]
+// (src/collision.c:82-167, 220-253; the term sums of the integrals are linear):
+//   Cc: V_1 += c4 (W_3 A_2 - W_2 A_3) and cyclic,
+//   Cd: V_j += c4 (eta2_j W_0 B_j + 2 W_j B_0 - eta2_j acc_j) + c2 (delta_j0 - W_j) sum_i eta2_i S_i,
+//       V_0 -= 2 c4 sum_j W_j B_j.
+// Every input is read once for the four outputs; an input that comes as partial sums over term ranges
+// is added up here.  CL > 1: CL threads share an element and add the parts c, c + CL, ... (few cells,
+// many ranges).  Replaces four launches that added the parts in place and 70 grid reads a cell in
+// k_combine (memory-bound): one cell, N = 32, FP64, 128 ranges: 218 -> 60 us with what k_combine keeps.
+template <typename R, int CL>
+__global__ __launch_bounds__(256) void k_assemble(AssembleArgs a)
+{
+	constexpr int NE = 256 / CL, NI = 15;
+	__shared__ cx<R> sh[CL > 1 ? NI : 1][CL > 1 ? 256 : 1];
+	const int c = threadIdx.x / NE, x = threadIdx.x % NE;
+	const long long i = (long long)blockIdx.x * NE + x;
+	const bool in = i < a.n;
+	const long long cell = in ? i / a.PP : 0, e = in ? i % a.PP : 0;
+	// this thread's share of the sum of a slot's parts
+	auto part = [&](const void* buf, int nslot, int slot, int nch) {
+		const cx<R>* p = (const cx<R>*)buf + ((cell * nslot + slot) * nch) * a.PP + e;
+		cx<R> z = czero<R>();
+		for (int k = c; k < nch; k += CL) z = cadd<R>(z, p[(long long)k * a.PP]);
+		return z;
+	};
+	// 0..2: A of spin component 1..3, 3..6: B, 7..10: S, 11..14: acc
+	cx<R> g[NI];
+#pragma unroll
+	for (int k = 0; k < NI; k++) g[k] = czero<R>();
+	auto two = [&](int k, cx<R> z) {         // a packed slot: two real values
+		g[k] = mk<R>(z.x, R(0));
+		g[k + 1] = mk<R>(z.y, R(0));
+	};
+	if (in && a.A) {
+		if (a.pairAB) {
+			two(1, part(a.A, 2, 0, a.nchA));
+			g[0] = mk<R>(part(a.A, 2, 1, a.nchA).x, R(0));
+		} else {
+			for (int k = 0; k < 3; k++) g[k] = part(a.A, 3, k, a.nchA);
+		}
+	}
+	if (in && a.B) {
+		if (a.pairAB)
+			for (int k = 0; k < 2; k++) two(3 + 2 * k, part(a.B, 2, k, a.nchB));
+		else
+			for (int k = 0; k < 4; k++) g[3 + k] = part(a.B, 4, k, a.nchB);
+		for (int k = 0; k < 4; k++) g[7 + k] = part(a.S, 4, k, a.nchS);
+		if (a.pairAcc)
+			for (int k = 0; k < 2; k++) two(11 + 2 * k, part(a.acc, 2, k, a.nchAcc));
+		else
+			for (int k = 0; k < 4; k++) g[11 + k] = part(a.acc, 4, k, a.nchAcc);
+	}
+	if constexpr (CL > 1) {
+#pragma unroll
+		for (int k = 0; k < NI; k++) sh[k][threadIdx.x] = g[k];
+		__syncthreads();
+		for (int k = c; k < NI; k += CL) {
+			cx<R> z = sh[k][x];
+			for (int d = 1; d < CL; d++) z = cadd<R>(z, sh[k][d * NE + x]);
+			sh[k][x] = z;
+		}
+		__syncthreads();
+#pragma unroll
+		for (int k = 0; k < NI; k++) g[k] = sh[k][x];
+	}
+	if (!in) return;
+	const cx<R>* Wp = (const cx<R>*)a.What + cell * 4 * a.PP + e;
+	cx<R>* V = (cx<R>*)a.V + cell * 4 * a.PP + e;
+	cx<R> W[4];
+#pragma unroll
+	for (int k = 0; k < 4; k++) W[k] = Wp[(long long)k * a.PP];
+	const R c4 = (R)a.c4, c2 = (R)a.c2;
+#pragma unroll
+	for (int j = 0; j < 4; j++) {
+		if (CL > 1 && j != c) continue;
+		cx<R> v = czero<R>();
+		if (a.A && j > 0) {
+			const int k = j % 3 + 1, l = (j + 1) % 3 + 1;      // (j, k, l) cyclic
+			v = cscale<R>(csub<R>(cmul<R>(W[l], g[k - 1]), cmul<R>(W[k], g[l - 1])), c4);
+		}
+		if (a.B) {
+			const R e2 = j == 0 ? R(2) : R(-2);
+			cx<R> q = cscale<R>(csub<R>(cmul<R>(W[0], g[3 + j]), g[11 + j]), e2);
+			q = cadd<R>(q, cscale<R>(cmul<R>(W[j], g[3]), R(2)));
+			if (j == 0) {
+				cx<R> t = cmul<R>(W[0], g[3]);
+#pragma unroll
+				for (int k = 1; k < 4; k++) t = cadd<R>(t, cmul<R>(W[k], g[3 + k]));
+				q = csub<R>(q, cscale<R>(t, R(2)));
+			}
+			const cx<R> S = cscale<R>(csub<R>(csub<R>(csub<R>(g[7], g[8]), g[9]), g[10]), R(2));
+			const cx<R> w = mk<R>((j == 0 ? R(1) : R(0)) - W[j].x, -W[j].y);
+			v = cadd<R>(v, cadd<R>(cscale<R>(q, c4), cscale<R>(cmul<R>(w, S), c2)));
+		}
+		V[(long long)j * a.PP] = v;
+	}
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -967,25 +1113,6 @@ __global__ __launch_bounds__(256) void k_pack_pairs(const double2* __restrict__ 
 	}
 	const double2 x = W[(cell * 4 + 2 * pr) * NN + e], y = W[(cell * 4 + 2 * pr + 1) * NN + e];
 	Wp[i] = make_double2(x.x - y.y, x.y + y.x);
-}
-
-// Unpacking of packed I1-type results: in [ncell][npk][nch][PP] -> out [ncell][nout][nch][PP],
-// the real part of packed slot k into slot dst[k][0], the imaginary part into dst[k][1] (each with
-// imaginary part zero; -1: dropped).  n = ncell * npk * nch * PP.
-template <typename R>
-__global__ __launch_bounds__(256) void k_unpack_real(UnpackArgs a, long long n, long long PP)
-{
-	const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= n) return;
-	const long long e = i % PP, t = i / PP;
-	const int ch = (int)(t % a.nch), k = (int)((t / a.nch) % a.npk);
-	const long long cell = t / ((long long)a.nch * a.npk);
-	const cx<R> z = ((const cx<R>*)a.in)[i];
-	for (int c = 0; c < 2; c++) {
-		const int d = a.dst[k][c];
-		if (d >= 0)
-			((cx<R>*)a.out)[((cell * a.nout + d) * a.nch + ch) * PP + e] = mk<R>(c ? z.y : z.x, R(0));
-	}
 }
 
 // Largest |real part| and |imaginary part| of n complex values: out[block] = (max |re|, max |im|)

@@ -23,14 +23,6 @@ struct PadFFTArgs {
 	const double2* tw256;
 };
 
-// Unpacking of packed real results (paired path)
-struct UnpackArgs {
-	const void* in;
-	void* out;
-	int npk, nout, nch;
-	int dst[4][2];
-};
-
 // I1-type accumulation (I1 for Cc, I1 with FourierI4 tables for I4):
 //   out[cell][inst] = FFT2( sum_g psi1_g .* IFFT2( (fa*Fhat + fb) .* FFT2(pad(phi_g .* src)) ) )
 struct I1Args {
@@ -88,6 +80,26 @@ struct I3Args {
 	const double2* tw256;
 };
 
+// I3 part of CdInt over mirrored quadrature terms (k_i3fold, k_i3fold_big): the layouts of F, S and
+// psi2n are I3Args'; the results are partial sums acc [cell][no][na] and D [cell][no][nd] (no = 4 outputs, or 2
+// packed pairs; na and nd follow from the kernel's split, see there).
+struct I3FoldArgs {
+	void* xs;             // per-workgroup scratch grids (N = 128)
+	const void* Shat;     // [ncell][no][P*P] R_b native
+	const void* F;        // [ncell][nq][no][P*P] R_b native
+	int nq, q0;
+	int nmir;             // terms with an index below it stand for a mirrored pair
+	const void* psi2n;    // [nqTotal][P*P] C_i native
+	const void* phase;    // [nmir][2][N+1] conj(E) along l and along k, frequencies 0 .. N/2, -N/2 .. -1
+	int nchunk;
+	int accumulate;
+	void* acc;            // [ncell][no][na][P*P] R_b native
+	void* D;              // [ncell][no][nd] mirror sums (MirrorBox), nblk blocks of terms per workgroup
+	int nblk, blk0, nper; // blocks in all launches, of the launches before this one, and of this one
+	int resumeD;          // the first terms continue block blk0 - 1
+	const double2* tw256;
+};
+
 // One product term of the physical-domain combination:
 //   coef * (X ? ax*X + bx : 1) .* (Y ? sum_{n<nsum} Y[n*ysum] : 1)
 struct CTerm {
@@ -115,7 +127,30 @@ struct CombineArgs {
 	const double2* Wcb;   // [ncell][4][N*N] or null (no magnetic rotation)
 	const double* Bext;   // [ncell][3] (used when Wcb != null)
 	double cf;
+	// frequency-space sums of the mirrored I3 terms (k_sum_mirror), added to the extracted value with the
+	// factor Dcoef[o]; null: none.  Dpair 0: [cell][4], the component's grid; 1: [cell][2], packed
+	// pairs of Hermitian spectra.  Dstep: elements between the grids of a cell, Dcell: between cells.
+	const double2* D;
+	int Dpair;
+	long long Dcell, Dstep;
+	double Dcoef[4];
 	const double2* tw256;
+};
+
+// Physical-domain sum of a collision evaluation (k_assemble), all grids in R_b native order.  pairAB:
+// A [ncell][2][nchA] = (A_2 + i A_3, A_1), B [ncell][2][nchB] = (B_0 + i B_1, B_2 + i B_3) packed real
+// grids; otherwise A [ncell][3][nchA], B [ncell][4][nchB].  pairAcc: acc [ncell][2][nchAcc] packed.
+struct AssembleArgs {
+	const void* What;     // [ncell][4]
+	const void* A;        // null: no Cc
+	const void* B;        // null: no Cd
+	const void* S;        // [ncell][4][nchS]
+	const void* acc;      // [ncell][4 or 2][nchAcc]
+	int nchA, nchB, nchS, nchAcc;
+	int pairAB, pairAcc;
+	double c4, c2;
+	void* V;              // [ncell][4]
+	long long n, PP;      // n = ncell * PP
 };
 
 } // namespace qbf
