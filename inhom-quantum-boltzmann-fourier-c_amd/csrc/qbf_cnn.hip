@@ -12,7 +12,7 @@
 // channels; K = 9 taps x input channels.
 // MFMA operand layout (16 x 16 x 32): lane l holds A[l%16][8*(l/16) .. +7],
 // B[8*(l/16) .. +7][l%16], and the result D[4*(l/16) + r][l%16], r < 4.
-// The weight gradient (a reduction over all pixels) runs on the VALU in fp32.
+// The weight gradient (a reduction over all pixels) runs there too, over pixels.
 // Options (qbf_cnn_configure): a dilation d_l per layer (tap offsets (ky-1, kx-1) * d_l), and
 // per-cell normalisation: a_b = max |x[b][0]| (trace channel); the network sees x / a_b and the
 // constant channel iscale * a_b, its output is scaled by oscale * a_b^2, and the training loss
@@ -253,79 +253,179 @@ __global__ __launch_bounds__(64 * CROWS) __attribute__((amdgpu_waves_per_eu(4)))
 		}
 }
 
-// Weight and bias gradients on the VALU, per workgroup:
+// Weight and bias gradients on the matrix cores, per workgroup:
 //   part[blk][(t * CO + co) * CI + ci] = sum_p dz[p][co] * x[p + dil off_t][ci],
-//   part[blk][9 CO CI + co] = sum_p dz[p][co]   (p over the workgroup's rows)
+//   part[blk][9 CO CI + co] = sum_p dz[p][co]   (p over the workgroup's pixels)
 // summed over the workgroups in a fixed order by k_wgrad_reduce (no atomics: the gradients are the
-// same bit for bit from run to run).  One workgroup per (image, block of ROWS rows); thread (co,
-// 16-channel ci block) keeps 9 x 16 accumulators; the three rows of x that a row of dz meets and that
-// row of dz are staged in LDS (periodic in x; the x rows with a pitch of CI + 4 floats, so that a
-// thread reads its 16 channels as four aligned 16-byte words).
+// same bit for bit from run to run).  The contraction runs over pixels: v_mfma_f32_16x16x32_bf16 with
+// A = dz^T (16 channels co x 32 pixels) and B = x (32 pixels x 16 channels ci), products of bf16 values
+// summed in fp32, as the sums over pixels on the VALU were.
+// One workgroup of 8 waves per (image, 64-pixel segment, block of rows): a wave keeps the 9 taps (5
+// and 4 where the layer has fewer tiles) of 32 x 16 channels in its accumulators.  The rows are staged
+// in LDS by channel, pixels contiguous, so that a fragment is one 16-byte read: x three times, shifted
+// by the three kx (fragments of a shifted row would not be aligned), in a ring of four rows (dil = 1:
+// each row is staged once, while the previous one is multiplied), dz in two.  Channel ch, 8-pixel block
+// k at word 36 ch + 4 (k ^ (ch / 8 % 8)): conflict-free for the fragment reads (pitch 36) and for the
+// staging writes (8 lanes load the 64 channels of one pixel, and write 8 channel groups).
+// Bound by the fragment reads and the staging (LDS) together with the matrix cores.  B = 32, N = 64,
+// 64 x 64 channels: 21.8 us (443 TFLOP/s), 682 us with the sums on the VALU from fp32 rows in LDS.
+constexpr int WPW = 36;              // LDS words per channel: 64 pixels of bf16 and 4 words of padding
+__device__ __forceinline__ int wg_word(int ch, int k) { return ch * WPW + ((k ^ (ch / 8 % 8)) * 4); }
 template <int S, int CI, int CO>
-__global__ __launch_bounds__(256) void k_conv_wgrad(const bf16* __restrict__ x, const bf16* __restrict__ dz,
+__global__ __launch_bounds__(512) void k_conv_wgrad(const bf16* __restrict__ x, const bf16* __restrict__ dz,
 	float* __restrict__ part, int rows, int dil)
 {
-	constexpr int NCB = CI / 16;                 // ci blocks of 16
-	constexpr int NTH = CO * NCB;                // active threads
-	__shared__ __attribute__((aligned(16))) float xs[3][S][CI + 4];
-	__shared__ float zs[S][CO + 1];
-	const int b = blockIdx.x / (S / rows);
-	const int y0 = (blockIdx.x % (S / rows)) * rows;
-	const int tid = threadIdx.x;
-	const int co = tid / NCB, cb = tid % NCB;
-	float acc[9][16];
+	constexpr int SEG = S / SEGP;
+	constexpr int WCO = CO / 32, WCI = CI / 16, TG = 8 / (WCO * WCI);   // waves over co, ci and taps
+	constexpr int NT = TG == 1 ? 9 : 5;                                 // taps per wave
+	static_assert(WCO * WCI * TG == 8 && TG <= 2, "8 waves");
+	constexpr int XW = CI * WPW, ZW = CO * WPW;
+	constexpr int XI = 3 * (CI / 8) * 32, ZI = (CO / 8) * 32;           // staging items: 2 pixels x 8 channels
+	static_assert(XI + ZI <= 1024, "two items per thread");
+	__shared__ __attribute__((aligned(16))) unsigned xs[4][3][XW];
+	__shared__ __attribute__((aligned(16))) unsigned zs[2][ZW];
+	const int seg = blockIdx.x % SEG;
+	const int b = blockIdx.x / SEG / (S / rows);
+	const int y0 = (blockIdx.x / SEG % (S / rows)) * rows;
+	const int x0 = seg * SEGP;
+	const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, i16 = lane & 15, kq = lane >> 4;
+	const int wco = w % WCO, wci = w / WCO % WCI, tg = w / (WCO * WCI);
+	struct Item { uint4 a, b; };
+	// items of x row yx (three shifts) and dz row yz (row indices modulo S)
+	auto load = [&](int yx, int yz, Item* it) {
 #pragma unroll
-	for (int t = 0; t < 9; t++)
-#pragma unroll
-		for (int j = 0; j < 16; j++) acc[t][j] = 0.f;
-	float bacc = 0.f;
-	for (int y = y0; y < y0 + rows; y++) {
-		__syncthreads();
-		for (int e = tid; e < 3 * S * CI; e += blockDim.x) {
-			const int r = e / (S * CI), rem = e % (S * CI);
-			const int xx = rem / CI, c = rem % CI;
-			const int ys = (y + dil * (r - 1) + 2 * S) & (S - 1);
-			xs[r][xx][c] = (float)x[(((size_t)b * S + ys) * S + xx) * CI + c];
+		for (int k = 0; k < 2; k++) {
+			const int id = threadIdx.x + 512 * k;
+			if (id >= XI + ZI) continue;
+			const bool isz = id >= XI;
+			const int e = isz ? id - XI : id % (XI / 3);
+			const int sh = isz ? 0 : dil * (id / (XI / 3) - 1);
+			const int nc = isz ? CO / 8 : CI / 8;
+			const int c = e % nc, pr = e / nc;
+			const bf16* src = isz ? dz + ((size_t)b * S + (yz & (S - 1))) * S * CO + c * 8
+				: x + ((size_t)b * S + (yx & (S - 1))) * S * CI + c * 8;
+			const int st = isz ? CO : CI;
+			it[k].a = *(const uint4*)(src + (size_t)((x0 + 2 * pr + sh) & (S - 1)) * st);
+			it[k].b = *(const uint4*)(src + (size_t)((x0 + 2 * pr + 1 + sh) & (S - 1)) * st);
 		}
-		for (int e = tid; e < S * CO; e += blockDim.x) {
-			const int xx = e / CO, c = e % CO;
-			zs[xx][c] = (float)dz[(((size_t)b * S + y) * S + xx) * CO + c];
+	};
+	auto store = [&](int xslot, int zslot, const Item* it) {
+#pragma unroll
+		for (int k = 0; k < 2; k++) {
+			const int id = threadIdx.x + 512 * k;
+			if (id >= XI + ZI) continue;
+			const bool isz = id >= XI;
+			const int e = isz ? id - XI : id % (XI / 3);
+			const int nc = isz ? CO / 8 : CI / 8;
+			const int c = e % nc, pr = e / nc;
+			unsigned* d = (isz ? zs[zslot] : xs[xslot][id / (XI / 3)]) + wg_word(8 * c, pr / 4) + pr % 4;
+			const unsigned* ua = (const unsigned*)&it[k].a;
+			const unsigned* ub = (const unsigned*)&it[k].b;
+#pragma unroll
+			for (int q = 0; q < 4; q++) {
+				d[(2 * q) * WPW] = (ua[q] & 0xffffu) | (ub[q] << 16);
+				d[(2 * q + 1) * WPW] = (ua[q] >> 16) | (ub[q] & 0xffff0000u);
+			}
 		}
-		__syncthreads();
-		if (tid < NTH) {
-			for (int px = 0; px < S; px++) {
-				const float g = zs[px][co];
-				bacc += g;
+	};
+	f32x4 acc[NT][2];
 #pragma unroll
-				for (int kx = 0; kx < 3; kx++) {
-					const int pxs = (px + dil * (kx - 1) + 2 * S) & (S - 1);
+	for (int t = 0; t < NT; t++)
 #pragma unroll
-					for (int ky = 0; ky < 3; ky++)
+		for (int m = 0; m < 2; m++) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+	float bsum[2] = {0.f, 0.f};
+	// one row of dz (zslot) against the x rows in slots (s0 + ky) & 3
+	auto row = [&](int s0, int zslot) {
+		bf16x8 a[2][2];
 #pragma unroll
-						for (int j = 0; j < 16; j++) acc[ky * 3 + kx][j] += g * xs[ky][pxs][cb * 16 + j];
+		for (int m = 0; m < 2; m++)
+#pragma unroll
+			for (int ks = 0; ks < 2; ks++) {
+				a[m][ks] = *(const bf16x8*)&zs[zslot][wg_word(32 * wco + 16 * m + i16, 4 * ks + kq)];
+				if (wci == 0 && tg == 0)
+#pragma unroll
+					for (int q = 0; q < 8; q++) bsum[m] += (float)a[m][ks][q];
+			}
+#pragma unroll
+		for (int t = 0; t < NT; t++) {
+			const int tap = tg * NT + t;
+			if (tap < 9) {
+				const unsigned* xr = xs[(s0 + tap / 3) & 3][tap % 3];
+#pragma unroll
+				for (int ks = 0; ks < 2; ks++) {
+					const bf16x8 f = *(const bf16x8*)&xr[wg_word(16 * wci + i16, 4 * ks + kq)];
+#pragma unroll
+					for (int m = 0; m < 2; m++) acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m][ks], f, acc[t][m], 0, 0, 0);
 				}
 			}
 		}
+	};
+	Item it[2];
+	if (dil == 1) {
+		// x row y0 + r sits in slot (r + 1) & 3
+		for (int r = -1; r <= 1; r++) {
+			load(y0 + r + S, y0, it);
+			store(r + 1, 0, it);
+		}
+		__syncthreads();
+		for (int i = 0; i < rows; i++) {
+			const bool more = i + 1 < rows;
+			if (more) load(y0 + i + 2, y0 + i + 1, it);
+			row(i, i & 1);
+			// slot (i + 3) & 3 and the other dz row were last read before the previous barrier
+			if (more) store((i + 3) & 3, (i + 1) & 1, it);
+			__syncthreads();
+		}
+	} else {
+		for (int i = 0; i < rows; i++) {
+			const int y = y0 + i;
+			__syncthreads();
+			for (int r = -1; r <= 1; r++) {
+				load(y + dil * r + 2 * S, y, it);
+				store(r + 1, 0, it);
+			}
+			__syncthreads();
+			row(0, 0);
+		}
 	}
-	if (tid < NTH) {
-		float* pb = part + (size_t)blockIdx.x * (9 * CO * CI + CO);
+	float* pb = part + (size_t)blockIdx.x * (9 * CO * CI + CO);
 #pragma unroll
-		for (int t = 0; t < 9; t++)
+	for (int t = 0; t < NT; t++) {
+		const int tap = tg * NT + t;
+		if (tap < 9)
 #pragma unroll
-			for (int j = 0; j < 16; j++) pb[((size_t)t * CO + co) * CI + cb * 16 + j] = acc[t][j];
-		if (cb == 0) pb[9 * CO * CI + co] = bacc;
+			for (int m = 0; m < 2; m++)
+#pragma unroll
+				for (int r = 0; r < 4; r++)
+					pb[((size_t)tap * CO + 32 * wco + 16 * m + 4 * kq + r) * CI + 16 * wci + i16] = acc[t][m][r];
 	}
+	if (wci == 0 && tg == 0)
+#pragma unroll
+		for (int m = 0; m < 2; m++) {
+			float v = bsum[m];
+			v += __shfl_xor(v, 16);
+			v += __shfl_xor(v, 32);
+			if (kq == 0) pb[9 * CO * CI + 32 * wco + 16 * m + i16] = v;
+		}
 }
 
-// dW[i] = sum_blk part[blk][i] (i < nw), db[i - nw] likewise (nw <= i < nw + nb), blocks in order
-__global__ void k_wgrad_reduce(const float* __restrict__ part, int nblk, int nw, int nb, float* __restrict__ dW,
-	float* __restrict__ db)
+// dW[i] = sum_blk part[blk][i] (i < nw), db[i - nw] likewise (nw <= i < nw + nb): 8 threads share an
+// element, thread c adds the blocks c, c + 8, ..., and the 8 sums are added in order (a read of part: 256
+// workgroups of 64 x 64 channels, 38 MB, in 11 us; one thread per element took 32)
+__global__ __launch_bounds__(256) void k_wgrad_reduce(const float* __restrict__ part, int nblk, int nw, int nb,
+	float* __restrict__ dW, float* __restrict__ db)
 {
-	const int i = blockIdx.x * blockDim.x + threadIdx.x;
+	__shared__ float sh[8][32];
+	const int c = threadIdx.x / 32, e = threadIdx.x % 32;
+	const int i = blockIdx.x * 32 + e;
 	const int stride = nw + nb;
-	if (i >= stride) return;
 	float s = 0.f;
-	for (int b = 0; b < nblk; b++) s += part[(size_t)b * stride + i];
+	if (i < stride)
+		for (int b = c; b < nblk; b += 8) s += part[(size_t)b * stride + i];
+	sh[c][e] = s;
+	__syncthreads();
+	if (c || i >= stride) return;
+	for (int k = 1; k < 8; k++) s += sh[k][e];
 	if (i < nw) dW[i] = s;
 	else db[i - nw] = s;
 }
@@ -538,7 +638,16 @@ struct qbf_cnn {
 	bf16* g[NL] = {};     // gradient of z[l] (bf16 NHWC), g[NL-1] = gradient of the output
 	float* loss = nullptr;
 	// deterministic reductions: per-workgroup partials of the weight gradients of one layer and of the loss
-	static constexpr int WG_ROWS = 16;    // image rows per workgroup of k_conv_wgrad
+	// image rows per workgroup of k_conv_wgrad: 16, fewer where that leaves less than one workgroup per
+	// CU (a workgroup's first row is staged with two more, and every workgroup writes its partial sums,
+	// so few rows cost more per row).  A training step at B = 32, N = 64: 781 us with 8 rows (256
+	// workgroups), 801 with 16, 888 with 4
+	int wg_rows(int B) const
+	{
+		int rows = 16;
+		while (rows > 4 && B * (S / rows) * (S / SEGP) < 256) rows /= 2;
+		return rows;
+	}
 	float* gpart = nullptr;
 	float* lpart = nullptr;
 	int dil[NL] = {1, 1, 1, 1, 1, 1};
@@ -610,7 +719,12 @@ int qbf_cnn_create(int N, int maxBatch, qbf_cnn** out)
 		}
 	}
 	c->loss = c->alloc_f(1);
-	c->gpart = c->alloc_f((size_t)c->maxTrain * (S / qbf_cnn::WG_ROWS) * (9 * CH * CH + CH));
+	size_t nwg = 0;
+	for (int B = 1; B <= c->maxTrain; B++) {
+		const size_t n = (size_t)B * (S / c->wg_rows(B)) * (S / SEGP);
+		nwg = n > nwg ? n : nwg;
+	}
+	c->gpart = c->alloc_f(nwg * (9 * CH * CH + CH));
 	c->lpart = c->alloc_f(pxt / 256 + 1);
 	c->amp = c->alloc_f(maxBatch);
 	c->sx = c->alloc_f(px * CREAL);
@@ -796,28 +910,28 @@ static int gradients_t(qbf_cnn* c, const float* dIn, const float* dTarget, int B
 		c->lpart, B, inv_n, oscale, c->norm ? c->amp : nullptr);
 	hipLaunchKernelGGL(k_loss_reduce, dim3(1), dim3(256), 0, c->stream, c->lpart, nlb, c->loss);
 	const dim3 grid = conv_grid<S>(B), cblk(64 * CROWS), blk(256);
-	const int rows = qbf_cnn::WG_ROWS;
-	const int nwb = B * (S / rows);
+	const int rows = c->wg_rows(B);
+	const int nwb = B * (S / rows) * (S / SEGP);
 	const dim3 wgrid(nwb);
 	auto reduce = [&](int l) {
 		const int nw = (int)wsize(l), nb = cout_of(l);
-		hipLaunchKernelGGL(k_wgrad_reduce, dim3((unsigned)((nw + nb + 255) / 256)), dim3(256), 0, c->stream, c->gpart,
+		hipLaunchKernelGGL(k_wgrad_reduce, dim3((unsigned)((nw + nb + 31) / 32)), dim3(256), 0, c->stream, c->gpart,
 			nwb, nw, nb, c->gw[l], c->gb[l]);
 	};
 	// last layer: weight gradient, then data gradient into the last hidden pre-activation
-	hipLaunchKernelGGL((k_conv_wgrad<S, CH, CIO>), wgrid, blk, 0, c->stream, c->x[NL - 1], c->g[NL - 1], c->gpart, rows,
+	hipLaunchKernelGGL((k_conv_wgrad<S, CH, CIO>), wgrid, dim3(512), 0, c->stream, c->x[NL - 1], c->g[NL - 1], c->gpart, rows,
 		c->dil[NL - 1]);
 	reduce(NL - 1);
 	hipLaunchKernelGGL((k_conv_mfma<S, CIO, CH, -1, 2>), grid, cblk, 0, c->stream, c->g[NL - 1], c->wbt[NL - 1], nullptr,
 		nullptr, c->g[NL - 2], nullptr, c->z[NL - 2], 1.0f, c->dil[NL - 1], nullptr);
 	for (int l = NL - 2; l >= 1; l--) {
-		hipLaunchKernelGGL((k_conv_wgrad<S, CH, CH>), wgrid, blk, 0, c->stream, c->x[l], c->g[l], c->gpart, rows,
+		hipLaunchKernelGGL((k_conv_wgrad<S, CH, CH>), wgrid, dim3(512), 0, c->stream, c->x[l], c->g[l], c->gpart, rows,
 			c->dil[l]);
 		reduce(l);
 		hipLaunchKernelGGL((k_conv_mfma<S, CH, CH, -1, 2>), grid, cblk, 0, c->stream, c->g[l], c->wbt[l], nullptr, nullptr,
 			c->g[l - 1], nullptr, c->z[l - 1], 1.0f, c->dil[l], nullptr);
 	}
-	hipLaunchKernelGGL((k_conv_wgrad<S, CIO, CH>), wgrid, blk, 0, c->stream, c->x[0], c->g[0], c->gpart, rows, c->dil[0]);
+	hipLaunchKernelGGL((k_conv_wgrad<S, CIO, CH>), wgrid, dim3(512), 0, c->stream, c->x[0], c->g[0], c->gpart, rows, c->dil[0]);
 	reduce(0);
 	HCHK(hipGetLastError());
 	if (hostLoss) {
