@@ -24,6 +24,7 @@
 #include <string.h>
 
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/qbf.h"
@@ -39,6 +40,9 @@ constexpr int NL = 6;           // layers
 constexpr int CH = 64;          // hidden channels
 constexpr int CIO = 32;         // padded input / output channel count
 constexpr int CREAL = 4;        // real input / output channels (Pauli components)
+// channels stored of the network input (CREAL, the amplitude, zeros).  The conversion of 512 images of 64 x 64
+// writes 34 MB instead of 134 (69 us with all 32 channels)
+constexpr int CIN0 = 8;
 
 __host__ __device__ constexpr int cin_of(int l) { return l == 0 ? CIO : CH; }
 __host__ __device__ constexpr int cout_of(int l) { return l == NL - 1 ? CIO : CH; }
@@ -81,8 +85,9 @@ __global__ __launch_bounds__(256) void k_cell_amp(const float* __restrict__ x, f
 	if (threadIdx.x == 0) amp[blockIdx.x] = fmaxf(fmaxf(sh[0], sh[1]), fmaxf(sh[2], sh[3]));
 }
 
-// planar fp32 [B][4][S][S] -> NHWC bf16 [B][S][S][CIO]: channels 0..3 = scale * x (or
-// scale * x / a[b] with amp), channel 4 = scale * a[b] with amp, the rest zero
+// planar fp32 [B][4][S][S] -> NHWC bf16 [B][S][S][CIN0]: channels 0..3 = scale * x (or
+// scale * x / a[b] with amp), channel 4 = scale * a[b] with amp, the rest zero (channels CIN0 ... CIO - 1
+// of the first layer are zero too and not stored)
 template <int S>
 __global__ void k_to_nhwc(const float* __restrict__ x, bf16* __restrict__ out, int B, float scale,
 	const float* __restrict__ amp)
@@ -92,165 +97,241 @@ __global__ void k_to_nhwc(const float* __restrict__ x, bf16* __restrict__ out, i
 	if (i >= n) return;
 	const int b = (int)(i / (S * S)), p = (int)(i % (S * S));
 	const float f = amp ? scale / fmaxf(amp[b], 1e-30f) : scale;
-	bf16* o = out + i * CIO;
-	for (int c = 0; c < CIO; c++) {
-		float v = 0.0f;
-		if (c < CREAL) v = x[((size_t)b * CREAL + c) * (S * S) + p] * f;
-		else if (c == CREAL && amp) v = scale * amp[b];
-		o[c] = (bf16)v;
-	}
+	bf16x8 v;
+	for (int c = 0; c < CIN0; c++) v[c] = (bf16)0.0f;
+	for (int c = 0; c < CREAL; c++) v[c] = (bf16)(x[((size_t)b * CREAL + c) * (S * S) + p] * f);
+	if (amp) v[CREAL] = (bf16)(scale * amp[b]);
+	*(bf16x8*)(out + i * CIN0) = v;
 }
 
 // Implicit-GEMM 3x3 periodic convolution on the matrix cores.
 //   out[b][y][x][n] = sum_t sum_k in[b][y + DIR*d*(ky-1)][x + DIR*d*(kx-1)][k] * Wt[t][n][k]
 // DIR = +1: forward (Wt = W[t][cout][cin]); DIR = -1: backward data (Wt = W^T[t][cin][cout]).
-// MODE 0: out = bias + value, store pre-activation z (fp32) and GELU(z) (bf16 NHWC)
+// MODE 0: out = bias + value, store GELU(out) (bf16 NHWC) and, with Z, out itself (fp32)
 // MODE 1: out = bias + value, store fp32 planar [B][4][S][S] (first 4 channels), times
 //         oscale (and a[b]^2 when amp is given)
 // MODE 2: backward data: g = value * gelu'(zprev) -> bf16 NHWC (gradient of the previous z)
-// A workgroup of CROWS waves computes CROWS consecutive row segments (64 pixels each: S / 64
-// per image row); the layer's weights are staged once in LDS (row pitch KC + 4 elements: the 16
-// lanes of a 16-byte read cover all 64 banks but one pair).  Each wave holds a 64-pixel x NC
-// accumulator (4 x NC/16 MFMA tiles): per tap and 32-channel block it loads 4 A fragments
-// and NC/16 B fragments from LDS for 4 * NC/16 MFMAs.
-// ROWS (S = 64, forward, dilation 1): the workgroup's CROWS rows are consecutive rows of one image,
-// so the CROWS + 2 input rows their taps read are staged in LDS once (each input row read once from
-// global memory instead of nine times) and the A fragments come from LDS too.  Row r, pixel px,
-// 16-byte channel chunk c sits at chunk slot (r S + px) CPP + (c ^ ((px / PPB) % CPP)) (CPP chunks
-// per pixel, PPB pixels per 256 bytes): the 16 lanes of a fragment read, 16 consecutive pixels,
-// then fall into 16 different 16-byte slots of a 256-byte bank line.  Otherwise the A fragments
+// A workgroup of CROWS waves works through a range of blocks of CROWS consecutive rows of one
+// 64-pixel segment, a row each: the layer's weights are staged once in LDS, and with ROWS also, per
+// block, the CROWS + 2 input rows that the taps read (each input row is read once from global memory
+// instead of nine times), the next block's loaded into registers while this one is multiplied.  ROWS 1:
+// dilation 1, rows of 66 pixels.  ROWS 2: other dilations at S = 64, whole rows; the block's rows are then
+// dil apart (k -> dil k mod S runs through a class of S / gcd(dil, S) rows).  ROWS 0: the input fragments
 // are loaded from global memory.
+// The products are W in^T (rows: 16 output channels, columns: 16 pixels) and row i of channel tile t is
+// channel 32 (t / 2) + 8 (i / 4) + 4 (t % 2) + i % 4, so that two tiles leave a lane with 8 consecutive
+// channels of a pixel, which it writes at once, and the four lanes of a pixel 64 contiguous bytes.
+// LDS: 16-byte channel chunk c of weight row n at chunk n CPP + (c ^ g(n)), of pixel px at chunk
+// px CPP + (c ^ ((px / PPB) % CPP)) (CPP chunks per row or pixel, PPB pixels per 256 bytes): the 16 lanes
+// of a fragment read (16 channels, 16 consecutive pixels) fall into 16 different 16-byte slots of a
+// 256-byte bank line.
+// What bounds it (512 images of 64 x 64, 64 -> 64 channels, ROWS 1): 191 us, of which the MFMAs alone 70
+// (busy 42 %), the GELU about 60, reading and writing 536 MB at the rate of a copy 103; they overlap only in
+// part.  It took 310 us with 2-byte stores (products in W^T, a channel per lane), weights staged again for every
+// block and the rows staged with nothing else in flight; dilated layers, from global memory, 330.  The output
+// bits are the same: taps and channels are summed in the same order.
 constexpr int CROWS = 8;
-template <int S, int KC, int NC, int DIR, int MODE, bool ROWS = false>
-__global__ __launch_bounds__(64 * CROWS) __attribute__((amdgpu_waves_per_eu(4))) void k_conv_mfma(const bf16* __restrict__ in, const bf16* __restrict__ Wt,
-	const float* __restrict__ bias, float* __restrict__ zout, bf16* __restrict__ aout, float* __restrict__ yout,
-	const float* __restrict__ zprev, float oscale, int dil, const float* __restrict__ amp)
+constexpr int NCU = 256;           // CUs: with ROWS one workgroup runs on each (LDS), without two
+template <int S, int KC, int NC, int DIR, int MODE, int ROWS, bool Z>
+__global__ __launch_bounds__(64 * CROWS, ROWS ? 2 : 4) void k_conv_mfma(const bf16* __restrict__ in,
+	const bf16* __restrict__ Wt, const float* __restrict__ bias, float* __restrict__ zout, bf16* __restrict__ aout,
+	float* __restrict__ yout, const float* __restrict__ zprev, float oscale, int dil, const float* __restrict__ amp, int nblk)
 {
-	constexpr int NT = NC / 16;       // 16-wide output-channel tiles
+	constexpr int NT = MODE == 1 ? 1 : NC / 16;   // 16-wide output-channel tiles (MODE 1: the real channels' one)
+	constexpr int NR = 16 * NT;       // weight rows per tap
 	constexpr int MT = SEGP / 16;     // 16-pixel tiles of a segment
 	constexpr int SEG = S / SEGP;     // segments per image row
-	constexpr int KP = KC + 4;        // LDS pitch of a weight row (elements)
-	constexpr int CPP = KC / 8;       // 16-byte channel chunks per pixel
-	constexpr int PPB = 16 / CPP;     // pixels per 256 bytes
-	static_assert(!ROWS || (S == SEGP && DIR == 1 && S % CROWS == 0), "row staging: S = 64, forward");
-	__shared__ __attribute__((aligned(16))) bf16 wl[9 * NC * KP];
-	__shared__ __attribute__((aligned(16))) bf16 xl[ROWS ? (CROWS + 2) * S * KC : 8];
-	const int tile = blockIdx.x * CROWS + (threadIdx.x >> 6);
-	const int b = tile / (S * SEG);
-	const int y = (tile / SEG) % S;
-	const int x0 = (tile % SEG) * SEGP;
-	const int lane = threadIdx.x & 63;
+	constexpr int CPP = KC / 8;       // 16-byte channel chunks per weight row
+	constexpr int KIN = DIR == 1 && KC == CIO ? CIN0 : KC;   // channels stored of the input
+	constexpr int CPI = KIN / 8;      // 16-byte channel chunks per pixel
+	constexpr int PPB = 16 / CPI;     // pixels per 256 bytes
+	constexpr int PX = ROWS == 1 ? SEGP + 2 : SEGP;   // staged pixels of a row
+	constexpr int NST = (CROWS + 2) * PX * CPI, NIT_ST = ROWS ? (NST + 64 * CROWS - 1) / (64 * CROWS) : 1;
+	static_assert(MODE != 1 || CREAL == 4, "4 channels of a lane");
+	static_assert(ROWS != 2 || S == SEGP, "whole rows");
+	static_assert(KIN == KC || (CPI == 1 && KC == 32), "the stored channels are the first lanes' chunk");
+	__shared__ __attribute__((aligned(16))) bf16x8 wl[9 * NR * CPP];
+	__shared__ __attribute__((aligned(16))) bf16x8 xl[ROWS ? NST : 1];
+	const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
 	const int i16 = lane & 15, kq = lane >> 4;
-	for (int v = threadIdx.x; v < 9 * NC * (KC / 8); v += 64 * CROWS) {
-		const int r = v / (KC / 8), c8 = v % (KC / 8);
-		const bf16x8 w = *(const bf16x8*)(Wt + (size_t)r * KC + c8 * 8);
-		bf16* d = wl + r * KP + c8 * 8;              // 8-byte aligned (KP = KC + 4)
-		*(uint2*)d = *(const uint2*)&w;
-		*(uint2*)(d + 4) = *((const uint2*)&w + 1);
-	}
-	if constexpr (ROWS) {
-		// input rows y0 - 1 .. y0 + CROWS of image b (periodic), y0 = the workgroup's first row
-		const int y0 = (blockIdx.x * CROWS) % S;
-		for (int q = threadIdx.x; q < (CROWS + 2) * S * CPP; q += 64 * CROWS) {
-			const int r = q / (S * CPP), px = (q / CPP) % S, c = q % CPP;
-			const int ys = (y0 - 1 + r + S) & (S - 1);
-			const bf16x8 v = *(const bf16x8*)(in + (((size_t)b * S + ys) * S + px) * KC + c * 8);
-			*(bf16x8*)(xl + ((r * S + px) * CPP + (c ^ ((px / PPB) % CPP))) * 8) = v;
-		}
-	}
-	__syncthreads();
-	f32x4 acc[MT][NT];
+	// weight row n, chunk c; pixel q of the staged rows, chunk c
+	auto row_of = [](int t, int i) { return NT == 1 ? i : 32 * (t / 2) + 8 * (i / 4) + 4 * (t % 2) + i % 4; };
+	auto wslot = [](int n, int c) {
+		const int i4 = NT == 1 ? n / 4 : n / 8 % 4;        // i / 4
+		return n * CPP + (c ^ ((CPP == 8 ? 2 * i4 + n / 2 % 2 : i4) % CPP));
+	};
+	auto xslot = [](int q, int c) { return q * CPI + (c ^ ((q / PPB) % CPI)); };
+	const int lo = (int)((long long)nblk * blockIdx.x / gridDim.x), hi = (int)((long long)nblk * (blockIdx.x + 1) / gridDim.x);
+	// block -> image, first pixel, row r = -1 ... CROWS
+	auto b_of = [](int blk) { return blk / (SEG * (S / CROWS)); };
+	auto x0_of = [](int blk) { return (blk / (S / CROWS)) % SEG * SEGP; };
+	const int ncl = ROWS == 2 ? S / (dil & -dil) : S;      // rows of a class
+	auto y_of = [&](int blk, int r) {
+		const int k = blk % (S / CROWS) * CROWS;
+		return ROWS == 2 ? (k / ncl + dil * (k % ncl + r + S)) & (S - 1) : (k + r) & (S - 1);
+	};
+	bf16x8 st[NIT_ST];
+	auto load_rows = [&](int blk) {
+		const int x0 = x0_of(blk);
+		const bf16* src = in + (size_t)b_of(blk) * S * S * KIN;
 #pragma unroll
-	for (int m = 0; m < MT; m++)
-#pragma unroll
-		for (int t = 0; t < NT; t++) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-	// K loop over the 9 taps x KC/32 channel blocks, the input fragments of the next iteration
-	// loaded while the MFMAs of this one run (two iterations per loop body: the fragments ping-pong
-	// between two register sets)
-	constexpr int KB = KC / 32, NIT = 9 * KB;
-	auto load_a = [&](int it, bf16x8* a) {
-		const int tap = it / KB, kb = it % KB;
-		if constexpr (ROWS) {
-			// LDS row of the tap: the wave's row (y - y0) + tap / 3 (row 0 holds y0 - 1)
-			const int r = (threadIdx.x >> 6) + tap / 3;
-			const int c = kb * 4 + kq;
-#pragma unroll
-			for (int m = 0; m < MT; m++) {
-				const int px = (m * 16 + i16 + tap % 3 - 1 + S) & (S - 1);
-				a[m] = *(const bf16x8*)(xl + ((r * S + px) * CPP + (c ^ ((px / PPB) % CPP))) * 8);
-			}
-		} else {
-			const int ys = (y + DIR * dil * (tap / 3 - 1) + 2 * S) & (S - 1);
-			const int sh = DIR * dil * (tap % 3 - 1) + 2 * S;
-			const bf16* rowp = in + ((size_t)b * S + ys) * S * KC + kb * 32 + kq * 8;
-#pragma unroll
-			for (int m = 0; m < MT; m++)
-				a[m] = *(const bf16x8*)(rowp + (size_t)((x0 + m * 16 + i16 + sh) & (S - 1)) * KC);
+		for (int k = 0; k < NIT_ST; k++) {
+			const int q = threadIdx.x + k * 64 * CROWS;
+			const int px = q / CPI, c = q % CPI;
+			const int ys = y_of(blk, px / PX - 1), xs = ROWS == 1 ? (x0 - 1 + px % PX) & (S - 1) : px % PX;
+			if (q < NST) st[k] = *(const bf16x8*)(src + (ys * S + xs) * KIN + c * 8);
 		}
 	};
-	bf16x8 a[MT];
-	load_a(0, a);
-#pragma unroll 2
-	for (int it = 0; it < NIT; it++) {
-		const int tap = it / KB, kb = it % KB;
-		const bf16* wt = wl + tap * NC * KP;
-		bf16x8 w[NT];
+	auto store_rows = [&]() {
 #pragma unroll
-		for (int t = 0; t < NT; t++) {
-			const bf16* q = wt + (t * 16 + i16) * KP + kb * 32 + kq * 8;
-			uint2 lo = *(const uint2*)q, hi = *(const uint2*)(q + 4);
-			uint4 u = {lo.x, lo.y, hi.x, hi.y};
-			w[t] = *(const bf16x8*)&u;
+		for (int k = 0; k < NIT_ST; k++) {
+			const int q = threadIdx.x + k * 64 * CROWS;
+			if (q < NST) xl[xslot(q / CPI, q % CPI)] = st[k];
 		}
-		bf16x8 an[MT];
-		load_a(it + 1 < NIT ? it + 1 : it, an);
+	};
+	float bs[4 * NT];
+	// the first block's rows, the weights and the bias are loaded together
+	if constexpr (ROWS)
+		if (lo < hi) load_rows(lo);
+	constexpr int NWL = 9 * NR * CPP, NIT_W = (NWL + 64 * CROWS - 1) / (64 * CROWS);
+	bf16x8 ws[NIT_W];
+#pragma unroll
+	for (int k = 0; k < NIT_W; k++) {
+		const int v = threadIdx.x + k * 64 * CROWS;
+		if (v < NWL) ws[k] = *(const bf16x8*)(Wt + ((size_t)(v / (NR * CPP)) * NC + v / CPP % NR) * KC + v % CPP * 8);
+	}
+	if constexpr (MODE != 2) {
+#pragma unroll
+		for (int k = 0; k < 4 * NT; k++) bs[k] = bias[row_of(k / 4, 4 * kq) + k % 4];
+#pragma unroll
+		for (int k = 0; k < 4 * NT; k++) asm volatile("" : "+v"(bs[k]));   // loaded before the loop over the blocks
+	}
+#pragma unroll
+	for (int k = 0; k < NIT_W; k++) {
+		const int v = threadIdx.x + k * 64 * CROWS;
+		if (v < NWL) wl[v / (NR * CPP) * NR * CPP + wslot(v / CPP % NR, v % CPP)] = ws[k];
+	}
+	if constexpr (ROWS) store_rows();
+	__syncthreads();
+	// the results of a block: lane holds channels row_of(t, 4 kq) + r of pixel m 16 + i16
+	f32x4 acc[MT][NT];
+	auto finish = [&](int blk) {
+		const int b = b_of(blk), x0 = x0_of(blk), y = y_of(blk, w);
+		if constexpr (MODE == 1) {
+			float osc = oscale;
+			if (amp) osc *= amp[b] * amp[b];
+			if (kq == 0)
+#pragma unroll
+				for (int m = 0; m < MT; m++)
+#pragma unroll
+					for (int r = 0; r < CREAL; r++)
+						yout[((size_t)b * CREAL + r) * (S * S) + (size_t)y * S + x0 + m * 16 + i16] = osc * (acc[m][0][r] + bs[r]);
+		} else {
+#pragma unroll
+			for (int m = 0; m < MT; m++) {
+				const size_t o = (((size_t)b * S + y) * S + x0 + m * 16 + i16) * NC + kq * 8;
+				bf16x8 v[NT / 2];
+#pragma unroll
+				for (int t = 0; t < NT; t++) {
+					f32x4 zp = acc[m][t];
+					if constexpr (MODE == 0) {
+#pragma unroll
+						for (int r = 0; r < 4; r++) zp[r] += bs[4 * t + r];
+						if constexpr (Z) *(f32x4*)(zout + o + 32 * (t / 2) + 4 * (t % 2)) = zp;
+#pragma unroll
+						for (int r = 0; r < 4; r++) v[t / 2][t % 2 * 4 + r] = (bf16)gelu(zp[r]);
+					} else {
+						const f32x4 z = *(const f32x4*)(zprev + o + 32 * (t / 2) + 4 * (t % 2));
+#pragma unroll
+						for (int r = 0; r < 4; r++) v[t / 2][t % 2 * 4 + r] = (bf16)(zp[r] * gelu_grad(z[r]));
+					}
+				}
+#pragma unroll
+				for (int k = 0; k < NT / 2; k++) *(bf16x8*)(aout + o + 32 * k) = v[k];
+			}
+		}
+	};
+	// With ROWS the workgroup's waves keep step at the barriers; half of them write a block's results
+	// only after the barriers, so that on each SIMD one wave's epilogue runs beside the other's MFMAs
+	// (six layers, 512 images: 934 us without, 907 with it and the MFMAs' priority)
+	const bool late = ROWS && __builtin_amdgcn_readfirstlane(w) >= CROWS / 2;
+	for (int blk = lo; blk < hi; blk++) {
+		const int b = b_of(blk), x0 = x0_of(blk), y = y_of(blk, w);
+		if constexpr (ROWS)
+			if (blk + 1 < hi) load_rows(blk + 1);
+		if (late && blk > lo) finish(blk - 1);
 #pragma unroll
 		for (int m = 0; m < MT; m++)
 #pragma unroll
-			for (int t = 0; t < NT; t++) acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], w[t], acc[m][t], 0, 0, 0);
+			for (int t = 0; t < NT; t++) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+		// K loop over the 9 taps x KC/32 channel blocks, the fragments of the next iteration
+		// loaded while the MFMAs of this one run (two iterations per loop body: the fragments ping-pong
+		// between two register sets)
+		constexpr int KB = KC / 32, NIT = 9 * KB;
+		bf16x8 zero;
 #pragma unroll
-		for (int m = 0; m < MT; m++) a[m] = an[m];
-	}
-	// lane holds D[4*kq + r][i16] of tile (m, t): pixel m*16 + 4*kq + r, channel t*16 + i16
-	float osc = oscale;
-	if (MODE == 1 && amp) osc *= amp[b] * amp[b];
-	if constexpr (MODE == 1) {
-		// the CREAL output channels of the segment go through LDS (the weights are no longer
-		// needed) so that the NCHW float rows are written whole: [c][64] per wave, 16 bytes a lane
-		__syncthreads();
-		float* ys = (float*)wl + (threadIdx.x >> 6) * (CREAL * SEGP);
-		if (i16 < CREAL)
+		for (int q = 0; q < 8; q++) zero[q] = (bf16)0.0f;
+		auto load_a = [&](int it, bf16x8* a) {
+			const int tap = it / KB, kb = it % KB;
+			if constexpr (ROWS) {
+				// staged row 0 is row -1 of the block, staged pixel 0 is x0 - 1 (ROWS 1) or 0 (ROWS 2)
+				const int row = (w + 1 + DIR * (tap / 3 - 1)) * PX, sh = DIR * (tap % 3 - 1);
+				const int c = CPI == 1 ? 0 : kb * 4 + kq;
+				const int p0 = row + 1 + sh + i16, q0 = i16 + dil * sh + 2 * S;
+#pragma unroll
+				for (int m = 0; m < MT; m++)
+					a[m] = xl[ROWS == 1 ? xslot(p0 + m * 16, c) : xslot(row + ((q0 + m * 16) & (S - 1)), c)];
+			} else {
+				const int ys = (y + DIR * dil * (tap / 3 - 1) + 2 * S) & (S - 1);
+				const int sh = DIR * dil * (tap % 3 - 1) + 2 * S;
+				const bf16* rowp = in + ((size_t)b * S + ys) * S * KIN + (CPI == 1 ? 0 : kb * 32 + kq * 8);
+#pragma unroll
+				for (int m = 0; m < MT; m++)
+					a[m] = *(const bf16x8*)(rowp + (size_t)((x0 + m * 16 + i16 + sh) & (S - 1)) * KIN);
+			}
+			if (CPI == 1 && kq)
+#pragma unroll
+				for (int m = 0; m < MT; m++) a[m] = zero;
+		};
+		auto load_w = [&](int it, bf16x8* wf) {
+			const int tap = it / KB, kb = it % KB;
+#pragma unroll
+			for (int t = 0; t < NT; t++)
+				wf[t] = wl[tap * NR * CPP + wslot(row_of(t, i16), kb * 4 + kq)];
+		};
+		bf16x8 a[MT], wf[NT];
+		load_a(0, a);
+		if constexpr (ROWS) load_w(0, wf);
+		__builtin_amdgcn_s_setprio(1);   // the MFMAs before the other waves' epilogues
+#pragma unroll(ROWS ? 2 : 1)
+		for (int it = 0; it < NIT; it++) {
+			bf16x8 an[MT], wn[NT];
+			if constexpr (!ROWS) load_w(it, wf);
+			load_a(it + 1 < NIT ? it + 1 : it, an);
+			if constexpr (ROWS) {
+				load_w(it + 1 < NIT ? it + 1 : it, wn);
+				__builtin_amdgcn_sched_barrier(0);   // or the loads sink to their use
+			}
 #pragma unroll
 			for (int m = 0; m < MT; m++)
 #pragma unroll
-				for (int r = 0; r < 4; r++) ys[i16 * SEGP + m * 16 + kq * 4 + r] = osc * (acc[m][0][r] + bias[i16]);
-		__syncthreads();
-		static_assert(CREAL * SEGP == 4 * 64, "one float4 per lane");
-		const int c = lane / (SEGP / 4), x4 = (lane % (SEGP / 4)) * 4;
-		*(float4*)(yout + ((size_t)b * CREAL + c) * (S * S) + (size_t)y * S + x0 + x4) = *(const float4*)(ys + c * SEGP + x4);
-		return;
-	}
+				for (int t = 0; t < NT; t++) acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[t], a[m], acc[m][t], 0, 0, 0);
 #pragma unroll
-	for (int m = 0; m < MT; m++)
+			for (int m = 0; m < MT; m++) a[m] = an[m];
 #pragma unroll
-		for (int t = 0; t < NT; t++) {
-			const int n = t * 16 + i16;
-#pragma unroll
-			for (int r = 0; r < 4; r++) {
-				const int xo = x0 + m * 16 + kq * 4 + r;
-				const size_t pix = ((size_t)b * S + y) * S + xo;
-				const float v = acc[m][t][r];
-				if (MODE == 0) {
-					const float z = v + bias[n];
-					if (zout) zout[pix * NC + n] = z;
-					aout[pix * NC + n] = (bf16)gelu(z);
-				} else if (MODE == 1) {
-					if (n < CREAL) yout[((size_t)b * CREAL + n) * (S * S) + (size_t)y * S + xo] = osc * (v + bias[n]);
-				} else {
-					aout[pix * NC + n] = (bf16)(v * gelu_grad(zprev[pix * NC + n]));
-				}
-			}
+			for (int t = 0; t < NT; t++)
+				if constexpr (ROWS) wf[t] = wn[t];
 		}
+		__builtin_amdgcn_s_setprio(0);
+		if (!late) finish(blk);
+		if constexpr (ROWS)
+			if (blk + 1 < hi) {
+				__syncthreads();
+				store_rows();
+				__syncthreads();
+			}
+	}
+	if (late && lo < hi) finish(hi - 1);
 }
 
 // Weight and bias gradients on the matrix cores, per workgroup:
@@ -276,6 +357,7 @@ __global__ __launch_bounds__(512) void k_conv_wgrad(const bf16* __restrict__ x, 
 	float* __restrict__ part, int rows, int dil)
 {
 	constexpr int SEG = S / SEGP;
+	constexpr int CIS = CI == CIO ? CIN0 : CI;   // channels stored of x
 	constexpr int WCO = CO / 32, WCI = CI / 16, TG = 8 / (WCO * WCI);   // waves over co, ci and taps
 	constexpr int NT = TG == 1 ? 9 : 5;                                 // taps per wave
 	static_assert(WCO * WCI * TG == 8 && TG <= 2, "8 waves");
@@ -303,8 +385,12 @@ __global__ __launch_bounds__(512) void k_conv_wgrad(const bf16* __restrict__ x, 
 			const int nc = isz ? CO / 8 : CI / 8;
 			const int c = e % nc, pr = e / nc;
 			const bf16* src = isz ? dz + ((size_t)b * S + (yz & (S - 1))) * S * CO + c * 8
-				: x + ((size_t)b * S + (yx & (S - 1))) * S * CI + c * 8;
-			const int st = isz ? CO : CI;
+				: x + ((size_t)b * S + (yx & (S - 1))) * S * CIS + c * 8;
+			const int st = isz ? CO : CIS;
+			if (!isz && 8 * c >= CIS) {
+				it[k].a = it[k].b = uint4{0, 0, 0, 0};
+				continue;
+			}
 			it[k].a = *(const uint4*)(src + (size_t)((x0 + 2 * pr + sh) & (S - 1)) * st);
 			it[k].b = *(const uint4*)(src + (size_t)((x0 + 2 * pr + 1 + sh) & (S - 1)) * st);
 		}
@@ -709,7 +795,7 @@ int qbf_cnn_create(int N, int maxBatch, qbf_cnn** out)
 		c->w[l] = c->alloc_f(nw); c->gw[l] = c->alloc_f(nw); c->mw[l] = c->alloc_f(nw); c->vw[l] = c->alloc_f(nw);
 		c->bias[l] = c->alloc_f(nb); c->gb[l] = c->alloc_f(nb); c->mb[l] = c->alloc_f(nb); c->vb[l] = c->alloc_f(nb);
 		c->wb[l] = c->alloc_b(nw); c->wbt[l] = c->alloc_b(nw);
-		c->x[l] = c->alloc_b(px * cin_of(l));
+		c->x[l] = c->alloc_b(px * (l ? CH : CIN0));
 		c->g[l] = c->alloc_b(pxt * cout_of(l));
 		if (l < NL - 1) c->z[l] = c->alloc_f(pxt * cout_of(l));
 		if (!c->w[l] || !c->gw[l] || !c->mw[l] || !c->vw[l] || !c->bias[l] || !c->gb[l] || !c->mb[l] || !c->vb[l] ||
@@ -840,9 +926,22 @@ int qbf_cnn_get_params(qbf_cnn* c, float* host, int grads)
 
 } // extern "C"
 
-// convolution grid: CROWS row segments of 64 pixels per workgroup
-template <int S>
-static dim3 conv_grid(int B) { return dim3((unsigned)(B * S * (S / SEGP) / CROWS)); }
+// one layer's convolution: staged rows where the rows that a block's taps reach fit into LDS beside the weights
+// (six layers of dilation 2, 512 images of 64 x 64: 1.02 ms, 2.25 ms from global memory), that is for dilation 1 and,
+// at 64 x 64, for the dilations whose classes hold a whole block
+template <int S, int KC, int NC, int DIR, int MODE, bool Z = false>
+static void conv(qbf_cnn* c, int B, const bf16* in, const bf16* W, const float* bias, float* zout, bf16* aout, float* yout,
+	const float* zprev, float oscale, int dil, const float* amp)
+{
+	const int nblk = B * (S / SEGP) * (S / CROWS);
+	auto launch = [&](auto k, int nwg) {
+		hipLaunchKernelGGL(k, dim3((unsigned)(nblk < nwg ? nblk : nwg)), dim3(64 * CROWS), 0, c->stream, in, W, bias, zout, aout,
+			yout, zprev, oscale, dil, amp, nblk);
+	};
+	if (dil == 1) launch(k_conv_mfma<S, KC, NC, DIR, MODE, 1, Z>, NCU);
+	else if (S == SEGP && S / (dil & -dil) >= CROWS) launch(k_conv_mfma<S, KC, NC, DIR, MODE, S == SEGP ? 2 : 0, Z>, NCU);
+	else launch(k_conv_mfma<S, KC, NC, DIR, MODE, 0, Z>, 2 * NCU);
+}
 
 template <int S>
 static int run_forward_t(qbf_cnn* c, const float* dIn, int B, float iscale, float* dOut, float oscale, bool train)
@@ -852,29 +951,20 @@ static int run_forward_t(qbf_cnn* c, const float* dIn, int B, float iscale, floa
 	if (c->norm) hipLaunchKernelGGL(k_cell_amp<S>, dim3(B), dim3(256), 0, c->stream, dIn, c->amp);
 	hipLaunchKernelGGL(k_to_nhwc<S>, dim3((unsigned)((npx + 255) / 256)), dim3(256), 0, c->stream, dIn, c->x[0], B,
 		iscale, amp);
-	const dim3 grid = conv_grid<S>(B), blk(64 * CROWS);
-	// the input rows staged in LDS where the taps allow it (S = 64, dilation 1)
-	constexpr bool R = S == SEGP;
-	if (R && c->dil[0] == 1)
-		hipLaunchKernelGGL((k_conv_mfma<S, CIO, CH, 1, 0, R>), grid, blk, 0, c->stream, c->x[0], c->wb[0], c->bias[0],
-			train ? c->z[0] : nullptr, c->x[1], nullptr, nullptr, 1.0f, 1, nullptr);
-	else
-		hipLaunchKernelGGL((k_conv_mfma<S, CIO, CH, 1, 0>), grid, blk, 0, c->stream, c->x[0], c->wb[0], c->bias[0],
-			train ? c->z[0] : nullptr, c->x[1], nullptr, nullptr, 1.0f, c->dil[0], nullptr);
-	for (int l = 1; l < NL - 1; l++) {
-		if (R && c->dil[l] == 1)
-			hipLaunchKernelGGL((k_conv_mfma<S, CH, CH, 1, 0, R>), grid, blk, 0, c->stream, c->x[l], c->wb[l], c->bias[l],
-				train ? c->z[l] : nullptr, c->x[l + 1], nullptr, nullptr, 1.0f, 1, nullptr);
+	// hidden layers: with the pre-activations where a backward pass follows
+	auto hidden = [&](auto first, int l) {
+		constexpr int K = decltype(first)::value ? CIO : CH;
+		if (train)
+			conv<S, K, CH, 1, 0, true>(c, B, c->x[l], c->wb[l], c->bias[l], c->z[l], c->x[l + 1], nullptr, nullptr, 1.0f, c->dil[l],
+				nullptr);
 		else
-			hipLaunchKernelGGL((k_conv_mfma<S, CH, CH, 1, 0>), grid, blk, 0, c->stream, c->x[l], c->wb[l], c->bias[l],
-				train ? c->z[l] : nullptr, c->x[l + 1], nullptr, nullptr, 1.0f, c->dil[l], nullptr);
-	}
-	if (R && c->dil[NL - 1] == 1)
-		hipLaunchKernelGGL((k_conv_mfma<S, CH, CIO, 1, 1, R>), grid, blk, 0, c->stream, c->x[NL - 1], c->wb[NL - 1],
-			c->bias[NL - 1], nullptr, nullptr, dOut, nullptr, oscale, 1, amp);
-	else
-		hipLaunchKernelGGL((k_conv_mfma<S, CH, CIO, 1, 1>), grid, blk, 0, c->stream, c->x[NL - 1], c->wb[NL - 1],
-			c->bias[NL - 1], nullptr, nullptr, dOut, nullptr, oscale, c->dil[NL - 1], amp);
+			conv<S, K, CH, 1, 0>(c, B, c->x[l], c->wb[l], c->bias[l], nullptr, c->x[l + 1], nullptr, nullptr, 1.0f, c->dil[l],
+				nullptr);
+	};
+	hidden(std::true_type{}, 0);
+	for (int l = 1; l < NL - 1; l++) hidden(std::false_type{}, l);
+	conv<S, CH, CIO, 1, 1>(c, B, c->x[NL - 1], c->wb[NL - 1], c->bias[NL - 1], nullptr, nullptr, dOut, nullptr, oscale,
+		c->dil[NL - 1], amp);
 	HCHK(hipGetLastError());
 	return 0;
 }
@@ -909,7 +999,6 @@ static int gradients_t(qbf_cnn* c, const float* dIn, const float* dTarget, int B
 	hipLaunchKernelGGL(k_loss_grad<S>, dim3((unsigned)nlb), dim3(256), 0, c->stream, dOut, dTarget, c->g[NL - 1],
 		c->lpart, B, inv_n, oscale, c->norm ? c->amp : nullptr);
 	hipLaunchKernelGGL(k_loss_reduce, dim3(1), dim3(256), 0, c->stream, c->lpart, nlb, c->loss);
-	const dim3 grid = conv_grid<S>(B), cblk(64 * CROWS), blk(256);
 	const int rows = c->wg_rows(B);
 	const int nwb = B * (S / rows) * (S / SEGP);
 	const dim3 wgrid(nwb);
@@ -922,14 +1011,14 @@ static int gradients_t(qbf_cnn* c, const float* dIn, const float* dTarget, int B
 	hipLaunchKernelGGL((k_conv_wgrad<S, CH, CIO>), wgrid, dim3(512), 0, c->stream, c->x[NL - 1], c->g[NL - 1], c->gpart, rows,
 		c->dil[NL - 1]);
 	reduce(NL - 1);
-	hipLaunchKernelGGL((k_conv_mfma<S, CIO, CH, -1, 2>), grid, cblk, 0, c->stream, c->g[NL - 1], c->wbt[NL - 1], nullptr,
-		nullptr, c->g[NL - 2], nullptr, c->z[NL - 2], 1.0f, c->dil[NL - 1], nullptr);
+	conv<S, CIO, CH, -1, 2>(c, B, c->g[NL - 1], c->wbt[NL - 1], nullptr, nullptr, c->g[NL - 2], nullptr, c->z[NL - 2], 1.0f,
+		c->dil[NL - 1], nullptr);
 	for (int l = NL - 2; l >= 1; l--) {
 		hipLaunchKernelGGL((k_conv_wgrad<S, CH, CH>), wgrid, dim3(512), 0, c->stream, c->x[l], c->g[l], c->gpart, rows,
 			c->dil[l]);
 		reduce(l);
-		hipLaunchKernelGGL((k_conv_mfma<S, CH, CH, -1, 2>), grid, cblk, 0, c->stream, c->g[l], c->wbt[l], nullptr, nullptr,
-			c->g[l - 1], nullptr, c->z[l - 1], 1.0f, c->dil[l], nullptr);
+		conv<S, CH, CH, -1, 2>(c, B, c->g[l], c->wbt[l], nullptr, nullptr, c->g[l - 1], nullptr, c->z[l - 1], 1.0f, c->dil[l],
+			nullptr);
 	}
 	hipLaunchKernelGGL((k_conv_wgrad<S, CIO, CH>), wgrid, dim3(512), 0, c->stream, c->x[0], c->g[0], c->gpart, rows, c->dil[0]);
 	reduce(0);
