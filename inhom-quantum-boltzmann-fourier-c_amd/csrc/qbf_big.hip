@@ -63,7 +63,7 @@ __device__ __forceinline__ void pad_rows(const double2* __restrict__ src, const 
 				v[s] = czero<R>();
 			}
 		}
-		line_fwd<R, P, G, E>(v, p, tw);
+		line16_fwd<R, P, E>(v, p, tw);
 		cx<R>* row = dst + (padrow(ln) ^ rx) * P + blk(p);
 #pragma unroll
 		for (int u = 0; u < E; u++) row[u] = v[u];
@@ -90,7 +90,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_padfft_big(PadFFTArgs a)
 	__shared__ cx<R> tw[TW];
 	load_twiddles_g<R, P, G, T>(tw, a.tw256);
 	const int o = blockIdx.x;
-	const int lt = threadIdx.x / G, p = threadIdx.x % G;
+	const int lt = threadIdx.x / G, p = dpp_p(threadIdx.x % G);
 	cx<R>* xs = (cx<R>*)a.xs + (size_t)blockIdx.x * PP;
 	cx<R>* out = (cx<R>*)a.out + (size_t)o * PP;
 	const int slot = o % a.nslot;
@@ -108,7 +108,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_padfft_big(PadFFTArgs a)
 		const int c = sw * L + lt;
 		cx<R> v[E];
 		load_padded_col<R>(v, xs, 0, c, p);
-		line_fwd<R, P, G, E>(v, p, tw);
+		line16_fwd<R, P, E>(v, p, tw);
 		const int r0 = blk(p);
 #pragma unroll
 		for (int u = 0; u < E; u++) out[(r0 + u) * P + c] = v[u];
@@ -131,7 +131,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_i1acc_big(I1Args a)
 	const int cell = lb / (a.nchunk * a.ninst);
 	const int qa = (int)(((long long)chunk * a.nterm) / a.nchunk);
 	const int qb = (int)(((long long)(chunk + 1) * a.nterm) / a.nchunk);
-	const int lt = threadIdx.x / G, p = threadIdx.x % G;
+	const int lt = threadIdx.x / G, p = dpp_p(threadIdx.x % G);
 	const double2* g = a.src + ((size_t)cell * a.nsrc + a.instSrc[inst]) * (N * N);
 	const cx<R>* Fh = (const cx<R>*)a.Fhat + ((size_t)cell * a.nFh + a.instFh[inst]) * PP;
 	cx<R>* xs = (cx<R>*)a.xs + (size_t)blockIdx.x * PP;
@@ -154,7 +154,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_i1acc_big(I1Args a)
 			const int c = sw * L + lt;
 			cx<R> v[E];
 			load_padded_col<R>(v, xs, 0, c, p);
-			line_fwd<R, P, G, E>(v, p, tw);
+			line16_fwd<R, P, E>(v, p, tw);
 			const int r0 = blk(p);
 #pragma unroll
 			for (int u = 0; u < E; u++) {
@@ -162,7 +162,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_i1acc_big(I1Args a)
 				f = mk<R>(fa * f.x + fb, fa * f.y);
 				v[u] = cmul<R>(f, v[u]);
 			}
-			line_bwd<R, P, G, E>(v, p, tw);
+			line16_bwd<R, P, E>(v, p, tw);
 #pragma unroll
 			for (int s = 0; s < E; s++) xs[(p + G * s) * P + c] = v[s];
 		}
@@ -176,7 +176,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_i1acc_big(I1Args a)
 			const cx<R>* row = xs + r * P + blk(p);
 #pragma unroll
 			for (int u = 0; u < E; u++) v[u] = row[u];
-			line_bwd<R, P, G, E>(v, p, tw);
+			line16_bwd<R, P, E>(v, p, tw);
 #pragma unroll
 			for (int s = 0; s < E; s++) {
 				const int i = r * P + p + G * s;
@@ -196,7 +196,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_i1acc_big(I1Args a)
 		cx<R> v[E];
 #pragma unroll
 		for (int s = 0; s < E; s++) v[s] = acc[r * P + p + G * s];
-		line_fwd<R, P, G, E>(v, p, tw);
+		line16_fwd<R, P, E>(v, p, tw);
 		cx<R>* row = acc + r * P + blk(p);
 #pragma unroll
 		for (int u = 0; u < E; u++) row[u] = v[u];
@@ -208,7 +208,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_i1acc_big(I1Args a)
 		cx<R> v[E];
 #pragma unroll
 		for (int s = 0; s < E; s++) v[s] = acc[(p + G * s) * P + c];
-		line_fwd<R, P, G, E>(v, p, tw);
+		line16_fwd<R, P, E>(v, p, tw);
 		const int r0 = blk(p);
 #pragma unroll
 		for (int u = 0; u < E; u++) acc[(r0 + u) * P + c] = v[u];
@@ -232,7 +232,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_i2acc_big(I2Args a)
 	const int cell = lb / (a.nchunk * a.ninst);
 	const int qa = (int)(((long long)chunk * a.nterm) / a.nchunk);
 	const int qb = (int)(((long long)(chunk + 1) * a.nterm) / a.nchunk);
-	const int lt = threadIdx.x / G, p = threadIdx.x % G;
+	const int lt = threadIdx.x / G, p = dpp_p(threadIdx.x % G);
 	const double2* f = a.src + ((size_t)cell * a.nsrc + a.instF[inst]) * (N * N);
 	const double2* g = a.src + ((size_t)cell * a.nsrc + a.instG[inst]) * (N * N);
 	cx<R>* xs = (cx<R>*)a.xs + (size_t)blockIdx.x * PP;
@@ -255,9 +255,9 @@ __global__ __launch_bounds__(big::TB<R>) void k_i2acc_big(I2Args a)
 			const int c = sw * L + lt;
 			cx<R> x[E], y[E];
 			load_padded_col<R>(x, xs, 0, c, p);
-			line_fwd<R, P, G, E>(x, p, tw);
+			line16_fwd<R, P, E>(x, p, tw);
 			load_padded_col<R>(y, xs, 128, c, p);
-			line_fwd<R, P, G, E>(y, p, tw);
+			line16_fwd<R, P, E>(y, p, tw);
 #pragma unroll
 			for (int u = 0; u < E; u++) {
 				const int i = (r0 + u) * P + c;
@@ -289,7 +289,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_i3acc_big(I3Args a)
 	const int cell = lb / (a.nchunk * a.nout);
 	const int qa = (int)(((long long)chunk * a.nq) / a.nchunk);
 	const int qb = (int)(((long long)(chunk + 1) * a.nq) / a.nchunk);
-	const int lt = threadIdx.x / G, p = threadIdx.x % G;
+	const int lt = threadIdx.x / G, p = dpp_p(threadIdx.x % G);
 	cx<R>* xs = (cx<R>*)a.xs + (size_t)blockIdx.x * (I3_NI * PP);
 	cx<R>* accp = (cx<R>*)a.acc + (((size_t)cell * a.nout + out) * a.nchunk + chunk) * PP;
 	const cx<R>* Sh = (const cx<R>*)a.Shat + (size_t)cell * a.nS * PP;
@@ -330,7 +330,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_i3acc_big(I3Args a)
 #pragma unroll
 					for (int u = 0; u < E; u++) v[u] = cmul<R>(Sg[u], Fh[u]);
 				}
-				line_bwd<R, P, G, E>(v, p, tw);
+				line16_bwd<R, P, E>(v, p, tw);
 				cx<R>* x = uni(xs, (long long)in * PP) + rb + p;
 #pragma unroll
 				for (int s = 0; s < E; s++) x[G * s] = v[s];
@@ -349,13 +349,13 @@ __global__ __launch_bounds__(big::TB<R>) void k_i3acc_big(I3Args a)
 				cx<R> v[E];
 #pragma unroll
 				for (int u = 0; u < E; u++) v[u] = x[u * P];
-				line_bwd<R, P, G, E>(v, p, tw);
+				line16_bwd<R, P, E>(v, p, tw);
 #pragma unroll
 				for (int s = 0; s < E; s++) {
 					v[s].x *= m[s];
 					v[s].y *= m[s];
 				}
-				line_fwd<R, P, G, E>(v, p, tw);
+				line16_fwd<R, P, E>(v, p, tw);
 #pragma unroll
 				for (int u = 0; u < E; u++) x[u * P] = v[u];
 			}
@@ -373,7 +373,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_i3acc_big(I3Args a)
 				cx<R> v[E];
 #pragma unroll
 				for (int s = 0; s < E; s++) v[s] = x[G * s];
-				line_fwd<R, P, G, E>(v, p, tw);
+				line16_fwd<R, P, E>(v, p, tw);
 				const cx<R>* Ff = uni(Fq, (long long)a.instF[out][in] * PP) + rb + r0;
 				if constexpr (PAIR) {
 					const R wa = (R)a.instW[out][2 * in], wb = (R)a.instW[out][2 * in + 1];
@@ -426,7 +426,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_i3fold_big(I3FoldArgs a)
 	const int cell = lb / (a.nchunk * NO);
 	const int qa = (int)(((long long)chunk * a.nq) / a.nchunk);
 	const int qb = (int)(((long long)(chunk + 1) * a.nq) / a.nchunk);
-	const int lt = threadIdx.x / G, p = threadIdx.x % G;
+	const int lt = threadIdx.x / G, p = dpp_p(threadIdx.x % G);
 	cx<R>* xs = (cx<R>*)a.xs + (size_t)blockIdx.x * (I3_NI * PP);
 	cx<R>* accp = (cx<R>*)a.acc + (((size_t)cell * NO + j) * a.nchunk + chunk) * PP;
 	using MB = MirrorBox<N, G, E, PAIR>;
@@ -481,7 +481,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_i3fold_big(I3FoldArgs a)
 #pragma unroll
 					for (int u = 0; u < E; u++) v[u] = cmul<R>(Sg[u], Fh[u]);
 				}
-				line_bwd<R, P, G, E>(v, p, tw);
+				line16_bwd<R, P, E>(v, p, tw);
 				cx<R>* x = uni(xs, (long long)in * PP) + rb + p;
 #pragma unroll
 				for (int s = 0; s < E; s++) x[G * s] = v[s];
@@ -500,13 +500,13 @@ __global__ __launch_bounds__(big::TB<R>) void k_i3fold_big(I3FoldArgs a)
 				cx<R> v[E];
 #pragma unroll
 				for (int u = 0; u < E; u++) v[u] = x[u * P];
-				line_bwd<R, P, G, E>(v, p, tw);
+				line16_bwd<R, P, E>(v, p, tw);
 #pragma unroll
 				for (int s = 0; s < E; s++) {
 					v[s].x *= m[s];
 					v[s].y *= m[s];
 				}
-				line_fwd<R, P, G, E>(v, p, tw);
+				line16_fwd<R, P, E>(v, p, tw);
 #pragma unroll
 				for (int u = 0; u < E; u++) x[u * P] = v[u];
 			}
@@ -525,7 +525,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_i3fold_big(I3FoldArgs a)
 				cx<R> v[E];
 #pragma unroll
 				for (int s = 0; s < E; s++) v[s] = x[G * s];
-				line_fwd<R, P, G, E>(v, p, tw);
+				line16_fwd<R, P, E>(v, p, tw);
 				const R ei = eta_sgn<R>(in);
 				const cx<R>* Ff = uni(Fq, (long long)(PAIR ? in >> 1 : in) * PP) + rb + r0;
 				const cx<R>* Sg = uni(Sj, 0) + rb + r0;
@@ -559,7 +559,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_i3fold_big(I3FoldArgs a)
 					for (int u = 0; u < E; u++) v[u] = cscale<R>(cmul<R>(Sg[u], v[u]), ej);
 				}
 				// row IFFT of the mirror grid into a scratch row that this line has read already
-				line_bwd<R, P, G, E>(v, p, tw);
+				line16_bwd<R, P, E>(v, p, tw);
 				cx<R>* y = uni(xs, (long long)(PAIR ? in >> 1 : in) * PP) + rb + p;
 #pragma unroll
 				for (int s = 0; s < E; s++)
@@ -583,7 +583,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_i3fold_big(I3FoldArgs a)
 				cx<R> v[E];
 #pragma unroll
 				for (int u = 0; u < E; u++) v[u] = x[u * P];
-				line_bwd<R, P, G, E>(v, p, tw);
+				line16_bwd<R, P, E>(v, p, tw);
 				cx<R>* d = uni(Dp, g * dstep) + MB::idx(c);
 				const cx<R> pk = ph[N + 1 + phase_idx<N>(c)];
 #pragma unroll
@@ -613,7 +613,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_combine_big(CombineArgs a)
 	load_twiddles_g<R, P, G, T>(tw, a.tw256);
 	const int o = blockIdx.x % a.nout;
 	const int cell = blockIdx.x / a.nout;
-	const int lt = threadIdx.x / G, p = threadIdx.x % G;
+	const int lt = threadIdx.x / G, p = dpp_p(threadIdx.x % G);
 	cx<R>* xs = (cx<R>*)a.xs + (size_t)blockIdx.x * PP;
 	const int r0 = blk(p);
 	__syncthreads();
@@ -644,7 +644,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_combine_big(CombineArgs a)
 				v[u].y += cf * y.y;
 			}
 		}
-		line_bwd<R, P, G, E>(v, p, tw);
+		line16_bwd<R, P, E>(v, p, tw);
 #pragma unroll
 		for (int s = 0; s < E; s++) xs[rb + p + G * s] = v[s];
 	}
@@ -661,7 +661,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_combine_big(CombineArgs a)
 		cx<R> v[E];
 #pragma unroll
 		for (int u = 0; u < E; u++) v[u] = xs[(r0 + u) * P + c];
-		line_bwd<R, P, G, E>(v, p, tw);
+		line16_bwd<R, P, E>(v, p, tw);
 #pragma unroll
 		for (int s = 0; s < E; s++) {
 			const int ln = unpad<N>(p + G * s);

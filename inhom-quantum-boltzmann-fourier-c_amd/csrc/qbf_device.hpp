@@ -4,12 +4,13 @@
 // one workgroup of T threads.  G = T / P threads share one "line" (a row or a
 // column); each thread holds E = P / G elements of its line in registers.
 // Four register layouts are used:
-//   R_i  line = row l,    thread p holds k = p + G*s          (s < E)  interleaved
-//   R_b  line = row l,    thread p holds k = E*brev_G(p) + u  (u < E)  blocked
+//   R_i  line = row l,    thread p holds k = p + G*s                     (s < E)  interleaved
+//   R_b  line = row l,    thread p holds k = blk_lane(p) + blk_reg(u)    (u < E)  blocked
 //   C_i  line = column k, thread p holds l = p + G*s
-//   C_b  line = column k, thread p holds l = E*brev_G(p) + u
+//   C_b  line = column k, thread p holds l = blk_lane(p) + blk_reg(u)
+// (see LineMap)
 // A forward line FFT maps an interleaved layout to the blocked one (in-register
-// DFT of length E, twiddle, radix-2 butterflies across the G lanes of the line);
+// DFT of length E, twiddle, DFT of length G across the lanes of the line);
 // the backward line FFT maps blocked to interleaved.  Rows and columns are
 // exchanged through LDS (R_i -> C_b and C_b -> R_i only).  Grids that live in
 // global memory between kernels are stored in "native" order: element u of
@@ -121,8 +122,48 @@ __device__ __forceinline__ cx<R> twmul(cx<R> c, int j, int m)
 	return mk<R>(c.x * cr - c.y * si, c.x * si + c.y * cr);
 }
 
+// Radix-2 butterfly with a constant twiddle: a +- b exp(SIGN 2 pi i j / m), j < m / 2 (constants after
+// unrolling).  FACTORED: a twiddle c (1 + i r), or i s (1 - i r) where |sin| > |cos|, takes two FMAs for the
+// factor in brackets, two additions for an eighth of a turn, and four FMAs for the sums with c or s, 6
+// operations instead of 8; |r| <= 1, so nothing is magnified.  For the VALU-bound FP32 grids of N <= 64 (step
+// of 512 cells at N = 64: 187.6 ms, 192.9 without; the same error).  With it the error of FP64 Strang steps at N = 32
+// was 3.2e-16 instead of 3.0e-16, and FP32 steps at N = 128 took 47.4 instead of 45.6 ms.
+template <typename R, int SIGN, bool FACTORED>
+__device__ __forceinline__ void bfly(cx<R>& a, cx<R>& b, int j, int m)
+{
+	if (j == 0 || 4 * j == m || !FACTORED) {
+		const cx<R> t = twmul<R, SIGN>(b, j, m);
+		b = csub<R>(a, t);
+		a = cadd<R>(a, t);
+		return;
+	}
+	const double wc = Tw64::c[j * (64 / m)], ws = SIGN * Tw64::s(j * (64 / m));
+	const bool eighth = 8 * j == m || 8 * j == 3 * m;
+	const bool big = eighth || (wc < 0 ? -wc : wc) > (ws < 0 ? -ws : ws);
+	R q, tx, ty;
+	if (big) {                                 // w = c (1 + i r)
+		q = (R)wc;
+		if (eighth) {
+			const bool neg = (wc < 0) != (ws < 0);
+			tx = neg ? b.x + b.y : b.x - b.y;
+			ty = neg ? b.y - b.x : b.y + b.x;
+		} else {
+			const R r = (R)(ws / wc);
+			tx = fma(-r, b.y, b.x);
+			ty = fma(r, b.x, b.y);
+		}
+	} else {                                   // w = s (r + i)
+		q = (R)ws;
+		const R r = (R)(wc / ws);
+		tx = fma(r, b.x, -b.y);
+		ty = fma(r, b.y, b.x);
+	}
+	b = mk<R>(fma(-q, tx, a.x), fma(-q, ty, a.y));
+	a = mk<R>(fma(q, tx, a.x), fma(q, ty, a.y));
+}
+
 // In-register DFT of length E (power of two <= 64), natural order in and out.
-template <typename R, int E, int SIGN>
+template <typename R, int E, int SIGN, bool FACTORED = false>
 __device__ __forceinline__ void dft(cx<R>* v)
 {
 	if constexpr (E > 1) {
@@ -134,12 +175,7 @@ __device__ __forceinline__ void dft(cx<R>* v)
 #pragma unroll
 			for (int b = 0; b < E; b += m) {
 #pragma unroll
-				for (int j = 0; j < m / 2; j++) {
-					const cx<R> t = twmul<R, SIGN>(w[b + j + m / 2], j, m);
-					const cx<R> a = w[b + j];
-					w[b + j] = cadd<R>(a, t);
-					w[b + j + m / 2] = csub<R>(a, t);
-				}
+				for (int j = 0; j < m / 2; j++) bfly<R, SIGN, FACTORED>(w[b + j], w[b + j + m / 2], j, m);
 			}
 		}
 #pragma unroll
@@ -147,46 +183,150 @@ __device__ __forceinline__ void dft(cx<R>* v)
 	}
 }
 
-// Exchange a 32-bit value with lane (lane ^ m).  m is a compile-time constant after
-// unrolling: lane distances 1 and 2 use DPP quad permutes (VALU, no LDS traffic),
-// 4, 8, 16 the ds_swizzle xor mode, 32 a bpermute.
-__device__ __forceinline__ int xor_lane_i32(int x, int m)
+// The 16 lanes of a line at N = 128: bit h of p flips with a DPP permutation of them.  The xor masks 1 and
+// 2 (quad permutes), 7 (half-row mirror) and 15 (row mirror) span the 16 lanes, so lane l has p = dpp_p(l)
+// and its partner p ^ h is one DPP operand away for every h (with p = l, lane distances 4 and 8 went
+// through the LDS unit).  FP32 Strang step of 32 cells 49.5 -> 45.6 ms.
+__host__ __device__ __forceinline__ constexpr int dpp_p(int l) { return l ^ (l & 4 ? 3 : 0) ^ (l & 8 ? 4 : 0); }
+
+template <int H>
+__device__ __forceinline__ int partner_i32(int x)
 {
-	switch (m) {
-	case 1: return __builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, false);   // quad_perm [1,0,3,2]
-	case 2: return __builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, false);   // quad_perm [2,3,0,1]
-	case 4: return __builtin_amdgcn_ds_swizzle(x, 0x101F);               // and 0x1f, xor 4
-	case 8: return __builtin_amdgcn_ds_swizzle(x, 0x201F);
-	case 16: return __builtin_amdgcn_ds_swizzle(x, 0x401F);
-	default: return __shfl_xor(x, m);
-	}
+	if constexpr (H == 1) return __builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, false);        // quad_perm [1,0,3,2]
+	else if constexpr (H == 2) return __builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, false);   // quad_perm [2,3,0,1]
+	else if constexpr (H == 4) return __builtin_amdgcn_mov_dpp(x, 0x141, 0xF, 0xF, false);  // row_half_mirror
+	else return __builtin_amdgcn_mov_dpp(x, 0x140, 0xF, 0xF, false);                        // row_mirror
 }
-__device__ __forceinline__ float xor_lane(float x, int m) { return __int_as_float(xor_lane_i32(__float_as_int(x), m)); }
-__device__ __forceinline__ double xor_lane(double x, int m)
+template <int H>
+__device__ __forceinline__ double partner(double x)
 {
-	const long long b = __double_as_longlong(x);
-	const int lo = xor_lane_i32((int)(b & 0xffffffffLL), m);
-	const int hi = xor_lane_i32((int)(b >> 32), m);
-	return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+	return __hiloint2double(partner_i32<H>(__double2hiint(x)), partner_i32<H>(__double2loint(x)));
 }
 
-template <typename R>
-__device__ __forceinline__ cx<R> shfl_xor_c(cx<R> v, int m)
+// x += s * (x of the partner) for 8 floats, one v_fmac with a DPP operand each (the compiler leaves a
+// move and an FMA).  A DPP operand is read two wait states after it was written at the earliest: the
+// s_nop, since the compiler does not look into the block.  FIXED: a fixed point of the instruction order
+// (N = 128: 45.4 ms instead of 47.7 for a step of 32 cells; k_i3fold_pair at N = 64 spills with it, 658 ms
+// instead of 196 for a step of 512 cells).
+#define QBF_FMAC8(ASM, DPP) \
+	ASM("s_nop 1\n\t" \
+		"v_fmac_f32_dpp %0, %0, %8 " DPP " row_mask:0xf bank_mask:0xf\n\t" \
+		"v_fmac_f32_dpp %1, %1, %8 " DPP " row_mask:0xf bank_mask:0xf\n\t" \
+		"v_fmac_f32_dpp %2, %2, %8 " DPP " row_mask:0xf bank_mask:0xf\n\t" \
+		"v_fmac_f32_dpp %3, %3, %8 " DPP " row_mask:0xf bank_mask:0xf\n\t" \
+		"v_fmac_f32_dpp %4, %4, %8 " DPP " row_mask:0xf bank_mask:0xf\n\t" \
+		"v_fmac_f32_dpp %5, %5, %8 " DPP " row_mask:0xf bank_mask:0xf\n\t" \
+		"v_fmac_f32_dpp %6, %6, %8 " DPP " row_mask:0xf bank_mask:0xf\n\t" \
+		"v_fmac_f32_dpp %7, %7, %8 " DPP " row_mask:0xf bank_mask:0xf" \
+		: "+v"(v[0].x), "+v"(v[0].y), "+v"(v[1].x), "+v"(v[1].y), "+v"(v[2].x), "+v"(v[2].y), "+v"(v[3].x), "+v"(v[3].y) \
+		: "v"(s))
+template <int H, bool FIXED>
+__device__ __forceinline__ void fmac_partner4(float2* v, float s)
 {
-	return mk<R>(xor_lane(v.x, m), xor_lane(v.y, m));
+#define QBF_FMAC8_DPP(DPP) do { if constexpr (FIXED) QBF_FMAC8(asm volatile, DPP); else QBF_FMAC8(asm, DPP); } while (0)
+	if constexpr (H == 1) QBF_FMAC8_DPP("quad_perm:[1,0,3,2]");
+	else if constexpr (H == 2) QBF_FMAC8_DPP("quad_perm:[2,3,0,1]");
+	else if constexpr (H == 4) QBF_FMAC8_DPP("row_half_mirror");
+	else QBF_FMAC8_DPP("row_mirror");
+#undef QBF_FMAC8_DPP
 }
+#undef QBF_FMAC8
+
+// v += s * (v of lane p ^ H)
+template <typename R, int E, int H, bool FIXED = false>
+__device__ __forceinline__ void add_partner(cx<R>* v, R s)
+{
+	static_assert(H == 1 || H == 2 || H == 4 || H == 8, "one bit of p");
+	if constexpr (sizeof(R) == 4) {
+#pragma unroll
+		for (int u = 0; u < E; u += 4) fmac_partner4<H, FIXED>(v + u, s);
+	} else {
+#pragma unroll
+		for (int u = 0; u < E; u++) v[u] = mk<R>(fma(partner<H>(v[u].x), s, v[u].x), fma(partner<H>(v[u].y), s, v[u].y));
+	}
+}
+
+// x and y of the lanes with bit B (16 or 32) of the lane index: y of the lower lanes <-> x of the upper
+// ones.  Afterwards x holds the lower lane's values (its x in the lower, its y in the upper lane), y the
+// upper lane's: one instruction transposes the lane bit with the register index.
+template <int B>
+__device__ __forceinline__ void lane_swap(int& x, int& y)
+{
+	static_assert(B == 16 || B == 32, "row and half-wave swaps");
+	if constexpr (B == 16) {
+		const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+		x = r[0];
+		y = r[1];
+	} else {
+		const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+		x = r[0];
+		y = r[1];
+	}
+}
+template <int B>
+__device__ __forceinline__ void lane_swap(float& x, float& y)
+{
+	int a = __float_as_int(x), b = __float_as_int(y);
+	lane_swap<B>(a, b);
+	x = __int_as_float(a);
+	y = __int_as_float(b);
+}
+template <int B>
+__device__ __forceinline__ void lane_swap(double& x, double& y)
+{
+	int al = __double2loint(x), ah = __double2hiint(x), bl = __double2loint(y), bh = __double2hiint(y);
+	lane_swap<B>(al, bl);
+	lane_swap<B>(ah, bh);
+	x = __hiloint2double(ah, al);
+	y = __hiloint2double(bh, bl);
+}
+
+// Where the G = 4 or 8 lanes of a line sit in a wave, and the blocked order of their elements.  Bits 5
+// and 4 of the lane index are the two high bits of p, for G = 8 bit 0 is the low one; the other bits are
+// the line.  The transform over p then begins (ends) with the permlane swaps that exchange bits 5 and 4
+// with the two high bits of the register index: the four values of a DFT-4 over them are in one lane, with
+// no selects and no lane-dependent factors, and only the last radix-2 stage of G = 8 needs a partner.  A
+// swap moves two registers in the time of two moves (8.4 cycles against 4.3 of a DPP move or an FMA).
+//   With p in the low lane bits, a move, an FMA and (lane distance 4) an LDS swizzle per value and stage, a
+// line of 128 took 516 VALU and 32 LDS operations in FP32, now about 410 (swaps counted twice) and none,
+// and the lines of a phase of LDS accesses are consecutive.  FP32 Strang step, N = 64, 512 cells:
+// 204 -> 188 ms; FP64, N = 64, 16 cells: 42.5 -> 41.4; FP64, N = 16, simulation steps of 24 cells: 2.40 ->
+// 2.26; FP64, N = 32, 128 cells the same (bound by L2: a quarter fewer VALU operations gained nothing).  A
+// v_fmac with a DPP operand per float and stage in FP32, as at N = 128: 193.8 ms.
+template <int G, int E>
+struct LineMap {
+	static_assert(G == 4 || G == 8, "4 or 8 lanes a line");
+	static_assert(E % 4 == 0, "two bits of the register index change places with lane bits");
+	static constexpr int P = G * E;
+	// line and p of thread t
+	static __host__ __device__ __forceinline__ constexpr int line(int t)
+	{
+		return G == 8 ? (t >> 6) * 8 + ((t >> 1) & 7) : (t >> 6) * 16 + (t & 15);
+	}
+	static __host__ __device__ __forceinline__ constexpr int lane(int t)
+	{
+		return G == 8 ? 2 * ((t >> 4) & 3) + (t & 1) : (t >> 4) & 3;
+	}
+	// index of blocked element u of lane p: blk_lane(p) + blk_reg(u)
+	static __device__ __forceinline__ constexpr int blk_lane(int p)
+	{
+		return G == 8 ? (E / 4) * (p >> 1) + (P / 2) * (p & 1) : (E / 4) * p;
+	}
+	static __device__ __forceinline__ constexpr int blk_reg(int u) { return E * (u / (E / 4)) + u % (E / 4); }
+};
 
 // Geometry of one P x P grid per workgroup of T threads.
 template <int P_, int T_>
-struct Geo {
+struct Geo : LineMap<T_ / P_, P_ * P_ / T_> {
 	static constexpr int P = P_;
 	static constexpr int T = T_;
 	static constexpr int G = T_ / P_;       // threads per line
 	static constexpr int E = P_ / G;        // elements per thread
-	static constexpr int PITCH = P_ + G;    // LDS row pitch (elements), see Xpose
+	static constexpr int PITCH = P_ + G / 4; // LDS row pitch (elements), see Xpose
+	static constexpr int SKEW = G == 8 ? 8 : 0;
 	static_assert(G * P_ == T_, "T must be a multiple of P");
 	static_assert(G * E == P_, "G must divide P");
-	static_assert(G <= 64 && (64 % G) == 0, "a line must sit inside one wavefront");
+	static_assert(T_ % 64 == 0, "whole waves");
 };
 
 // Logical block index that keeps consecutive logical blocks on one XCD.  The dispatcher hands
@@ -247,105 +387,175 @@ struct TwTab {
 // of one read fall into distinct banks: entry u of lane p at G u + p.  (FP64, [p][u]: a fifth of the
 // I3 kernel's LDS cycles were conflicts.)
 
-// Forward FFT of one line: interleaved layout in, blocked layout out.
-// twP[j] = (cos, sin)(2 pi j / P), j < P; the per-lane table (cos, sin)(2 pi p u / P) follows it
-// (in LDS).
-template <typename R, int P, int G, int E>
-__device__ __forceinline__ void line_fwd(cx<R>* v, int p, const cx<R>* twP)
+// Exchange bits 5 and 4 of the lane index with the two high bits of the register index of v.
+template <typename R, int E>
+__device__ __forceinline__ void lane_transpose(cx<R>* v)
 {
-	dft<R, E, -1>(v);
-	if constexpr (G > 1) {
-		const cx<R>* tl = twP + P + p + opaque_zero();
+	constexpr int Q = E / 4;
 #pragma unroll
-		for (int u = 1; u < E; u++) v[u] = cmulc<R>(v[u], tl[G * u]);
+	for (int u = 0; u < 2 * Q; u++) {
+		lane_swap<32>(v[u].x, v[u + 2 * Q].x);
+		lane_swap<32>(v[u].y, v[u + 2 * Q].y);
+	}
 #pragma unroll
-		for (int h = G / 2; h >= 1; h >>= 1) {
-			// DIF butterfly across lanes p, p^h:  lo: a + b,  hi: (a - b) * conj(w)
-			// as  (partner + sgn * self) * wl  with lane constants sgn = +-1, wl = 1 or conj(w)
-			const bool hi = (p & h) != 0;
-			const R sgn = hi ? R(-1) : R(1);
-			if (h == 1) {                      // twiddle exp(0) = 1
+	for (int u = 0; u < Q; u++)
 #pragma unroll
-				for (int u = 0; u < E; u++) {
-					const cx<R> pv = shfl_xor_c<R>(v[u], h);
-					v[u] = mk<R>(pv.x + sgn * v[u].x, pv.y + sgn * v[u].y);
-				}
-			} else if (h == 2) {               // twiddle w^((p & 1) P / 4) = 1 or i
-				// the hi lanes with odd p multiply by conj(i) = -i: a swap and a sign (two selects)
-				const bool q = hi && (p & 1);
-#pragma unroll
-				for (int u = 0; u < E; u++) {
-					const cx<R> pv = shfl_xor_c<R>(v[u], h);
-					const cx<R> t = mk<R>(pv.x + sgn * v[u].x, pv.y + sgn * v[u].y);
-					v[u] = mk<R>(q ? t.y : t.x, q ? -t.x : t.y);
-				}
-			} else {
-				const cx<R> w = pin<R>(twP[2 * P + h + (p & (h - 1)) + opaque_zero()]);
-				const cx<R> wl = hi ? mk<R>(w.x, -w.y) : mk<R>(R(1), R(0));
-#pragma unroll
-				for (int u = 0; u < E; u++) {
-					const cx<R> pv = shfl_xor_c<R>(v[u], h);
-					const cx<R> t = mk<R>(pv.x + sgn * v[u].x, pv.y + sgn * v[u].y);
-					v[u] = cmul<R>(t, wl);
-				}
-			}
+		for (int h = 0; h < 4; h += 2) {
+			lane_swap<16>(v[h * Q + u].x, v[(h + 1) * Q + u].x);
+			lane_swap<16>(v[h * Q + u].y, v[(h + 1) * Q + u].y);
 		}
+}
+
+// DFT-4 over the two high bits of the register index, in place
+template <typename R, int E, int SIGN>
+__device__ __forceinline__ void dft4_high(cx<R>* v)
+{
+	constexpr int Q = E / 4;
+#pragma unroll
+	for (int u = 0; u < Q; u++) {
+		cx<R> w[4] = {v[u], v[Q + u], v[2 * Q + u], v[3 * Q + u]};
+		dft<R, 4, SIGN>(w);
+#pragma unroll
+		for (int q = 0; q < 4; q++) v[q * Q + u] = w[q];
 	}
 }
 
-// Backward FFT of one line: blocked layout in, interleaved layout out.
-template <typename R, int P, int G, int E>
+// v times exp(SIGN 2 pi i f / 8) in the upper lanes of a pair, f the two high bits of the register index
+template <typename R, int E, int SIGN>
+__device__ __forceinline__ void pair_twiddle(cx<R>* v, bool up)
+{
+	constexpr int Q = E / 4;
+	constexpr R H = (R)Tw64::c[8];
+	const R c1 = up ? H : R(1), s1 = up ? SIGN * H : R(0), c3 = up ? -H : R(1);
+#pragma unroll
+	for (int u = 0; u < Q; u++) {
+		const cx<R> a = v[Q + u], b = v[2 * Q + u], c = v[3 * Q + u];
+		v[Q + u] = mk<R>(a.x * c1 - a.y * s1, a.x * s1 + a.y * c1);
+		v[2 * Q + u] = SIGN < 0 ? mk<R>(up ? b.y : b.x, up ? -b.x : b.y) : mk<R>(up ? -b.y : b.x, up ? b.x : b.y);
+		v[3 * Q + u] = mk<R>(c.x * c3 - c.y * s1, c.x * s1 + c.y * c3);
+	}
+}
+
+// A radix-2 stage across lanes is v + s (v of the partner) with s = +-1: a + b in the lower lane p, b - a
+// of its own b in the upper lane p ^ h, the negative of the butterfly's a - b.  Where the upper lane's
+// values come in negated, s = -1 in the lower and +1 in the upper lane give a + b and a - b.  The signs
+// are in the lane-dependent factors that precede or follow the stages.
+
+// Forward FFT of one line: interleaved layout in, blocked layout out.
+// twP[j] = (cos, sin)(2 pi j / P), j < P; the per-lane table (cos, sin)(2 pi p u / P) follows it
+// (in LDS).  n = p + G s, p = (G / 4) g + b: a DFT-E over s, twiddles w^(p u), a DFT-4 over g (frequency
+// f), for G = 8 twiddles w8^(f b) and the sum over b (frequency c): k = u + E f + 4 E c with the high bits
+// of u in the lane.  G = 8: the upper lanes b = 1 are negated by the per-lane twiddles (load_twiddles_g)
+// and here for u = 0.
+template <typename R, class GE>
+__device__ __forceinline__ void line_fwd(cx<R>* v, int p, const cx<R>* twP)
+{
+	constexpr int P = GE::P, G = GE::G, E = GE::E;
+	dft<R, E, -1, sizeof(R) == 4>(v);
+	const cx<R>* tl = twP + P + p + opaque_zero();
+#pragma unroll
+	for (int u = 1; u < E; u++) v[u] = cmulc<R>(v[u], tl[G * u]);
+	const bool up = p & 1;
+	const R sgn = up ? R(-1) : R(1);
+	if constexpr (G == 8) v[0] = cscale<R>(v[0], sgn);
+	lane_transpose<R, E>(v);
+	dft4_high<R, E, -1>(v);
+	if constexpr (G == 8) {
+		pair_twiddle<R, E, -1>(v, up);
+		add_partner<R, E, 1>(v, -sgn);
+	}
+}
+
+// Backward FFT of one line: blocked layout in, interleaved layout out; the same stages in the opposite
+// order (the stage over c leaves the upper lanes negated).
+template <typename R, class GE>
 __device__ __forceinline__ void line_bwd(cx<R>* v, int p, const cx<R>* twP)
 {
-	if constexpr (G > 1) {
-#pragma unroll
-		for (int h = 1; h < G; h <<= 1) {
-			// DIT butterfly across lanes p, p^h:  lo: a + w b,  hi: a - w b  (a on lo, b on hi):
-			// the hi lane pre-multiplies its own value by w, then  partner' + sgn * self'
-			const bool hi = (p & h) != 0;
-			const R sgn = hi ? R(-1) : R(1);
-			if (h == 1) {                      // twiddle exp(0) = 1
-#pragma unroll
-				for (int u = 0; u < E; u++) {
-					const cx<R> pv = shfl_xor_c<R>(v[u], h);
-					v[u] = mk<R>(pv.x + sgn * v[u].x, pv.y + sgn * v[u].y);
-				}
-			} else if (h == 2) {               // twiddle w^((p & 1) P / 4) = 1 or i
-				// the hi lanes with odd p pre-multiply by i: a swap and a sign (two selects)
-				const bool q = hi && (p & 1);
-#pragma unroll
-				for (int u = 0; u < E; u++) {
-					const cx<R> sv = mk<R>(q ? -v[u].y : v[u].x, q ? v[u].x : v[u].y);
-					const cx<R> pv = shfl_xor_c<R>(sv, h);
-					v[u] = mk<R>(pv.x + sgn * sv.x, pv.y + sgn * sv.y);
-				}
-			} else {
-				const cx<R> w = pin<R>(twP[2 * P + h + (p & (h - 1)) + opaque_zero()]);
-				const cx<R> wl = hi ? w : mk<R>(R(1), R(0));
-#pragma unroll
-				for (int u = 0; u < E; u++) {
-					const cx<R> sv = cmul<R>(v[u], wl);
-					const cx<R> pv = shfl_xor_c<R>(sv, h);
-					v[u] = mk<R>(pv.x + sgn * sv.x, pv.y + sgn * sv.y);
-				}
-			}
-		}
-		const cx<R>* tl = twP + P + p + opaque_zero();
-#pragma unroll
-		for (int u = 1; u < E; u++) v[u] = cmul<R>(v[u], tl[G * u]);
+	constexpr int P = GE::P, G = GE::G, E = GE::E;
+	const bool up = p & 1;
+	const R sgn = up ? R(-1) : R(1);
+	if constexpr (G == 8) {
+		add_partner<R, E, 1>(v, sgn);
+		pair_twiddle<R, E, +1>(v, up);
 	}
+	dft4_high<R, E, +1>(v);
+	lane_transpose<R, E>(v);
+	const cx<R>* tl = twP + P + p + opaque_zero();
+	if constexpr (G == 8) v[0] = cscale<R>(v[0], sgn);
+#pragma unroll
+	for (int u = 1; u < E; u++) v[u] = cmul<R>(v[u], tl[G * u]);
+	dft<R, E, +1, sizeof(R) == 4>(v);
+}
+
+// (-1)^(bits 0 and 1 of p)
+template <typename R>
+__device__ __forceinline__ R low_parity(int p) { return (p ^ (p >> 1)) & 1 ? R(-1) : R(1); }
+
+// The factor of a stage H >= 4: the twiddle exp(SIGN 2 pi i (p mod H) / 2H) in the upper lanes, negated there,
+// and the sign s
+template <typename R, int P, int H, int SIGN>
+__device__ __forceinline__ cx<R> stage_factor(int p, const cx<R>* twP, R s)
+{
+	const cx<R> w = pin<R>(twP[2 * P + H + (p & (H - 1)) + opaque_zero()]);
+	return p & H ? mk<R>(-s * w.x, SIGN * -s * w.y) : mk<R>(s, R(0));
+}
+
+// Lines of P = 16 E elements over 16 consecutive lanes (dpp_p), the blocked element u of lane p being
+// k = E brev(p) + u: radix-2 stages over the bits of p
+template <typename R, int P, int E>
+__device__ __forceinline__ void line16_fwd(cx<R>* v, int p, const cx<R>* twP)
+{
+	dft<R, E, -1>(v);
+	const cx<R>* tl = twP + P + p + opaque_zero();
+#pragma unroll
+	for (int u = 1; u < E; u++) v[u] = cmulc<R>(v[u], tl[16 * u]);
+	// before the last two stages the lanes carry the sign low_parity
+	add_partner<R, E, 8, true>(v, p & 8 ? R(-1) : R(1));
+	const cx<R> w8 = stage_factor<R, P, 8, -1>(p, twP, R(1));
+#pragma unroll
+	for (int u = 0; u < E; u++) v[u] = cmul<R>(v[u], w8);
+	add_partner<R, E, 4, true>(v, p & 4 ? R(-1) : R(1));
+	const cx<R> w4 = stage_factor<R, P, 4, -1>(p, twP, low_parity<R>(p));
+#pragma unroll
+	for (int u = 0; u < E; u++) v[u] = cmul<R>(v[u], w4);
+	add_partner<R, E, 2, true>(v, p & 2 ? R(1) : R(-1));
+	// twiddle 1 or -i: a swap and a sign (two selects)
+	const bool q = (p & 3) == 3;
+#pragma unroll
+	for (int u = 0; u < E; u++) v[u] = mk<R>(q ? v[u].y : v[u].x, q ? -v[u].x : v[u].y);
+	add_partner<R, E, 1, true>(v, p & 1 ? R(1) : R(-1));
+}
+
+template <typename R, int P, int E>
+__device__ __forceinline__ void line16_bwd(cx<R>* v, int p, const cx<R>* twP)
+{
+	// after the first two stages the lanes carry the sign low_parity
+	add_partner<R, E, 1, true>(v, p & 1 ? R(-1) : R(1));
+	const bool q = (p & 3) == 3;
+#pragma unroll
+	for (int u = 0; u < E; u++) v[u] = mk<R>(q ? -v[u].y : v[u].x, q ? v[u].x : v[u].y);
+	add_partner<R, E, 2, true>(v, p & 2 ? R(-1) : R(1));
+	const cx<R> w4 = stage_factor<R, P, 4, +1>(p, twP, low_parity<R>(p));
+#pragma unroll
+	for (int u = 0; u < E; u++) v[u] = cmul<R>(v[u], w4);
+	add_partner<R, E, 4, true>(v, p & 4 ? R(1) : R(-1));
+	const cx<R> w8 = stage_factor<R, P, 8, +1>(p, twP, R(1));
+#pragma unroll
+	for (int u = 0; u < E; u++) v[u] = cmul<R>(v[u], w8);
+	add_partner<R, E, 8, true>(v, p & 8 ? R(1) : R(-1));
+	const cx<R>* tl = twP + P + p + opaque_zero();
+#pragma unroll
+	for (int u = 1; u < E; u++) v[u] = cmul<R>(v[u], tl[16 * u]);
 	dft<R, E, +1>(v);
 }
 
-// LDS exchanges.  The grid is stored row-major with pitch P + G and a skew of SKEW elements
-// per block of E rows.  An 8-byte LDS access of a wave is served 128 bytes per phase: LANES
-// consecutive lanes of one element each, conflict-free when their addresses are distinct modulo
-// LANES elements.  (Measured with SQ_LDS_BANK_CONFLICT of k_i3acc for the column skews of the
-// 512-, 256- and 128-byte phase models: 1.31e7, 4.72e6 and 5.2e5 cycles; lane-linear and stride-2
-// probes do not tell the models apart.)  Writes / reads of rows (R_i) hit LANES/G consecutive
-// rows times G consecutive columns: distinct because the pitch is G modulo LANES.  Writes /
-// reads of columns (C_b) hit LANES/G consecutive columns in G row blocks E rows apart: E*pitch
-// is a multiple of LANES, and the per-block skew LANES/G separates the blocks.
+// LDS exchanges.  The grid is stored row-major.  An 8-byte LDS access of a wave is served 128 bytes
+// per phase: 16 consecutive lanes of one element each, conflict-free when their addresses are
+// distinct modulo 16 elements (measured with SQ_LDS_BANK_CONFLICT of k_i3acc; 16-byte elements: 8 lanes).
+//   G = 4: the lanes of a phase have one p and consecutive lines, in the accesses of columns (C_b)
+// consecutive elements, in those of rows (R_i) the pitch apart, P + 1.  G = 8: eight consecutive lines with
+// the two lanes of a pair, one element (rows) or P / 2 rows (columns) apart: pitch P + 2, and the rows from
+// P / 2 on are skewed by 8.
 //
 // SPLIT: a grid that does not fit in the 160 KiB of LDS whole (FP64 128 x 128: 256 KiB) goes through
 // it in two halves, real parts then imaginary parts: each half is the same grid of 8-byte elements,
@@ -356,12 +566,13 @@ __device__ __forceinline__ void line_bwd(cx<R>* v, int p, const cx<R>* twP)
 template <typename R, class GE, bool SPLIT = false>
 struct Xpose {
 	using El = typename std::conditional<SPLIT, R, cx<R>>::type;
-	static constexpr int LANES = 128 / (int)sizeof(El);
-	static constexpr int SKEW = LANES / GE::G;
-	static constexpr int SIZE = GE::P * GE::PITCH + GE::G * SKEW;
+	static constexpr int SIZE = GE::P * GE::PITCH + GE::SKEW;
 	El* g0;
 	__device__ __forceinline__ El* gp() const { return g0 + opaque_zero(); }
-	__device__ __forceinline__ int a(int row, int col) const { return row * GE::PITCH + col + (row / GE::E) * SKEW; }
+	__device__ __forceinline__ int a(int row, int col) const { return row * GE::PITCH + col + (row / (GE::P / 2)) * GE::SKEW; }
+	// blocked element u of a column, c0 = col_base(line, p) (all of a lane's rows have its element 0's skew)
+	__device__ __forceinline__ int blk(int c0, int u) const { return c0 + GE::blk_reg(u) * GE::PITCH; }
+	__device__ __forceinline__ int col_base(int line, int p) const { return a(GE::blk_lane(p), line); }
 	static __device__ __forceinline__ void out(El& e, cx<R> v, int c)
 	{
 		if constexpr (SPLIT) e = c ? v.y : v.x;
@@ -394,15 +605,15 @@ struct Xpose {
 	}
 	__device__ __forceinline__ void put_Cb(El* g, const cx<R>* v, int line, int p, int c) const
 	{
-		const int r0 = GE::E * brev<GE::G>(p);
+		const int c0 = col_base(line, p);
 #pragma unroll
-		for (int u = 0; u < GE::E; u++) out(g[a(r0 + u, line)], v[u], c);
+		for (int u = 0; u < GE::E; u++) out(g[blk(c0, u)], v[u], c);
 	}
 	__device__ __forceinline__ void get_Cb(const El* g, cx<R>* v, int line, int p, int c) const
 	{
-		const int r0 = GE::E * brev<GE::G>(p);
+		const int c0 = col_base(line, p);
 #pragma unroll
-		for (int u = 0; u < GE::E; u++) in(v[u], g[a(r0 + u, line)], c);
+		for (int u = 0; u < GE::E; u++) in(v[u], g[blk(c0, u)], c);
 	}
 	__device__ __forceinline__ void get_Ri(const El* g, cx<R>* v, int line, int p, int c) const
 	{
@@ -421,7 +632,8 @@ struct Xpose {
 };
 
 // Fill the LDS twiddle tables from a global table of (cos, sin)(2 pi j / 256) in double:
-// twP[j] = w^j for j < P, the per-lane table w^(p*u) at twP[P + G u + p], and the
+// twP[j] = w^j for j < P, the per-lane table w^(p*u) at twP[P + G u + p] (G = 8:
+// negated for odd p, see line_fwd), and the
 // twiddles of the cross-lane stages at twP[2P + h + m] = w^(m P / 2h), m < h < G, kept apart so
 // that the lanes of one stage read consecutive entries; w = exp(2 pi i / P).
 // (load_twiddles_g: G lanes per line, filled by the NT threads of the workgroup)
@@ -441,7 +653,8 @@ __device__ __forceinline__ void load_twiddles_g(cx<R>* twP, const double2* tw256
 			k = i == 0 ? 0 : (i - h) * (P / (2 * h));
 		}
 		const double2 w = tw256[k * (256 / P)];
-		twP[j] = mk<R>((R)w.x, (R)w.y);
+		const double sg = G == 8 && j >= P && j < 2 * P && (j & 1) ? -1.0 : 1.0;
+		twP[j] = mk<R>((R)(sg * w.x), (R)(sg * w.y));
 	}
 }
 template <typename R, int P, int T>

@@ -311,7 +311,7 @@ struct EngineT final : public qbf_engine {
 	static constexpr bool SP = Cfg<R, N>::SP;
 	static constexpr bool BIG = N == 128;        // P = 256 kernels of qbf_big.hip, natural grid order
 	static_assert(!BIG || T == big::TB<R>, "launch size of the N = 128 kernels");
-	using GE = Geo<P, T>;
+	using GE = typename std::conditional<BIG, Geo<128, 1024>, Geo<P, T>>::type;   // (not used at N = 128)
 	using C = cx<R>;
 	static constexpr size_t GB = sizeof(C) * PP;    // bytes of one padded grid
 		// workgroups of the fold kernels resident at once: 16 waves a CU, 8 at FP64 N = 32 (registers)
@@ -362,7 +362,7 @@ struct EngineT final : public qbf_engine {
 			return;
 		}
 		for (int t = 0; t < T; t++) {
-			const int line = t / GE::G, p = t % GE::G;
+			const int line = GE::line(t), p = GE::lane(t);
 			for (int s = 0; s < GE::E; s++) {
 				const int l = p + GE::G * s, k = line;
 				out[(size_t)s * T + t] = (R)tab[k + (size_t)P * l];
@@ -556,7 +556,7 @@ struct EngineT final : public qbf_engine {
 		if (!r && nmir) r = upload(i3ph, ph.data(), sizeof(C) * ph.size());
 		if (r) return r;
 		if (mfmaI3) {
-			// k_i3acc_mfma's order: psi2 of row 16 w + i16, column 4 kq + r + 16 t at
+			// k_i3acc_mfma's order: psi2 of column 16 w + i16, row 4 kq + r + 16 t at
 			// ((w * 8 + t) * 4 + r) * 64 + 16 kq + i16
 			static_assert(P == mf::P || N != 64, "the matrix-core kernel is built for P = 128");
 			std::vector<float> p2m((size_t)num * PP);
@@ -565,7 +565,7 @@ struct EngineT final : public qbf_engine {
 					for (int t = 0; t < 8; t++)
 						for (int rr = 0; rr < 4; rr++)
 							for (int ln = 0; ln < 64; ln++) {
-								const int l = 16 * w + (ln & 15), k = 4 * (ln >> 4) + rr + 16 * t;
+								const int k = 16 * w + (ln & 15), l = 4 * (ln >> 4) + rr + 16 * t;
 								p2m[(size_t)q * PP + ((w * 8 + t) * 4 + rr) * 64 + ln] =
 									(float)p2[(size_t)order[q] * PP + k + (size_t)P * l];
 							}

@@ -38,7 +38,7 @@ __device__ __forceinline__ void mirror_add(cx<R>* v, const XP& X, const cx<R>* t
 	using MB = MirrorBox<N, G, E, EDGE>;
 	line = opaque_lane(line);
 	p = opaque_lane(p);
-	line_bwd<R, P, G, E>(v, p, tw);
+	line_bwd<R, GE>(v, p, tw);
 	// whole waves skip the column pass (a branch that the compiler can see is uniform): they go on to the
 	// next product's row pass meanwhile
 	constexpr int LW = 64 / G;                  // lines per wave
@@ -52,11 +52,11 @@ __device__ __forceinline__ void mirror_add(cx<R>* v, const XP& X, const cx<R>* t
 		},
 		[&](const El* g, int c) { if (box) X.get_Cb(g, v, line, p, c); });
 	if (!box) return;
-	line_bwd<R, P, G, E>(v, p, tw);
+	line_bwd<R, GE>(v, p, tw);
 	__builtin_amdgcn_sched_barrier(0);
 	const bool keep = unpad<N>(line) >= 0 || (EDGE && line == N / 2);
 	const BufRef<cx<R>> Dr(Dp, MB::SIZE);
-	const int d0 = keep ? MB::idx(line) * G + p : 0;
+	const int d0 = keep ? MB::lane(line, p) : 0;
 	const cx<R> pk = ph[N + 1 + (keep ? phase_idx<N>(line) : 0)];
 	constexpr int NB = E / 2 + EDGE;            // elements in the box, EDGE: the last one in lane 0 only
 	constexpr int BL = 4;                       // loads in flight together
@@ -185,7 +185,7 @@ __global__ __launch_bounds__(T, (FOLD_WPE<R, N>)) void k_i3fold(I3FoldArgs a)
 	const FoldRange w(a, 4);
 	const int j = w.grp;
 	const int t = threadIdx.x;
-	const int line = t / G, p = t % G;
+	const int line = GE::line(t), p = GE::lane(t);
 	const size_t dstep = (size_t)4 * a.nchunk * a.nblk * MB::SIZE;
 	cx<R>* Dp = (cx<R>*)a.D + 4 * w.cell * dstep + (size_t)((j * a.nchunk + w.chunk) * a.nblk + a.blk0 - 1) * MB::SIZE;
 	int nb = 0;                                 // blocks begun
@@ -262,7 +262,7 @@ __global__ __launch_bounds__(T, (FOLD_WPE<R, N>)) void k_i3fold_pair(I3FoldArgs 
 	const FoldRange w(a, 4);
 	const int J = w.grp >> 1, pr = w.grp & 1;
 	const int t = threadIdx.x;
-	const int line = t / G, p = t % G;
+	const int line = GE::line(t), p = GE::lane(t);
 	cx<R>* Dp = (cx<R>*)a.D + ((((size_t)w.cell * 2 + pr) * 2 + J) * a.nchunk + w.chunk) * a.nblk * MB::SIZE +
 		(long long)(a.blk0 - 1) * MB::SIZE;
 	int nb = 0;                                 // blocks begun

@@ -61,7 +61,7 @@ __device__ __forceinline__ void padfft_reg(cx<R>* v, const double2* __restrict__
 				v[s] = czero<R>();
 			}
 		}
-		line_fwd<R, P, G, E>(v, p, tw);
+		line_fwd<R, GE>(v, p, tw);
 	}
 	X.pass([&](El* g, int c) { if (kn >= 0) X.put_Cb(g, v, line, p, c); },
 		[&](const El* g, int c) {
@@ -72,7 +72,7 @@ __device__ __forceinline__ void padfft_reg(cx<R>* v, const double2* __restrict__
 #pragma unroll
 	for (int s = 0; s < E; s++)
 		if (!padded_nonzero<E>(s)) v[s] = czero<R>();
-	line_fwd<R, P, G, E>(v, p, tw);
+	line_fwd<R, GE>(v, p, tw);
 }
 
 // R_b (physical) -> IFFT2 -> C_i (frequency)
@@ -80,9 +80,9 @@ template <typename R, class GE, class XP>
 __device__ __forceinline__ void ifft2_reg(cx<R>* v, const XP& X, const cx<R>* tw, int line, int p)
 {
 	constexpr int G = GE::G, E = GE::E, P = GE::P;
-	line_bwd<R, P, G, E>(v, p, tw);
+	line_bwd<R, GE>(v, p, tw);
 	X.RiCb(v, line, p);
-	line_bwd<R, P, G, E>(v, p, tw);
+	line_bwd<R, GE>(v, p, tw);
 }
 
 // C_i (frequency) -> FFT2 -> R_b (physical)
@@ -90,9 +90,9 @@ template <typename R, class GE, class XP>
 __device__ __forceinline__ void fft2_reg(cx<R>* v, const XP& X, const cx<R>* tw, int line, int p)
 {
 	constexpr int G = GE::G, E = GE::E, P = GE::P;
-	line_fwd<R, P, G, E>(v, p, tw);
+	line_fwd<R, GE>(v, p, tw);
 	X.CbRi(v, line, p);
-	line_fwd<R, P, G, E>(v, p, tw);
+	line_fwd<R, GE>(v, p, tw);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -109,7 +109,7 @@ __global__ __launch_bounds__(T) void k_padfft(PadFFTArgs a)
 	__shared__ cx<R> tw[TwTab<P, T>::SIZE];
 	load_twiddles<R, P, T>(tw, a.tw256);
 	const int o0 = 2 * blockIdx.x;
-	const int line = threadIdx.x / G, p = threadIdx.x % G;
+	const int line = GE::line(threadIdx.x), p = GE::lane(threadIdx.x);
 	const int o = o0 + line / N, kn = line % N;
 	XP X{lds};
 	cx<R> v[E];
@@ -138,7 +138,7 @@ __global__ __launch_bounds__(T) void k_padfft(PadFFTArgs a)
 				v[s] = czero<R>();
 			}
 		}
-		line_fwd<R, P, G, E>(v, p, tw);
+		line_fwd<R, GE>(v, p, tw);
 	}
 	// the non-zero elements of this line's row of either grid
 	using El = typename XP::El;
@@ -155,7 +155,7 @@ __global__ __launch_bounds__(T) void k_padfft(PadFFTArgs a)
 		if (o0 + k >= a.ngrid) break;
 #pragma unroll
 		for (int s = 0; s < E; s++) v[s] = padded_nonzero<E>(s) ? r[k][s < E / 4 ? s : s - E / 2] : czero<R>();
-		line_fwd<R, P, G, E>(v, p, tw);
+		line_fwd<R, GE>(v, p, tw);
 		store_native<R, GE>((cx<R>*)a.out + (size_t)(o0 + k) * (P * P), v);
 	}
 }
@@ -176,7 +176,7 @@ __global__ __launch_bounds__(T) void k_i1acc(I1Args a)
 	const int cell = lb / (a.nchunk * a.ninst);
 	const int qa = (int)(((long long)chunk * a.nterm) / a.nchunk);
 	const int qb = (int)(((long long)(chunk + 1) * a.nterm) / a.nchunk);
-	const int line = threadIdx.x / GE::G, p = threadIdx.x % GE::G;
+	const int line = GE::line(threadIdx.x), p = GE::lane(threadIdx.x);
 	const double2* g = a.src + ((size_t)cell * a.nsrc + a.instSrc[inst]) * (N * N);
 	const cx<R>* Fh = (const cx<R>*)a.Fhat + ((size_t)cell * a.nFh + a.instFh[inst]) * (P * P);
 	const R fa = (R)a.fa, fb = (R)a.fb;
@@ -225,7 +225,7 @@ __global__ __launch_bounds__(T) void k_i2acc(I2Args a)
 	const int cell = lb / (a.nchunk * a.ninst);
 	const int qa = (int)(((long long)chunk * a.nterm) / a.nchunk);
 	const int qb = (int)(((long long)(chunk + 1) * a.nterm) / a.nchunk);
-	const int line = threadIdx.x / GE::G, p = threadIdx.x % GE::G;
+	const int line = GE::line(threadIdx.x), p = GE::lane(threadIdx.x);
 	const double2* f = a.src + ((size_t)cell * a.nsrc + a.instF[inst]) * (N * N);
 	const double2* g = a.src + ((size_t)cell * a.nsrc + a.instG[inst]) * (N * N);
 	XP X{lds};
@@ -272,7 +272,7 @@ __global__ __launch_bounds__(T) void k_i3acc(I3Args a)
 	const int chunk = lb % a.nchunk;
 	const int out = (lb / a.nchunk) % a.nout;
 	const int cell = lb / (a.nchunk * a.nout);
-	const int line = threadIdx.x / GE::G, p = threadIdx.x % GE::G;
+	const int line = GE::line(threadIdx.x), p = GE::lane(threadIdx.x);
 	const int t = threadIdx.x;
 	const int qa = (int)(((long long)chunk * a.nq) / a.nchunk);
 	const int qb = (int)(((long long)(chunk + 1) * a.nq) / a.nchunk);
@@ -358,7 +358,7 @@ __global__ __launch_bounds__(T) void k_padfft_loop(PadFFTArgs a)
 	__shared__ typename XP::El lds[XP::SIZE];
 	__shared__ cx<R> tw[TwTab<P, T>::SIZE];
 	load_twiddles<R, P, T>(tw, a.tw256);
-	const int line = threadIdx.x / G, p = threadIdx.x % G;
+	const int line = GE::line(threadIdx.x), p = GE::lane(threadIdx.x);
 	const int kn = line % N;
 	const int npair = (a.ngrid + 1) / 2;
 	XP X{lds};
@@ -406,7 +406,7 @@ __global__ __launch_bounds__(T) void k_padfft_loop(PadFFTArgs a)
 					v[s] = czero<R>();
 				}
 			}
-			line_fwd<R, P, G, E>(v, p, tw);
+			line_fwd<R, GE>(v, p, tw);
 			X.put_Cb(X.gp(), v, line, p, 0);
 		}
 		__syncthreads();
@@ -415,7 +415,7 @@ __global__ __launch_bounds__(T) void k_padfft_loop(PadFFTArgs a)
 #pragma unroll
 			for (int s = 0; s < E; s++)
 				v[s] = padded_nonzero<E>(s) ? X.gp()[X.a(line, g * N + p + G * s - (s >= E / 4 ? N : 0))] : czero<R>();
-			line_fwd<R, P, G, E>(v, p, tw);
+			line_fwd<R, GE>(v, p, tw);
 			// non-temporal stores: the F grids of a launch (GiBs) are read back from HBM by the I3
 			// kernel, so they need not displace other lines from L2 (FP32 step 329 -> 327 ms)
 			cx<R>* dst = (cx<R>*)a.out + (size_t)(o0 + g) * (P * P);
@@ -431,8 +431,8 @@ __global__ __launch_bounds__(T) void k_padfft_loop(PadFFTArgs a)
 
 // ---------------------------------------------------------------------------------------------
 // Layout of a mirror sum D: the N x N box of the padded frequency grid (EDGE: and its +N/2 row and
-// column), in the C_i native order of the lines and elements that lie in it: line' (element s' of it)
-// at (s' * DL + line') * G + p.  N = 128 (k_i3fold_big): row' * DL + column'.
+// column), elements s' of lines line' that lie in it, in the C_i order of the lanes: (s' * G + p) * DL + line'.
+// N = 128 (k_i3fold_big): row' * DL + column'.
 template <int N, int G, int E, bool EDGE>
 struct MirrorBox {
 	static constexpr int DL = N + EDGE, DS = E / 2 + EDGE;
@@ -440,8 +440,10 @@ struct MirrorBox {
 	// padded line / row / column index 0 .. N/2 - 1 (EDGE: N/2), 3N/2 .. 2N - 1
 	static __device__ __forceinline__ constexpr int idx(int x) { return x < N / 2 + EDGE ? x : x - N + EDGE; }
 	static __device__ __forceinline__ constexpr int elem(int s) { return s < E / 4 + EDGE ? s : s - E / 2 + EDGE; }
+	// element s' = 0 of lane p of a line
+	static __device__ __forceinline__ int lane(int line, int p) { return p * DL + idx(line); }
 	// element (l, k) of the padded grid
-	static __device__ __forceinline__ int at(int l, int k) { return (elem(l / G) * DL + idx(k)) * G + l % G; }
+	static __device__ __forceinline__ int at(int l, int k) { return elem(l / G) * (DL * G) + lane(k, l % G); }
 };
 
 // One of two Hermitian spectra a, b from their packed sum z = a + i b at r and w = (a + i b)(-r)
@@ -462,7 +464,7 @@ __global__ __launch_bounds__(T) void k_combine(CombineArgs a)
 	load_twiddles<R, P, T>(tw, a.tw256);
 	const int o = blockIdx.x % a.nout;
 	const int cell = blockIdx.x / a.nout;
-	const int line = threadIdx.x / G, p = threadIdx.x % G;
+	const int line = GE::line(threadIdx.x), p = GE::lane(threadIdx.x);
 	const int t = threadIdx.x;
 	XP X{lds};
 	cx<R> v[E];
@@ -692,7 +694,7 @@ __global__ __launch_bounds__(T) void k_phys2fourier(const double* __restrict__ i
 	load_twiddles<double, N, T>(tw, tw256);
 	const int gi = blockIdx.x;
 	if (gi >= ngrid) return;
-	const int line = threadIdx.x / G, p = threadIdx.x % G;
+	const int line = GE::line(threadIdx.x), p = GE::lane(threadIdx.x);
 	const double* src = in + (size_t)gi * (N * N);
 	XP X{lds};
 	cx<double> v[E];
@@ -702,9 +704,9 @@ __global__ __launch_bounds__(T) void k_phys2fourier(const double* __restrict__ i
 	fft2_reg<double, GE>(v, X, tw, line, p);
 	const double sc = 1.0 / ((double)N * N);
 	double2* dst = out + (size_t)gi * (N * N);
-	const int k0 = E * brev<G>(p);
+	const int k0 = GE::blk_lane(p);
 #pragma unroll
-	for (int u = 0; u < E; u++) dst[line * N + k0 + u] = make_double2(v[u].x * sc, v[u].y * sc);
+	for (int u = 0; u < E; u++) dst[line * N + k0 + GE::blk_reg(u)] = make_double2(v[u].x * sc, v[u].y * sc);
 }
 
 template <int N, int T, bool SP>
@@ -719,13 +721,13 @@ __global__ __launch_bounds__(T) void k_fourier2phys(const double2* __restrict__ 
 	load_twiddles<double, N, T>(tw, tw256);
 	const int gi = blockIdx.x;
 	if (gi >= ngrid) return;
-	const int line = threadIdx.x / G, p = threadIdx.x % G;
+	const int line = GE::line(threadIdx.x), p = GE::lane(threadIdx.x);
 	const double2* src = in + (size_t)gi * (N * N);
 	XP X{lds};
 	cx<double> v[E];
-	const int k0 = E * brev<G>(p);
+	const int k0 = GE::blk_lane(p);
 #pragma unroll
-	for (int u = 0; u < E; u++) v[u] = src[line * N + k0 + u];
+	for (int u = 0; u < E; u++) v[u] = src[line * N + k0 + GE::blk_reg(u)];
 	__syncthreads();
 	ifft2_reg<double, GE>(v, X, tw, line, p);
 	double* dst = out + (size_t)gi * (N * N);
