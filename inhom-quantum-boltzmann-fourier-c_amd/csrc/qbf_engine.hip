@@ -821,13 +821,21 @@ struct EngineT final : public qbf_engine {
 	// resident workgroups times terms per workgroup (a workgroup's start and end cost about half a term);
 	// the fewest ranges where that is equal.  10 cells, N = 64, FP32, 256 terms: 32 ranges, 5 full rounds
 	// of 8 terms; 8 ranges would be two rounds of 32, the second one a quarter full.
-	static int fold_chunks(int wg, int nq)
+	//   N <= 32: the S grids of the cells that run on an XCD at the same time are read again for every
+	// term, and with more ranges they are fewer cells' (consecutive workgroups are the ranges of a cell).
+	// FP64 N = 32, 128 cells (4 MiB of S grids per XCD, as large as its L2): 1, 2, 4, 8, 16 ranges take 45.3,
+	// 43.4, 41.9, 41.6 and 43.0 ms per step.  At N = 64 more ranges than rounds need gain nothing (FP32, 512
+	// cells, 1, 2, 4: 195.9, 197.2, 199.1 ms).  0.12 per L2 of S grids follows these times, and those of 64,
+	// 100 and 300 cells, of FP32 N = 32 and of FP64 N = 16, 512 cells (19.1 -> 17.2 ms), within 2 %.
+	static int fold_chunks(int wg, int nq, int ncell, int ngrid)
 	{
 		int best = 1;
 		double cost = INFINITY;
 		for (int c = 1; c <= nq && (c == 1 || (long long)wg * (c - 1) < 8LL * FOLD_RES); c++) {
 			const long long rounds = ((long long)wg * c + FOLD_RES - 1) / FOLD_RES;
-			const double x = (double)rounds * ((nq + c - 1) / c + 0.5);
+			const long long resident = std::min((long long)wg * c, (long long)FOLD_RES);
+			const double S = N <= 32 ? (double)resident * ncell / ((double)wg * c) * ngrid * GB / (8 * (4 << 20)) : 0;
+			const double x = (double)rounds * ((nq + c - 1) / c + 0.5) * (1 + 0.12 * S);
 			if (x < cost * (1 - 1e-9)) {
 				cost = x;
 				best = c;
@@ -851,7 +859,7 @@ struct EngineT final : public qbf_engine {
 		int qr = (int)(fBudget / perQ);
 		if (qr < 1) qr = 1;
 		if (qr > nq) qr = nq;
-		const int nchunk = fold_chunks(wg, qr);
+		const int nchunk = fold_chunks(wg, qr, ncell, NO);
 		int r = Fscr.ensure((size_t)ncell * NO * GB * qr);
 		if (!r) r = acc3.ensure((size_t)ncell * NO * NI * nchunk * GB);
 		// blocks of mirror sums per workgroup (FP64: one over all launches)
