@@ -464,10 +464,10 @@ def main():
                           "counts executed applications"}
     achieved = kapps * flop_per_k / (kms / 1e3) if kms > 0 else 0.0
     headline = (N, Nx) == (64, 512)
-    i3_kernel = ("k_i3acc<float,64,1024,false,%s> (I3 K-operator: IFFT2 -> psi2 -> FFT2)" % ("true" if used else "false")
-                 if N == 64 else f"k_i3acc_big<float,{'true' if used else 'false'}> (I3 K-operator on {P} x {P} grids "
+    i3_kernel = ("k_i3fold%s<float,64,1024,false> (I3 K-operator: IFFT2 -> psi2 -> FFT2, over mirrored terms)" % ("_pair" if used else "")
+                 if N == 64 else f"k_i3fold_big<float,{'true' if used else 'false'}> (I3 K-operator on {P} x {P} grids "
                  "in global memory)" if N == 128
-                 else f"k_i3acc<float,{N},...> (I3 K-operator)")
+                 else f"k_i3fold<float,{N},...> (I3 K-operator)")
     line = {
         "metric": METRIC if headline else f"collision evals/s at N={N},Nx={Nx}: FP32 exact vs FP64 plain",
         "value": round(F["value"], 3),
