@@ -432,7 +432,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_i3fold_big(I3FoldArgs a)
 	using MB = MirrorBox<N, G, E, PAIR>;
 	constexpr int DN = MB::DL * MB::DL;
 	const long long dstep = (long long)NO * a.nchunk * a.nblk * DN;
-	cx<R>* Dp = (cx<R>*)a.D + NO * cell * dstep + (long long)((j * a.nchunk + chunk) * a.nblk + a.blk0 - 1) * DN;
+	cx<R>* Dp = (cx<R>*)a.D + NO * cell * dstep + (long long)((j * a.nchunk + chunk) * a.nblk + a.resumeD - 1) * DN;
 	const cx<R>* Sh = (const cx<R>*)a.Shat + (size_t)cell * NO * PP;
 	const cx<R>* Sj = Sh + (size_t)j * PP;
 	const int r0 = blk(p);
@@ -599,7 +599,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_i3fold_big(I3FoldArgs a)
 		}
 		__syncthreads();
 	}
-	while (nb < a.nper) next_block();
+	while (nb < a.nblk - a.resumeD) next_block();
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -844,11 +844,15 @@ struct EngineT final : public qbf_engine {
 		return best;
 	}
 
-	// I3 part of CdInt with one pass per mirrored pair of terms (see k_i3fold): acc3 [cell][no][*na] and
-	// Dmir [cell][no][*nd] partial sums, no = 4 outputs or (PAIR) 2 packed pairs.  F and S as run_i3 (src
-	// with nsrc grids per cell, the first no of them).
+	// I3 part of CdInt with one pass per mirrored pair of terms (see k_i3fold): acc3 [cell][no][*na] partial
+	// sums and the mirrored terms' sums Dsum [cell][no], no = 4 outputs or (PAIR) 2 packed pairs.  F and S as
+	// run_i3 (src with nsrc grids per cell, the first no of them).
+	//   Dmir holds the blocks of one launch, or one block that several launches fill together until it has DBLOCK
+	// terms; they are then added to Dsum and used again, so that Dmir does not grow with the number of launches,
+	// which is the number of terms times that of cells: FP32, N = 128, complex, 2048 cells, 256 folded terms, one
+	// of them a launch: 4 GiB, where a block per launch took 1 TiB.
 	template <bool PAIR>
-	int run_i3_fold(const double2* src, int nsrc, const void* Shat, int ncell, int* na, int* nd)
+	int run_i3_fold(const double2* src, int nsrc, const void* Shat, int ncell, int* na)
 	{
 		// four workgroups per cell and term range: outputs, or (output pair, instance pair), of which the
 		// pair kernel at N = 128 takes both instance pairs
@@ -862,13 +866,15 @@ struct EngineT final : public qbf_engine {
 		const int nchunk = fold_chunks(wg, qr, ncell, NO);
 		int r = Fscr.ensure((size_t)ncell * NO * GB * qr);
 		if (!r) r = acc3.ensure((size_t)ncell * NO * NI * nchunk * GB);
-		// blocks of mirror sums per workgroup (FP64: one over all launches)
-		const bool blocks = DBLOCK<R> < nq;
-		const int perLaunch = blocks ? ((qr + nchunk - 1) / nchunk + DBLOCK<R> - 1) / DBLOCK<R> : 0;
-		const int nblk = blocks ? perLaunch * ((nq + qr - 1) / qr) : 1;
+		// blocks of mirror sums of a workgroup, and launches that fill one together (FP64: all of them)
+		const int perWg = (qr + nchunk - 1) / nchunk;
+		const int nblk = (perWg + DBLOCK<R> - 1) / DBLOCK<R>;
+		const int group = nblk > 1 ? 1 : DBLOCK<R> / perWg;
 		if (!r) r = Dmir.ensure(sizeof(C) * (size_t)ncell * NO * NO * nchunk * nblk * mirror_size(PAIR));
+		if (!r) r = Dsum.ensure(sizeof(double2) * (size_t)ncell * NO * mirror_size(PAIR));
 		if (r) return r;
 		const int slots[4] = {0, 1, 2, 3};
+		int done = 0;                           // launches of the current group
 		for (int q0 = 0; q0 < nq; q0 += qr) {
 			const int nqr = (nq - q0) < qr ? (nq - q0) : qr;
 			r = launch_padfft(src, nsrc, i3p1.p, 2, q0, nqr, NO, slots, Fscr.p, ncell);
@@ -877,8 +883,7 @@ struct EngineT final : public qbf_engine {
 			a.Shat = Shat; a.F = Fscr.p; a.nq = nqr; a.q0 = q0; a.nmir = n3m;
 			a.psi2n = i3p2n.p; a.phase = i3ph.p;
 			a.nchunk = nchunk; a.accumulate = q0 > 0; a.acc = acc3.p; a.D = Dmir.p; a.nblk = nblk;
-			a.blk0 = blocks ? (q0 / qr) * perLaunch : (q0 > 0); a.resumeD = !blocks && q0 > 0;
-			a.nper = blocks ? perLaunch : (q0 == 0); a.tw256 = g_tw256;
+			a.resumeD = done > 0; a.tw256 = g_tw256;
 			r = xs_for(wg * nchunk, &a.xs, BIG ? big::I3_NI : 1);
 			if (r) return r;
 			hipEvent_t eb = nullptr, ee = nullptr;
@@ -894,9 +899,13 @@ struct EngineT final : public qbf_engine {
 				HIPCHK(hipEventRecord(ee, stream));
 				profK += (PAIR ? 8.0 : 16.0) * ncell * nqr;
 			}
+			if (++done == group || q0 + qr >= nq) {
+				r = sum_mirror(PAIR, ncell, NO * nchunk * nblk, q0 / qr >= group);
+				if (r) return r;
+				done = 0;
+			}
 		}
 		*na = NI * nchunk;
-		*nd = NO * nchunk * nblk;
 		return 0;
 	}
 
@@ -976,15 +985,16 @@ struct EngineT final : public qbf_engine {
 		return 0;
 	}
 
-	// Dsum = the mirror sums from their nd parts per grid
-	int sum_mirror(bool pair, int ncell, int nd)
+	// Dsum (accumulate: +)= the mirror sums from their nd parts per grid
+	int sum_mirror(bool pair, int ncell, int nd, bool accumulate)
 	{
 		const long long nel = mirror_size(pair), n = nel * ncell * (pair ? 2 : 4);
-		int r = Dsum.ensure(sizeof(double2) * n);
-		if (r) return r;
-		const int ne = 256 / SUM_CL;
-		hipLaunchKernelGGL((k_sum_mirror<R>), dim3((unsigned)((n + ne - 1) / ne)), dim3(256), 0, stream, (const C*)Dmir.p,
-			Dsum.template as<double2>(), nd, n, nel);
+		auto launch = [&](auto k, int ne) {
+			hipLaunchKernelGGL(k, dim3((unsigned)((n + ne - 1) / ne)), dim3(256), 0, stream, (const C*)Dmir.p,
+				Dsum.template as<double2>(), nd, n, nel, (int)accumulate);
+		};
+		if (nd > 4) launch(k_sum_mirror<R, 8>, 256 / 8);
+		else launch(k_sum_mirror<R, 1>, 256);
 		HIPCHK(hipGetLastError());
 		return 0;
 	}
@@ -1052,7 +1062,7 @@ struct EngineT final : public qbf_engine {
 				: launch_i1(QBF_TAB_I1, W, 4, What.p, 4, -4.0, 2.0, 3, g3, zero4, Ahat, ncell, &nchA);
 			if (r) return r;
 		}
-		int nchAcc = 1, nD = 1;
+		int nchAcc = 1;
 		// one pass per mirrored pair of I3 terms where the table has any (k_i3acc_mfma has no such form)
 		const bool fold = cd && n3m > 0 && !mfmaI3;
 		if (cd) {
@@ -1068,9 +1078,9 @@ struct EngineT final : public qbf_engine {
 				r = WhatP.ensure((size_t)ncell * 2 * GB);
 				const int two[2] = {0, 1};
 				if (!r) r = launch_padfft(Wpk.template as<double2>(), 3, nullptr, 0, 0, 1, 2, two, WhatP.p, ncell);
-				if (!r) r = run_i3_fold<true>(Wpk.template as<double2>(), 3, WhatP.p, ncell, &nchAcc, &nD);
+				if (!r) r = run_i3_fold<true>(Wpk.template as<double2>(), 3, WhatP.p, ncell, &nchAcc);
 			} else if (fold) {
-				r = run_i3_fold<false>(W, 4, What.p, ncell, &nchAcc, &nD);
+				r = run_i3_fold<false>(W, 4, What.p, ncell, &nchAcc);
 			} else if (pair) {
 				r = run_i3_pairs(ncell, &nchAcc);
 			} else {
@@ -1089,7 +1099,6 @@ struct EngineT final : public qbf_engine {
 		a.What = What.p; a.A = cc ? Ahat.p : nullptr; a.B = cd ? Bhat.p : nullptr; a.S = Sbuf.p; a.acc = acc3.p;
 		a.nchA = nchA; a.nchB = nchB; a.nchS = nchS; a.nchAcc = nchAcc; a.pairAB = pair; a.pairAcc = pairAcc;
 		r = assemble(a, ncell);
-		if (!r && fold) r = sum_mirror(pairAcc, ncell, nD);
 		if (r) return r;
 		std::vector<CTerm> tl[4];
 		double Dcoef[4];

@@ -187,7 +187,7 @@ __global__ __launch_bounds__(T, (FOLD_WPE<R, N>)) void k_i3fold(I3FoldArgs a)
 	const int t = threadIdx.x;
 	const int line = GE::line(t), p = GE::lane(t);
 	const size_t dstep = (size_t)4 * a.nchunk * a.nblk * MB::SIZE;
-	cx<R>* Dp = (cx<R>*)a.D + 4 * w.cell * dstep + (size_t)((j * a.nchunk + w.chunk) * a.nblk + a.blk0 - 1) * MB::SIZE;
+	cx<R>* Dp = (cx<R>*)a.D + 4 * w.cell * dstep + (long long)((j * a.nchunk + w.chunk) * a.nblk + a.resumeD - 1) * MB::SIZE;
 	int nb = 0;                                 // blocks begun
 	auto next_block = [&]() {
 		Dp += MB::SIZE;
@@ -235,7 +235,7 @@ __global__ __launch_bounds__(T, (FOLD_WPE<R, N>)) void k_i3fold(I3FoldArgs a)
 			}
 		}
 	}
-	while (nb < a.nper) next_block();
+	while (nb < a.nblk - a.resumeD) next_block();
 	acc.store();
 }
 
@@ -264,7 +264,7 @@ __global__ __launch_bounds__(T, (FOLD_WPE<R, N>)) void k_i3fold_pair(I3FoldArgs 
 	const int t = threadIdx.x;
 	const int line = GE::line(t), p = GE::lane(t);
 	cx<R>* Dp = (cx<R>*)a.D + ((((size_t)w.cell * 2 + pr) * 2 + J) * a.nchunk + w.chunk) * a.nblk * MB::SIZE +
-		(long long)(a.blk0 - 1) * MB::SIZE;
+		(long long)(a.resumeD - 1) * MB::SIZE;
 	int nb = 0;                                 // blocks begun
 	auto next_block = [&]() {
 		Dp += MB::SIZE;
@@ -330,7 +330,7 @@ __global__ __launch_bounds__(T, (FOLD_WPE<R, N>)) void k_i3fold_pair(I3FoldArgs 
 		}
 		__builtin_amdgcn_sched_barrier(0);
 	}
-	while (nb < a.nper) next_block();
+	while (nb < a.nblk - a.resumeD) next_block();
 	acc.store();
 }
 

@@ -542,15 +542,14 @@ __global__ __launch_bounds__(T) void k_combine(CombineArgs a)
 }
 
 // ---------------------------------------------------------------------------------------------
-// Mirror sums of the I3 terms from their parts in[o][c][e] (c < nch, e < nel): out[o][e] = sum_c in[o][c][e]
-// in FP64.  SUM_CL threads share an element: thread c adds the parts c, c + SUM_CL, ..., and the sums
-// are added in order.
-constexpr int SUM_CL = 8;
-template <typename R>
+// Mirror sums of the I3 terms from their parts in[o][c][e] (c < nch, e < nel): out[o][e] (accumulate: +)=
+// sum_c in[o][c][e] in FP64.  CL threads share an element: thread c adds the parts c, c + CL, ..., and the
+// sums are added in order (CL = 8 where there are many parts, that is few cells).
+template <typename R, int CL>
 __global__ __launch_bounds__(256) void k_sum_mirror(const cx<R>* __restrict__ in, double2* __restrict__ out, int nch,
-	long long n, long long nel)
+	long long n, long long nel, int accumulate)
 {
-	constexpr int CL = SUM_CL, NE = 256 / CL;
+	constexpr int NE = 256 / CL;
 	__shared__ double2 sh[CL][NE];
 	const int c = threadIdx.x / NE, x = threadIdx.x % NE;
 	const long long i = (long long)blockIdx.x * NE + x;
@@ -565,6 +564,7 @@ __global__ __launch_bounds__(256) void k_sum_mirror(const cx<R>* __restrict__ in
 	__syncthreads();
 	if (c || i >= n) return;
 	for (int k = 1; k < CL; k++) s = make_double2(s.x + sh[k][x].x, s.y + sh[k][x].y);
+	if (accumulate) s = make_double2(out[i].x + s.x, out[i].y + s.y);
 	out[i] = s;
 }
 

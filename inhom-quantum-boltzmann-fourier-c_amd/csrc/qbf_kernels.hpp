@@ -95,8 +95,8 @@ struct I3FoldArgs {
 	int accumulate;
 	void* acc;            // [ncell][no][na][P*P] R_b native
 	void* D;              // [ncell][no][nd] mirror sums (MirrorBox), nblk blocks of terms per workgroup
-	int nblk, blk0, nper; // blocks in all launches, of the launches before this one, and of this one
-	int resumeD;          // the first terms continue block blk0 - 1
+	int nblk;
+	int resumeD;          // the terms of this launch continue block 0 (nblk = 1) of the launch before
 	const double2* tw256;
 };
 
