@@ -126,7 +126,8 @@ int qbf_last_collision(qbf_engine *e, int ncell, double *dWin, double *dC);
  * choice (qbf_set_real_pairs mode 0 or 2) and no buffer growth during the capture.  Launches replay
  * on the capture stream, asynchronously, ordered after the work queued on the engine's current
  * stream and before the work queued there afterwards.  The graph uses the engine's buffers: while
- * it is alive, calls that would grow a buffer or drop a cached table fail (-1); after
+ * it is alive, calls that would grow a buffer or drop a cached table fail (-1); an I3 table that replaces
+ * one of as many terms is what later replays use, and one that is refused changes nothing; after
  * qbf_engine_destroy the graph is dead (qbf_graph_launch fails, qbf_graph_destroy frees it). */
 typedef struct qbf_graph qbf_graph;
 int  qbf_graph_capture_inhom_step_periodic(qbf_engine *e, const double *dW, int ncell, double L, double h,

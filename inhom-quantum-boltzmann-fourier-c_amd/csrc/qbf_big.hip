@@ -88,6 +88,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_padfft_big(PadFFTArgs a)
 	using namespace big;
 	constexpr int T = TB<R>, L = T / G;         // L: lines per sweep
 	__shared__ cx<R> tw[TW];
+	if (a.live && a.q0 >= *a.live) return;
 	load_twiddles_g<R, P, G, T>(tw, a.tw256);
 	const int o = blockIdx.x;
 	const int lt = threadIdx.x / G, p = dpp_p(threadIdx.x % G);
@@ -419,13 +420,10 @@ __global__ __launch_bounds__(big::TB<R>) void k_i3fold_big(I3FoldArgs a)
 	// step of 32 cells against 54.1)
 	auto form = [](cx<R> x) { return sizeof(R) == 8 ? pin<R>(x) : x; };
 	__shared__ cx<R> tw[TW];
+	const FoldRange w(a, NO);
+	if (w.none) return;
 	load_twiddles_g<R, P, G, T>(tw, a.tw256);
-	const int lb = xcd_block();
-	const int chunk = lb % a.nchunk;
-	const int j = (lb / a.nchunk) % NO;
-	const int cell = lb / (a.nchunk * NO);
-	const int qa = (int)(((long long)chunk * a.nq) / a.nchunk);
-	const int qb = (int)(((long long)(chunk + 1) * a.nq) / a.nchunk);
+	const int chunk = w.chunk, j = w.grp, cell = w.cell, qa = w.qa, qb = w.qb;
 	const int lt = threadIdx.x / G, p = dpp_p(threadIdx.x % G);
 	cx<R>* xs = (cx<R>*)a.xs + (size_t)blockIdx.x * (I3_NI * PP);
 	cx<R>* accp = (cx<R>*)a.acc + (((size_t)cell * NO + j) * a.nchunk + chunk) * PP;
@@ -460,7 +458,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_i3fold_big(I3FoldArgs a)
 	for (int qq = qa; qq < qb; qq++) {
 		const cx<R>* Fq = (const cx<R>*)a.F + ((size_t)cell * a.nq + qq) * NO * PP;
 		const R* ps = (const R*)a.psi2n + (size_t)(a.q0 + qq) * PP;
-		const bool mir = a.q0 + qq < a.nmir;
+		const bool mir = a.q0 + qq < w.nmir;
 		if ((qq - qa) % DBLOCK<R> == 0 && (qq > qa || !a.resumeD)) {
 			// (barriers follow before D is read)
 			next_block();

@@ -321,8 +321,10 @@ struct EngineT final : public qbf_engine {
 	I1Tab i1[2];
 	int n2 = 0; DevBuf i2p1, i2p2, i2pc;
 	// I3 terms in the order: one of each mirrored pair (n3m of them), terms without a mirror (up to
-	// n3f), the other ones of the pairs (see mirror_order and k_i3fold)
-	int n3 = 0, n3m = 0, n3f = 0; DevBuf i3p1, i3p2n, i3ph;
+	// n3f), the other ones of the pairs (see mirror_order and k_i3fold).  i3n: n3m and n3f on the device, where
+	// the kernels of a captured graph read them: a table that replaces another one of as many terms while the
+	// graph is alive may pair otherwise
+	int n3 = 0, n3m = 0, n3f = 0; DevBuf i3p1, i3p2n, i3ph, i3n;
 	// BF16 hi/lo split path (precision QBF_BF16X3, N = 64): the I3 K-operator runs k_i3acc_mfma,
 	// whose psi2 table has its own order (i3p2m)
 	bool mfmaI3 = false;
@@ -347,7 +349,7 @@ struct EngineT final : public qbf_engine {
 
 	int init()
 	{
-		for (DevBuf* b : {&i1[0].phi, &i1[0].psi1n, &i1[1].phi, &i1[1].psi1n, &i2p1, &i2p2, &i2pc, &i3p1, &i3p2n, &i3ph,
+		for (DevBuf* b : {&i1[0].phi, &i1[0].psi1n, &i1[1].phi, &i1[1].psi1n, &i2p1, &i2p2, &i2pc, &i3p1, &i3p2n, &i3ph, &i3n, &i3p2m,
 			     &What, &Ahat, &Bhat, &Sbuf, &acc3, &Dmir, &Dsum, &Vsum, &Fscr, &xscr, &Wmid, &WF, &WF2, &Wt1, &Wt2, &src3, &Wpk,
 			     &WhatP, &reim, &Cf})
 			b->lock = &liveGraphs;
@@ -540,7 +542,14 @@ struct EngineT final : public qbf_engine {
 			memcpy(&s1[(size_t)q * 2 * NN], p1 + (size_t)order[q] * 2 * NN, sizeof(double) * 2 * NN);
 			to_Ci_native(p2 + (size_t)order[q] * PP, &p2n[(size_t)q * PP]);
 		});
-		int r = upload(i3p1, s1.get(), sizeof(double2) * NN * (size_t)num);
+		// every buffer before the first copy: a table that is refused leaves the one before it whole.  The
+		// phases have room for as many pairs as num terms can make
+		int r = i3p1.ensure(sizeof(double2) * NN * (size_t)num);
+		if (!r) r = i3p2n.ensure(sizeof(R) * p2n.size());
+		if (!r) r = i3ph.ensure(sizeof(C) * (size_t)(num / 2 + 1) * 2 * (N + 1));
+		if (!r) r = i3n.ensure(2 * sizeof(int));
+		if (!r && mfmaI3) r = i3p2m.ensure(sizeof(float) * (size_t)num * PP);
+		if (!r) r = upload(i3p1, s1.get(), sizeof(double2) * NN * (size_t)num);
 		if (!r) r = upload(i3p2n, p2n.data(), sizeof(R) * p2n.size());
 		// conj(psi1) of the representatives along l and along k, frequencies 0 .. N/2, -N/2 .. -1 (+N/2: the
 		// conjugate of -N/2)
@@ -554,6 +563,8 @@ struct EngineT final : public qbf_engine {
 					ph.push_back(mk<R>((R)z[0], (R)(x == N / 2 ? z[1] : -z[1])));
 				}
 		if (!r && nmir) r = upload(i3ph, ph.data(), sizeof(C) * ph.size());
+		const int terms[2] = {nmir, nfold};
+		if (!r) r = upload(i3n, terms, sizeof(terms));
 		if (r) return r;
 		if (mfmaI3) {
 			// k_i3acc_mfma's order: psi2 of column 16 w + i16, row 4 kq + r + 16 t at
@@ -591,9 +602,10 @@ struct EngineT final : public qbf_engine {
 	}
 
 	int launch_padfft(const double2* src, int nsrc, const void* pre, int preKind, int q0, int nq, int nslot,
-		const int* srcOfSlot, void* out, int ncell)
+		const int* srcOfSlot, void* out, int ncell, const int* live = nullptr)
 	{
 		PadFFTArgs a{};
+		a.live = live;
 		a.src = src; a.nsrc = nsrc; a.pre = pre; a.preKind = preKind; a.q0 = q0; a.nq = nq; a.nslot = nslot;
 		for (int i = 0; i < nslot; i++) a.srcOfSlot[i] = srcOfSlot[i];
 		a.out = out; a.tw256 = g_tw256;
@@ -875,12 +887,16 @@ struct EngineT final : public qbf_engine {
 		if (r) return r;
 		const int slots[4] = {0, 1, 2, 3};
 		int done = 0;                           // launches of the current group
-		for (int q0 = 0; q0 < nq; q0 += qr) {
-			const int nqr = (nq - q0) < qr ? (nq - q0) : qr;
-			r = launch_padfft(src, nsrc, i3p1.p, 2, q0, nqr, NO, slots, Fscr.p, ncell);
+		// a captured graph has launches for all n3 terms: those beyond the table's n3f return at once, and a table
+		// with fewer pairs that replaces this one needs them
+		const int nqAll = tl_capturing ? n3 : nq;
+		const int* live = i3n.template as<int>() + 1;
+		for (int q0 = 0; q0 < nqAll; q0 += qr) {
+			const int nqr = (nqAll - q0) < qr ? (nqAll - q0) : qr;
+			r = launch_padfft(src, nsrc, i3p1.p, 2, q0, nqr, NO, slots, Fscr.p, ncell, live);
 			if (r) return r;
 			I3FoldArgs a{};
-			a.Shat = Shat; a.F = Fscr.p; a.nq = nqr; a.q0 = q0; a.nmir = n3m;
+			a.Shat = Shat; a.F = Fscr.p; a.nq = nqr; a.q0 = q0; a.terms = i3n.template as<int>();
 			a.psi2n = i3p2n.p; a.phase = i3ph.p;
 			a.nchunk = nchunk; a.accumulate = q0 > 0; a.acc = acc3.p; a.D = Dmir.p; a.nblk = nblk;
 			a.resumeD = done > 0; a.tw256 = g_tw256;
@@ -899,8 +915,8 @@ struct EngineT final : public qbf_engine {
 				HIPCHK(hipEventRecord(ee, stream));
 				profK += (PAIR ? 8.0 : 16.0) * ncell * nqr;
 			}
-			if (++done == group || q0 + qr >= nq) {
-				r = sum_mirror(PAIR, ncell, NO * nchunk * nblk, q0 / qr >= group);
+			if (++done == group || q0 + qr >= nqAll) {
+				r = sum_mirror(PAIR, ncell, NO * nchunk * nblk, q0 - (done - 1) * qr, live);
 				if (r) return r;
 				done = 0;
 			}
@@ -985,13 +1001,13 @@ struct EngineT final : public qbf_engine {
 		return 0;
 	}
 
-	// Dsum (accumulate: +)= the mirror sums from their nd parts per grid
-	int sum_mirror(bool pair, int ncell, int nd, bool accumulate)
+	// Dsum (q0 > 0: +)= the mirror sums from their nd parts per grid, q0 the first of their terms
+	int sum_mirror(bool pair, int ncell, int nd, int q0, const int* live)
 	{
 		const long long nel = mirror_size(pair), n = nel * ncell * (pair ? 2 : 4);
 		auto launch = [&](auto k, int ne) {
 			hipLaunchKernelGGL(k, dim3((unsigned)((n + ne - 1) / ne)), dim3(256), 0, stream, (const C*)Dmir.p,
-				Dsum.template as<double2>(), nd, n, nel, (int)accumulate);
+				Dsum.template as<double2>(), nd, n, nel, q0, live);
 		};
 		if (nd > 4) launch(k_sum_mirror<R, 8>, 256 / 8);
 		else launch(k_sum_mirror<R, 1>, 256);

@@ -105,17 +105,23 @@ __device__ __forceinline__ void k_apply(cx<R>* v, const R* ps, const XP& X, cons
 // 2.3e-10, as with the sums in FP64, which took 220 ms instead of 206 for the step of 512 cells).
 template <typename R> constexpr int DBLOCK = sizeof(R) == 4 ? 32 : 1 << 30;
 
-// Workgroup -> (cell, group, term range) of the fold kernels
+// Workgroup -> (cell, group, term range) of the fold kernels; nmir: see I3FoldArgs::terms.  none: the launch
+// is beyond the table's terms
 struct FoldRange {
-	int chunk, grp, cell, qa, qb;
+	int chunk, grp, cell, qa, qb, nmir;
+	bool none;
 	__device__ __forceinline__ FoldRange(const I3FoldArgs& a, int ngrp)
 	{
+		nmir = __builtin_amdgcn_readfirstlane(a.terms[0]);
+		const int left = __builtin_amdgcn_readfirstlane(a.terms[1]) - a.q0;
+		const int nq = left < a.nq ? left : a.nq;
+		none = nq <= 0;
 		const int lb = xcd_block();
 		chunk = lb % a.nchunk;
 		grp = (lb / a.nchunk) % ngrp;
 		cell = lb / (a.nchunk * ngrp);
-		qa = (int)(((long long)chunk * a.nq) / a.nchunk);
-		qb = (int)(((long long)(chunk + 1) * a.nq) / a.nchunk);
+		qa = (int)(((long long)chunk * nq) / a.nchunk);
+		qb = (int)(((long long)(chunk + 1) * nq) / a.nchunk);
 	}
 };
 
@@ -181,8 +187,9 @@ __global__ __launch_bounds__(T, (FOLD_WPE<R, N>)) void k_i3fold(I3FoldArgs a)
 	__shared__ typename XP::El lds[XP::SIZE];
 	__shared__ cx<R> tw[TwTab<P, T>::SIZE];
 	__shared__ cx<R> ph[2 * (N + 1)];           // the mirror's phases of the current term
-	load_twiddles<R, P, T>(tw, a.tw256);
 	const FoldRange w(a, 4);
+	if (w.none) return;
+	load_twiddles<R, P, T>(tw, a.tw256);
 	const int j = w.grp;
 	const int t = threadIdx.x;
 	const int line = GE::line(t), p = GE::lane(t);
@@ -204,7 +211,7 @@ __global__ __launch_bounds__(T, (FOLD_WPE<R, N>)) void k_i3fold(I3FoldArgs a)
 	for (int qq = w.qa; qq < w.qb; qq++) {
 		const cx<R>* Fq = (const cx<R>*)a.F + ((size_t)w.cell * a.nq + qq) * 4 * (P * P);
 		const R* ps = (const R*)a.psi2n + (size_t)(a.q0 + qq) * (P * P);
-		const bool mir = a.q0 + qq < a.nmir;
+		const bool mir = a.q0 + qq < w.nmir;
 		if ((qq - w.qa) % DBLOCK<R> == 0 && (qq > w.qa || !a.resumeD)) {
 			// (the term's barriers are before the mirror's reads)
 			next_block();
@@ -258,8 +265,9 @@ __global__ __launch_bounds__(T, (FOLD_WPE<R, N>)) void k_i3fold_pair(I3FoldArgs 
 	__shared__ typename XP::El lds[XP::SIZE];
 	__shared__ cx<R> tw[TwTab<P, T>::SIZE];
 	__shared__ cx<R> ph[2 * (N + 1)];           // the mirror's phases of the current term
-	load_twiddles<R, P, T>(tw, a.tw256);
 	const FoldRange w(a, 4);
+	if (w.none) return;
+	load_twiddles<R, P, T>(tw, a.tw256);
 	const int J = w.grp >> 1, pr = w.grp & 1;
 	const int t = threadIdx.x;
 	const int line = GE::line(t), p = GE::lane(t);
@@ -286,7 +294,7 @@ __global__ __launch_bounds__(T, (FOLD_WPE<R, N>)) void k_i3fold_pair(I3FoldArgs 
 		const cx<R>* SJ = Sh + (size_t)J * (P * P);
 		const cx<R>* Fp = Fq + (size_t)pr * (P * P);
 		const cx<R>* FJ = Fq + (size_t)J * (P * P);
-		const bool mir = a.q0 + qq < a.nmir;
+		const bool mir = a.q0 + qq < w.nmir;
 		if ((qq - w.qa) % DBLOCK<R> == 0 && (qq > w.qa || !a.resumeD)) {
 			// (the term's barriers are before the mirror's reads)
 			next_block();

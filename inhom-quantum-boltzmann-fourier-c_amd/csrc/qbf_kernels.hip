@@ -107,6 +107,7 @@ __global__ __launch_bounds__(T) void k_padfft(PadFFTArgs a)
 	using XP = Xpose<R, GE, SP>;
 	__shared__ typename XP::El lds[XP::SIZE];
 	__shared__ cx<R> tw[TwTab<P, T>::SIZE];
+	if (a.live && a.q0 >= *a.live) return;
 	load_twiddles<R, P, T>(tw, a.tw256);
 	const int o0 = 2 * blockIdx.x;
 	const int line = GE::line(threadIdx.x), p = GE::lane(threadIdx.x);
@@ -357,6 +358,7 @@ __global__ __launch_bounds__(T) void k_padfft_loop(PadFFTArgs a)
 	using XP = Xpose<R, GE>;
 	__shared__ typename XP::El lds[XP::SIZE];
 	__shared__ cx<R> tw[TwTab<P, T>::SIZE];
+	if (a.live && a.q0 >= *a.live) return;
 	load_twiddles<R, P, T>(tw, a.tw256);
 	const int line = GE::line(threadIdx.x), p = GE::lane(threadIdx.x);
 	const int kn = line % N;
@@ -542,13 +544,15 @@ __global__ __launch_bounds__(T) void k_combine(CombineArgs a)
 }
 
 // ---------------------------------------------------------------------------------------------
-// Mirror sums of the I3 terms from their parts in[o][c][e] (c < nch, e < nel): out[o][e] (accumulate: +)=
+// Mirror sums of the I3 terms from their parts in[o][c][e] (c < nch, e < nel): out[o][e] (q0 > 0: +)=
 // sum_c in[o][c][e] in FP64.  CL threads share an element: thread c adds the parts c, c + CL, ..., and the
-// sums are added in order (CL = 8 where there are many parts, that is few cells).
+// sums are added in order (CL = 8 where there are many parts, that is few cells).  q0: first term of the
+// parts, beyond *live there are none.
 template <typename R, int CL>
 __global__ __launch_bounds__(256) void k_sum_mirror(const cx<R>* __restrict__ in, double2* __restrict__ out, int nch,
-	long long n, long long nel, int accumulate)
+	long long n, long long nel, int q0, const int* live)
 {
+	if (q0 >= *live) return;
 	constexpr int NE = 256 / CL;
 	__shared__ double2 sh[CL][NE];
 	const int c = threadIdx.x / NE, x = threadIdx.x % NE;
@@ -564,7 +568,7 @@ __global__ __launch_bounds__(256) void k_sum_mirror(const cx<R>* __restrict__ in
 	__syncthreads();
 	if (c || i >= n) return;
 	for (int k = 1; k < CL; k++) s = make_double2(s.x + sh[k][x].x, s.y + sh[k][x].y);
-	if (accumulate) s = make_double2(out[i].x + s.x, out[i].y + s.y);
+	if (q0 > 0) s = make_double2(out[i].x + s.x, out[i].y + s.y);
 	out[i] = s;
 }
 

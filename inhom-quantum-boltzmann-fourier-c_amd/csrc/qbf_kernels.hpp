@@ -20,6 +20,7 @@ struct PadFFTArgs {
 	int srcOfSlot[4];
 	int ngrid;            // ncell * nq * nslot grids, two per workgroup
 	void* out;
+	const int* live;      // launches with q0 at or beyond *live do nothing (null: none)
 	const double2* tw256;
 };
 
@@ -88,7 +89,8 @@ struct I3FoldArgs {
 	const void* Shat;     // [ncell][no][P*P] R_b native
 	const void* F;        // [ncell][nq][no][P*P] R_b native
 	int nq, q0;
-	int nmir;             // terms with an index below it stand for a mirrored pair
+	const int* terms;     // [0]: terms with an index below it stand for a mirrored pair, [1]: terms to take in all
+	                      // (read on the device: a captured launch follows a table that is replaced)
 	const void* psi2n;    // [nqTotal][P*P] C_i native
 	const void* phase;    // [nmir][2][N+1] conj(E) along l and along k, frequencies 0 .. N/2, -N/2 .. -1
 	int nchunk;
