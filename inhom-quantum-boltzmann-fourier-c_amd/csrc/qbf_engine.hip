@@ -249,6 +249,15 @@ struct DevBuf {
 	void* p = nullptr;
 	size_t bytes = 0;
 	const int* lock = nullptr;     // the owner's live-graph count: no reallocation while it is non-zero
+	// the buffer keeps its size: a split that another one can replace is then chosen to fit it
+	bool fixed() const { return tl_capturing || tl_noalloc || (lock && *lock); }
+	// the largest k >= 1 with k * unit in the buffer, at most most; most where the buffer can grow
+	int fit(size_t unit, int most) const
+	{
+		if (!fixed() || unit == 0 || bytes / unit >= (size_t)most) return most;
+		return bytes < unit ? 1 : (int)(bytes / unit);
+	}
+	bool holds(size_t n) const { return !fixed() || n <= bytes; }
 	int ensure(size_t n)
 	{
 		if (n <= bytes) return 0;
@@ -601,6 +610,15 @@ struct EngineT final : public qbf_engine {
 		return 0;
 	}
 
+	// Term ranges of an I3 launch of wg workgroups a range: nchunk, or what the accumulators (and at N = 128 the
+	// scratch grids) hold where they cannot grow.  The ranges of few cells can take more than those of many, so that
+	// an evaluation of fewer cells than a captured graph's is not a smaller one in every buffer
+	int fit_ranges(int wg, int nchunk) const
+	{
+		nchunk = acc3.fit((size_t)wg * GB, nchunk);
+		return BIG ? xscr.fit((size_t)wg * big::I3_NI * GB, nchunk) : nchunk;
+	}
+
 	int launch_padfft(const double2* src, int nsrc, const void* pre, int preKind, int q0, int nq, int nslot,
 		const int* srcOfSlot, void* out, int ncell, const int* live = nullptr)
 	{
@@ -711,7 +729,9 @@ struct EngineT final : public qbf_engine {
 		int qr = (int)(fBudget / perQ);
 		if (qr < 1) qr = 1;
 		if (qr > nq) qr = nq;
+		qr = Fscr.fit((size_t)ncell * nF * GB, qr);
 		if (nchunk > qr) nchunk = qr;
+		nchunk = fit_ranges(ncell * nout, nchunk);
 		int r = Fscr.ensure((size_t)ncell * nF * GB * qr);
 		if (!r) r = acc3.ensure((size_t)ncell * nout * nchunk * GB);
 		if (r) return r;
@@ -875,14 +895,20 @@ struct EngineT final : public qbf_engine {
 		int qr = (int)(fBudget / perQ);
 		if (qr < 1) qr = 1;
 		if (qr > nq) qr = nq;
-		const int nchunk = fold_chunks(wg, qr, ncell, NO);
+		qr = Fscr.fit((size_t)ncell * NO * GB, qr);
+		// ranges, blocks of mirror sums of a workgroup, and launches that fill one together (FP64: all of them);
+		// fewer ranges, then fewer terms a launch, where the buffers cannot grow
+		const size_t blkB = sizeof(C) * (size_t)ncell * NO * NO * mirror_size(PAIR);
+		int nchunk = fit_ranges(wg, fold_chunks(wg, qr, ncell, NO));
+		auto blocks = [&]() { return ((qr + nchunk - 1) / nchunk + DBLOCK<R> - 1) / DBLOCK<R>; };
+		while (nchunk > 1 && !Dmir.holds(blkB * nchunk * blocks())) nchunk--;
+		while (qr > DBLOCK<R> && !Dmir.holds(blkB * nchunk * blocks())) qr = (blocks() - 1) * DBLOCK<R>;
+		const int nblk = blocks();
+		const int group = nblk > 1 ? 1 : DBLOCK<R> / ((qr + nchunk - 1) / nchunk);
 		int r = Fscr.ensure((size_t)ncell * NO * GB * qr);
-		if (!r) r = acc3.ensure((size_t)ncell * NO * NI * nchunk * GB);
-		// blocks of mirror sums of a workgroup, and launches that fill one together (FP64: all of them)
-		const int perWg = (qr + nchunk - 1) / nchunk;
-		const int nblk = (perWg + DBLOCK<R> - 1) / DBLOCK<R>;
-		const int group = nblk > 1 ? 1 : DBLOCK<R> / perWg;
-		if (!r) r = Dmir.ensure(sizeof(C) * (size_t)ncell * NO * NO * nchunk * nblk * mirror_size(PAIR));
+		// (four grids a cell, as run_i3 takes, also where the pair kernel at N = 128 has two)
+		if (!r) r = acc3.ensure((size_t)ncell * GB * std::max(NO * NI * nchunk, 4));
+		if (!r) r = Dmir.ensure(blkB * nchunk * nblk);
 		if (!r) r = Dsum.ensure(sizeof(double2) * (size_t)ncell * NO * mirror_size(PAIR));
 		if (r) return r;
 		const int slots[4] = {0, 1, 2, 3};
@@ -923,6 +949,20 @@ struct EngineT final : public qbf_engine {
 		}
 		*na = NI * nchunk;
 		return 0;
+	}
+
+	// Whether the terms of an evaluation are taken in mirrored pairs: where the table has any.  Where the buffers
+	// cannot grow (a table or a kind of grids that came after them) the other way serves as well: term by term any
+	// table, and the fold kernels one without a pair.
+	bool use_fold(int ncell, bool pair) const
+	{
+		if (mfmaI3 || n3 <= 0) return false;        // (k_i3acc_mfma has no such form)
+		const size_t no = pair ? 2 : 4;
+		const bool fold = Dmir.holds(sizeof(C) * ncell * no * no * mirror_size(pair)) &&
+			Dsum.holds(sizeof(double2) * ncell * no * mirror_size(pair)) && acc3.holds(ncell * (pair && BIG ? 2 : 4) * GB) &&
+			(!BIG || xscr.holds(ncell * no * big::I3_NI * GB));
+		const bool plain = acc3.holds(ncell * 4 * GB) && (!BIG || xscr.holds(ncell * 4 * big::I3_NI * GB));
+		return n3m > 0 ? fold || !plain : fold && !plain;
 	}
 
 	// Dm: the mirrored terms' sums (sum_mirror; null: none), added with the factors Dcoef
@@ -1068,6 +1108,12 @@ struct EngineT final : public qbf_engine {
 		if (pair) {
 			pairUsed = 1;
 			r = pack_sources(W, ncell);
+			// room for the complex grids' results too: a call whose measured ratio does not allow the pairs
+			// must not need to grow them under a captured graph
+			if (!r && cc && i1[QBF_TAB_I1].n > 0 && !Ahat.fixed())
+				r = Ahat.ensure((size_t)ncell * 3 * term_chunks(ncell, 3, i1[QBF_TAB_I1].n, 4) * GB);
+			if (!r && cd && i1[QBF_TAB_I4].n > 0 && !Bhat.fixed())
+				r = Bhat.ensure((size_t)ncell * 4 * term_chunks(ncell, 4, i1[QBF_TAB_I4].n, 4) * GB);
 			if (r) return r;
 		}
 		if (cc) {
@@ -1079,8 +1125,8 @@ struct EngineT final : public qbf_engine {
 			if (r) return r;
 		}
 		int nchAcc = 1;
-		// one pass per mirrored pair of I3 terms where the table has any (k_i3acc_mfma has no such form)
-		const bool fold = cd && n3m > 0 && !mfmaI3;
+		// one pass per mirrored pair of I3 terms
+		const bool fold = cd && use_fold(ncell, pair);
 		if (cd) {
 			// I4 with Fhat = FFT2(pad(2 W0 - delta)) = 2 What_0 - 1 (src/collision.c:127-134); packed sources
 			// W0 + i W1 and W2 + i W3, or the components

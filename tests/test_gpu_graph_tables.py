@@ -66,6 +66,8 @@ def test_replay_takes_the_new_table(N, prec, pairs, n, J, M, first, then):
             g.launch()
             torch.cuda.synchronize()
             assert (out - ref).norm() < tol * apart
+        # eager, in the buffers that the graph pins
+        assert (e.inhom_step_periodic(W, L, h, dt) - ref).norm() < tol * apart
     # more terms than the buffers hold: refused, and nothing is written
     with pytest.raises(qbf.QBFError, match="captured graph"):
         e.set_quadrature(*qbf.quadrature(N, J, L, R, M + 2))
