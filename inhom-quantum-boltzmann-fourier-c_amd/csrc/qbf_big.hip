@@ -570,7 +570,7 @@ __global__ __launch_bounds__(big::TB<R>) void k_i3fold_big(I3FoldArgs a)
 		__syncthreads();
 		if (!mir) continue;
 		// columns of the box: IFFT along l, times conj(E(r)), into D
-		const cx<R>* ph = (const cx<R>*)a.phase + (size_t)(a.q0 + qq) * (2 * (N + 1));
+		const double2* ph = (const double2*)a.phase + (size_t)(a.q0 + qq) * (2 * (N + 1));
 #pragma unroll 1
 		for (int sw = 0; sw < NSW; sw++) {
 			const int c = mcol(sw);
@@ -583,15 +583,14 @@ __global__ __launch_bounds__(big::TB<R>) void k_i3fold_big(I3FoldArgs a)
 				for (int u = 0; u < E; u++) v[u] = x[u * P];
 				line16_bwd<R, P, E>(v, p, tw);
 				cx<R>* d = uni(Dp, g * dstep) + MB::idx(c);
-				const cx<R> pk = ph[N + 1 + phase_idx<N>(c)];
+				const double2 pk = ph[N + 1 + phase_idx<N>(c)];
 #pragma unroll
 				for (int s = 0; s < E; s++) {
 					if (!padded_nonzero<E>(s) && !(PAIR && s == E / 4)) continue;
 					const int l = p + G * s;
 					if (!padded_nonzero<E>(s) && l != N / 2) continue;
-					const cx<R> e = cmul<R>(ph[phase_idx<N>(l)], pk);
 					const int i = MB::idx(l) * MB::DL;
-					d[i] = cadd<R>(d[i], cmul<R>(v[s], e));
+					d[i] = add_phased<R>(d[i], v[s], cmul<double>(ph[phase_idx<N>(l)], pk));
 				}
 			}
 		}

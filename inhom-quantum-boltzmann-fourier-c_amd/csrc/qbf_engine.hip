@@ -555,23 +555,23 @@ struct EngineT final : public qbf_engine {
 		// phases have room for as many pairs as num terms can make
 		int r = i3p1.ensure(sizeof(double2) * NN * (size_t)num);
 		if (!r) r = i3p2n.ensure(sizeof(R) * p2n.size());
-		if (!r) r = i3ph.ensure(sizeof(C) * (size_t)(num / 2 + 1) * 2 * (N + 1));
+		if (!r) r = i3ph.ensure(sizeof(double2) * (size_t)(num / 2 + 1) * 2 * (N + 1));
 		if (!r) r = i3n.ensure(2 * sizeof(int));
 		if (!r && mfmaI3) r = i3p2m.ensure(sizeof(float) * (size_t)num * PP);
 		if (!r) r = upload(i3p1, s1.get(), sizeof(double2) * NN * (size_t)num);
 		if (!r) r = upload(i3p2n, p2n.data(), sizeof(R) * p2n.size());
 		// conj(psi1) of the representatives along l and along k, frequencies 0 .. N/2, -N/2 .. -1 (+N/2: the
 		// conjugate of -N/2)
-		std::vector<C> ph;
+		std::vector<double2> ph;
 		ph.reserve((size_t)nmir * 2 * (N + 1));
 		for (int q = 0; q < nmir; q++)
 			for (int axis = 0; axis < 2; axis++)
 				for (int x = 0; x <= N; x++) {
 					const int f = x <= N / 2 ? x : x - 1;       // index on the N grid
 					const double* z = p1 + 2 * ((size_t)order[q] * NN + (size_t)f * (axis == 0 ? N : 1));
-					ph.push_back(mk<R>((R)z[0], (R)(x == N / 2 ? z[1] : -z[1])));
+					ph.push_back(make_double2(z[0], x == N / 2 ? z[1] : -z[1]));
 				}
-		if (!r && nmir) r = upload(i3ph, ph.data(), sizeof(C) * ph.size());
+		if (!r && nmir) r = upload(i3ph, ph.data(), sizeof(double2) * ph.size());
 		const int terms[2] = {nmir, nfold};
 		if (!r) r = upload(i3n, terms, sizeof(terms));
 		if (r) return r;

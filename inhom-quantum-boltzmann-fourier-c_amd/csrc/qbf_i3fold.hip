@@ -29,9 +29,18 @@ template <typename R> __device__ __forceinline__ R eta_sgn(int i) { return i == 
 // conj(E(r)) = ph[idx(l)] ph[N + 1 + idx(k)] (I3FoldArgs::phase of one term, staged in LDS)
 template <int N> __device__ __forceinline__ constexpr int phase_idx(int x) { return x <= N / 2 ? x : x - N + 1; }
 
+// d + v e, formed in 64 bits: the phases are held and applied as psi1 is in k_padfft.  (FP32 N = 64, 512 cells: 187.4
+// ms per step, with phases and products in FP32 187.6; 193.1 with the phases of the box from a table in memory.)
+template <typename R>
+__device__ __forceinline__ cx<R> add_phased(cx<R> d, cx<R> v, double2 e)
+{
+	const double x = v.x, y = v.y;
+	return mk<R>((R)((double)d.x + x * e.x - y * e.y), (R)((double)d.y + x * e.y + y * e.x));
+}
+
 // IFFT2 of v (R_b), multiplied by conj(E(r)) and added to D on the box of the N x N grid.
 template <typename R, int N, class GE, bool EDGE, class XP>
-__device__ __forceinline__ void mirror_add(cx<R>* v, const XP& X, const cx<R>* tw, int line, int p, const cx<R>* ph, cx<R>* Dp)
+__device__ __forceinline__ void mirror_add(cx<R>* v, const XP& X, const cx<R>* tw, int line, int p, const double2* ph, cx<R>* Dp)
 {
 	constexpr int G = GE::G, E = GE::E, P = GE::P;
 	using El = typename XP::El;
@@ -57,7 +66,7 @@ __device__ __forceinline__ void mirror_add(cx<R>* v, const XP& X, const cx<R>* t
 	const bool keep = unpad<N>(line) >= 0 || (EDGE && line == N / 2);
 	const BufRef<cx<R>> Dr(Dp, MB::SIZE);
 	const int d0 = keep ? MB::lane(line, p) : 0;
-	const cx<R> pk = ph[N + 1 + (keep ? phase_idx<N>(line) : 0)];
+	const double2 pk = ph[N + 1 + (keep ? phase_idx<N>(line) : 0)];
 	constexpr int NB = E / 2 + EDGE;            // elements in the box, EDGE: the last one in lane 0 only
 	constexpr int BL = 4;                       // loads in flight together
 #pragma unroll
@@ -70,10 +79,9 @@ __device__ __forceinline__ void mirror_add(cx<R>* v, const XP& X, const cx<R>* t
 		}
 #pragma unroll
 		for (int k = b; k < b + BL && k < NB; k++) {
-			if ((k - b) % 2 == 0) __builtin_amdgcn_sched_barrier(0);
+			if (E == 8 && (k - b) % 2 == 0) __builtin_amdgcn_sched_barrier(0);
 			const int s = k < E / 4 ? k : (k < E / 2 ? k + E / 2 : E / 4);
-			const cx<R> e = cmul<R>(ph[phase_idx<N>(k == E / 2 ? N / 2 : p + G * s)], pk);
-			const cx<R> x = cadd<R>(d[k - b], cmul<R>(v[s], e));
+			const cx<R> x = add_phased<R>(d[k - b], v[s], cmul<double>(ph[phase_idx<N>(k == E / 2 ? N / 2 : p + G * s)], pk));
 			if (keep && (k < E / 2 || p == 0)) Dr.put(d0, MB::elem(s) * (MB::DL * G), x);
 		}
 		__builtin_amdgcn_sched_barrier(0);
@@ -186,7 +194,7 @@ __global__ __launch_bounds__(T, (FOLD_WPE<R, N>)) void k_i3fold(I3FoldArgs a)
 	using MB = MirrorBox<N, G, E, false>;
 	__shared__ typename XP::El lds[XP::SIZE];
 	__shared__ cx<R> tw[TwTab<P, T>::SIZE];
-	__shared__ cx<R> ph[2 * (N + 1)];           // the mirror's phases of the current term
+	__shared__ double2 ph[2 * (N + 1)];         // the mirror's phases of the current term
 	const FoldRange w(a, 4);
 	if (w.none) return;
 	load_twiddles<R, P, T>(tw, a.tw256);
@@ -196,6 +204,7 @@ __global__ __launch_bounds__(T, (FOLD_WPE<R, N>)) void k_i3fold(I3FoldArgs a)
 	const size_t dstep = (size_t)4 * a.nchunk * a.nblk * MB::SIZE;
 	cx<R>* Dp = (cx<R>*)a.D + 4 * w.cell * dstep + (long long)((j * a.nchunk + w.chunk) * a.nblk + a.resumeD - 1) * MB::SIZE;
 	int nb = 0;                                 // blocks begun
+	auto phase_of = [](const I3FoldArgs& a, int qq) { return (const double2*)a.phase + (size_t)(a.q0 + qq) * (2 * (N + 1)); };
 	auto next_block = [&]() {
 		Dp += MB::SIZE;
 		nb++;
@@ -216,8 +225,6 @@ __global__ __launch_bounds__(T, (FOLD_WPE<R, N>)) void k_i3fold(I3FoldArgs a)
 			// (the term's barriers are before the mirror's reads)
 			next_block();
 		}
-		cx<R> phv = czero<R>();
-		if (mir && t < 2 * (N + 1)) phv = ((const cx<R>*)a.phase)[(size_t)(a.q0 + qq) * (2 * (N + 1)) + t];
 #pragma unroll 1
 		for (int i = 0; i < 4; i++) {
 			{
@@ -226,14 +233,16 @@ __global__ __launch_bounds__(T, (FOLD_WPE<R, N>)) void k_i3fold(I3FoldArgs a)
 					[&](int u, const Two<cx<R>, cx<R>>& x) { v[u] = cmul<R>(x.a, x.b); });
 			}
 			k_apply<R, GE>(v, ps, X, tw, line, p);
-			// (this product's barriers are behind the previous term's reads, the mirror's before this one's)
-			if (i == 0 && t < 2 * (N + 1)) ph[t] = phv;
+			// (this product's barriers are behind the previous term's reads of ph, the mirror's before this one's)
+			double2 phv = make_double2(0, 0);
+			if (i == 0 && mir && t < 2 * (N + 1)) phv = phase_of(a, qq)[t];
 			{
 				const R ei = eta_sgn<R>(i);
 				const BufRef<cx<R>> f(Fq + (size_t)i * (P * P), P * P);
 				acc.template add<B>([&](int u) { return f.get(t, u * T); },
 					[&](int u, cx<R> x) { return cscale<R>(cmul<R>(x, v[u]), ei); });
 			}
+			if (i == 0 && t < 2 * (N + 1)) ph[t] = phv;
 			if (mir) {
 				const BufRef<cx<R>> s(Sh + (size_t)j * (P * P), P * P);
 				batched<E, B>([&](int u) { return s.get(t, u * T); },
@@ -264,7 +273,7 @@ __global__ __launch_bounds__(T, (FOLD_WPE<R, N>)) void k_i3fold_pair(I3FoldArgs 
 	using MB = MirrorBox<N, G, E, true>;
 	__shared__ typename XP::El lds[XP::SIZE];
 	__shared__ cx<R> tw[TwTab<P, T>::SIZE];
-	__shared__ cx<R> ph[2 * (N + 1)];           // the mirror's phases of the current term
+	__shared__ double2 ph[2 * (N + 1)];         // the mirror's phases of the current term
 	const FoldRange w(a, 4);
 	if (w.none) return;
 	load_twiddles<R, P, T>(tw, a.tw256);
@@ -274,6 +283,7 @@ __global__ __launch_bounds__(T, (FOLD_WPE<R, N>)) void k_i3fold_pair(I3FoldArgs 
 	cx<R>* Dp = (cx<R>*)a.D + ((((size_t)w.cell * 2 + pr) * 2 + J) * a.nchunk + w.chunk) * a.nblk * MB::SIZE +
 		(long long)(a.resumeD - 1) * MB::SIZE;
 	int nb = 0;                                 // blocks begun
+	auto phase_of = [](const I3FoldArgs& a, int qq) { return (const double2*)a.phase + (size_t)(a.q0 + qq) * (2 * (N + 1)); };
 	auto next_block = [&]() {
 		Dp += MB::SIZE;
 		nb++;
@@ -299,8 +309,6 @@ __global__ __launch_bounds__(T, (FOLD_WPE<R, N>)) void k_i3fold_pair(I3FoldArgs 
 			// (the term's barriers are before the mirror's reads)
 			next_block();
 		}
-		cx<R> phv = czero<R>();
-		if (mir && t < 2 * (N + 1)) phv = ((const cx<R>*)a.phase)[(size_t)(a.q0 + qq) * (2 * (N + 1)) + t];
 		R bx[E];
 		// v = component c of the instance pair times F_J
 		auto product = [&](int c) {
@@ -316,9 +324,11 @@ __global__ __launch_bounds__(T, (FOLD_WPE<R, N>)) void k_i3fold_pair(I3FoldArgs 
 		};
 		product(0);
 		k_apply<R, GE>(v, ps, X, tw, line, p);
-		// (the barriers of this product are behind the previous term's reads, those of the next before this one's)
-		if (t < 2 * (N + 1)) ph[t] = phv;
+		// (the barriers of this product are behind the previous term's reads of ph, those of the next before this one's)
+		double2 phv = make_double2(0, 0);
+		if (mir && t < 2 * (N + 1)) phv = phase_of(a, qq)[t];
 		accumulate(0, ei);
+		if (t < 2 * (N + 1)) ph[t] = phv;
 		{
 			const BufRef<cx<R>> s(SJ, P * P);
 			batched<E, B>([&](int u) { return s.get(t, u * T); },

@@ -182,9 +182,12 @@ __global__ __launch_bounds__(T) void k_i1acc(I1Args a)
 	const cx<R>* Fh = (const cx<R>*)a.Fhat + ((size_t)cell * a.nFh + a.instFh[inst]) * (P * P);
 	const R fa = (R)a.fa, fb = (R)a.fb;
 	XP X{lds};
-	cx<R> acc[E], v[E];
+	// 64-bit sums: the low frequencies of the terms are sums over the whole grid.  32 terms added in FP32 there
+	// were the largest part of an FP32 step's error with one range per cell (N = 64, 512 cells: 3.2e-10 -> 2.2e-10)
+	double2 acc[E];
+	cx<R> v[E];
 #pragma unroll
-	for (int s = 0; s < E; s++) acc[s] = czero<R>();
+	for (int s = 0; s < E; s++) acc[s].x = acc[s].y = 0;
 	__syncthreads();
 	for (int q = qa; q < qb; q++) {
 		padfft_reg<R, N, GE>(v, g, a.phi + (size_t)q * (N * N), 1, X, tw, line, p);
@@ -199,12 +202,14 @@ __global__ __launch_bounds__(T) void k_i1acc(I1Args a)
 #pragma unroll
 		for (int s = 0; s < E; s++) {
 			const R w = uni(ps, (long long)s * T)[threadIdx.x];
-			acc[s].x += w * v[s].x;
-			acc[s].y += w * v[s].y;
+			acc[s].x += (double)w * v[s].x;
+			acc[s].y += (double)w * v[s].y;
 		}
 	}
-	fft2_reg<R, GE>(acc, X, tw, line, p);
-	store_native<R, GE>((cx<R>*)a.out + (((size_t)cell * a.ninst + inst) * a.nchunk + chunk) * (P * P), acc);
+#pragma unroll
+	for (int s = 0; s < E; s++) v[s] = mk<R>((R)acc[s].x, (R)acc[s].y);
+	fft2_reg<R, GE>(v, X, tw, line, p);
+	store_native<R, GE>((cx<R>*)a.out + (((size_t)cell * a.ninst + inst) * a.nchunk + chunk) * (P * P), v);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -572,6 +577,8 @@ __global__ __launch_bounds__(256) void k_sum_mirror(const cx<R>* __restrict__ in
 	out[i] = s;
 }
 
+template <typename R> __device__ __forceinline__ double2 wide(cx<R> z) { return make_double2((double)z.x, (double)z.y); }
+
 // The physical-domain sum of a collision evaluation, per cell and grid element, V [cell][4][PP]
 // (src/collision.c:82-167, 220-253; the term sums of the integrals are linear):
 //   Cc: V_1 += c4 (W_3 A_2 - W_2 A_3) and cyclic,
@@ -579,13 +586,18 @@ __global__ __launch_bounds__(256) void k_sum_mirror(const cx<R>* __restrict__ in
 //       V_0 -= 2 c4 sum_j W_j B_j.
 // Every input is read once for the four outputs; an input that comes as partial sums over term ranges
 // is added up here.  CL > 1: CL threads share an element and add the parts c, c + CL, ... (few cells,
-// many ranges).  Replaces four launches that added the parts in place and 70 grid reads a cell in
-// k_combine (memory-bound): one cell, N = 32, FP64, 128 ranges: 218 -> 60 us with what k_combine keeps.
+// many ranges).  Formed in 64 bits also for FP32 grids: the gain and loss terms cancel in part, and their products
+// in FP32 were a sixth of an FP32 step's error (N = 64, 10 cells: 1.98e-10 -> 1.71e-10).
+// Replaces four launches that added the parts in place and 70 grid reads a cell in k_combine (memory-bound):
+// one cell, N = 32, FP64, 128 ranges: 218 -> 60 us with what k_combine keeps.
 template <typename R, int CL>
 __global__ __launch_bounds__(256) void k_assemble(AssembleArgs a)
 {
 	constexpr int NE = 256 / CL, NI = 15;
 	__shared__ cx<R> sh[CL > 1 ? NI : 1][CL > 1 ? 256 : 1];
+	// a slot's sums take the place of its parts, all of which the half wave that writes them has read (in a place of
+	// their own one workgroup less fits on a CU: FP32 N = 32, 256 cells 238 us instead of 194)
+	auto sum = [&](int k) { return (double2*)&sh[k][0]; };
 	const int c = threadIdx.x / NE, x = threadIdx.x % NE;
 	const long long i = (long long)blockIdx.x * NE + x;
 	const bool in = i < a.n;
@@ -593,22 +605,22 @@ __global__ __launch_bounds__(256) void k_assemble(AssembleArgs a)
 	// this thread's share of the sum of a slot's parts
 	auto part = [&](const void* buf, int nslot, int slot, int nch) {
 		const cx<R>* p = (const cx<R>*)buf + ((cell * nslot + slot) * nch) * a.PP + e;
-		cx<R> z = czero<R>();
-		for (int k = c; k < nch; k += CL) z = cadd<R>(z, p[(long long)k * a.PP]);
+		double2 z = czero<double>();
+		for (int k = c; k < nch; k += CL) z = cadd<double>(z, wide<R>(p[(long long)k * a.PP]));
 		return z;
 	};
 	// 0..2: A of spin component 1..3, 3..6: B, 7..10: S, 11..14: acc
-	cx<R> g[NI];
+	double2 g[NI];
 #pragma unroll
-	for (int k = 0; k < NI; k++) g[k] = czero<R>();
-	auto two = [&](int k, cx<R> z) {         // a packed slot: two real values
-		g[k] = mk<R>(z.x, R(0));
-		g[k + 1] = mk<R>(z.y, R(0));
+	for (int k = 0; k < NI; k++) g[k] = czero<double>();
+	auto two = [&](int k, double2 z) {         // a packed slot: two real values
+		g[k] = make_double2(z.x, 0.0);
+		g[k + 1] = make_double2(z.y, 0.0);
 	};
 	if (in && a.A) {
 		if (a.pairAB) {
 			two(1, part(a.A, 2, 0, a.nchA));
-			g[0] = mk<R>(part(a.A, 2, 1, a.nchA).x, R(0));
+			g[0] = make_double2(part(a.A, 2, 1, a.nchA).x, 0.0);
 		} else {
 			for (int k = 0; k < 3; k++) g[k] = part(a.A, 3, k, a.nchA);
 		}
@@ -626,47 +638,47 @@ __global__ __launch_bounds__(256) void k_assemble(AssembleArgs a)
 	}
 	if constexpr (CL > 1) {
 #pragma unroll
-		for (int k = 0; k < NI; k++) sh[k][threadIdx.x] = g[k];
+		for (int k = 0; k < NI; k++) sh[k][threadIdx.x] = mk<R>((R)g[k].x, (R)g[k].y);
 		__syncthreads();
 		for (int k = c; k < NI; k += CL) {
-			cx<R> z = sh[k][x];
-			for (int d = 1; d < CL; d++) z = cadd<R>(z, sh[k][d * NE + x]);
-			sh[k][x] = z;
+			double2 z = wide<R>(sh[k][x]);
+			for (int d = 1; d < CL; d++) z = cadd<double>(z, wide<R>(sh[k][d * NE + x]));
+			sum(k)[x] = z;
 		}
 		__syncthreads();
 #pragma unroll
-		for (int k = 0; k < NI; k++) g[k] = sh[k][x];
+		for (int k = 0; k < NI; k++) g[k] = sum(k)[x];
 	}
 	if (!in) return;
 	const cx<R>* Wp = (const cx<R>*)a.What + cell * 4 * a.PP + e;
 	cx<R>* V = (cx<R>*)a.V + cell * 4 * a.PP + e;
-	cx<R> W[4];
+	double2 W[4];
 #pragma unroll
-	for (int k = 0; k < 4; k++) W[k] = Wp[(long long)k * a.PP];
-	const R c4 = (R)a.c4, c2 = (R)a.c2;
+	for (int k = 0; k < 4; k++) W[k] = wide<R>(Wp[(long long)k * a.PP]);
+	const double c4 = a.c4, c2 = a.c2;
 #pragma unroll
 	for (int j = 0; j < 4; j++) {
 		if (CL > 1 && j != c) continue;
-		cx<R> v = czero<R>();
+		double2 v = czero<double>();
 		if (a.A && j > 0) {
 			const int k = j % 3 + 1, l = (j + 1) % 3 + 1;      // (j, k, l) cyclic
-			v = cscale<R>(csub<R>(cmul<R>(W[l], g[k - 1]), cmul<R>(W[k], g[l - 1])), c4);
+			v = cscale<double>(csub<double>(cmul<double>(W[l], g[k - 1]), cmul<double>(W[k], g[l - 1])), c4);
 		}
 		if (a.B) {
-			const R e2 = j == 0 ? R(2) : R(-2);
-			cx<R> q = cscale<R>(csub<R>(cmul<R>(W[0], g[3 + j]), g[11 + j]), e2);
-			q = cadd<R>(q, cscale<R>(cmul<R>(W[j], g[3]), R(2)));
+			const double e2 = j == 0 ? 2.0 : -2.0;
+			double2 q = cscale<double>(csub<double>(cmul<double>(W[0], g[3 + j]), g[11 + j]), e2);
+			q = cadd<double>(q, cscale<double>(cmul<double>(W[j], g[3]), 2.0));
 			if (j == 0) {
-				cx<R> t = cmul<R>(W[0], g[3]);
+				double2 t = cmul<double>(W[0], g[3]);
 #pragma unroll
-				for (int k = 1; k < 4; k++) t = cadd<R>(t, cmul<R>(W[k], g[3 + k]));
-				q = csub<R>(q, cscale<R>(t, R(2)));
+				for (int k = 1; k < 4; k++) t = cadd<double>(t, cmul<double>(W[k], g[3 + k]));
+				q = csub<double>(q, cscale<double>(t, 2.0));
 			}
-			const cx<R> S = cscale<R>(csub<R>(csub<R>(csub<R>(g[7], g[8]), g[9]), g[10]), R(2));
-			const cx<R> w = mk<R>((j == 0 ? R(1) : R(0)) - W[j].x, -W[j].y);
-			v = cadd<R>(v, cadd<R>(cscale<R>(q, c4), cscale<R>(cmul<R>(w, S), c2)));
+			const double2 S = cscale<double>(csub<double>(csub<double>(csub<double>(g[7], g[8]), g[9]), g[10]), 2.0);
+			const double2 w = make_double2((j == 0 ? 1.0 : 0.0) - W[j].x, -W[j].y);
+			v = cadd<double>(v, cadd<double>(cscale<double>(q, c4), cscale<double>(cmul<double>(w, S), c2)));
 		}
-		V[(long long)j * a.PP] = v;
+		V[(long long)j * a.PP] = mk<R>((R)v.x, (R)v.y);
 	}
 }
 

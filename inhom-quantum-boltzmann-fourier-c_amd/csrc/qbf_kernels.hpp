@@ -92,7 +92,7 @@ struct I3FoldArgs {
 	const int* terms;     // [0]: terms with an index below it stand for a mirrored pair, [1]: terms to take in all
 	                      // (read on the device: a captured launch follows a table that is replaced)
 	const void* psi2n;    // [nqTotal][P*P] C_i native
-	const void* phase;    // [nmir][2][N+1] conj(E) along l and along k, frequencies 0 .. N/2, -N/2 .. -1
+	const void* phase;    // [nmir][2][N+1] conj(E) along l and along k, frequencies 0 .. N/2, -N/2 .. -1, 64 bits
 	int nchunk;
 	int accumulate;
 	void* acc;            // [ncell][no][na][P*P] R_b native
