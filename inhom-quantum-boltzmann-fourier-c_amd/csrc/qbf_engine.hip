@@ -484,7 +484,7 @@ struct EngineT final : public qbf_engine {
 	static constexpr double MIRROR_TOL = 4e-13;
 	static bool is_mirror(const double* a1, const double* a2, const double* b1, const double* b2)
 	{
-		const double scale = fabs(a2[0]) > 0 ? fabs(a2[0]) : 1.0;     // psi2's value at the origin sets its scale
+		const double scale = fabs(a2[0]);       // psi2's value at the origin sets its scale (0: equal values only)
 		auto near = [](const double* a, const double* b, int n, double sgn, double tol) {
 			double worst = 0;
 			for (int i = 0; i < n; i++) {
