@@ -24,7 +24,9 @@
 // for T = 1024 threads: with k = 64 b + 16 f + 4 c + j (b < 2, f, c, j < 4), element (l, k) at
 // (4 f + j) * 1024 + 64 (l / 8) + 16 c + 2 (l % 8) + b.  In a load of the rows pass the 8 lanes of a
 // row block and the lanes kq, kq + 2 read 128 contiguous bytes (columns first: 16 bytes, 65.0 instead of
-// 56.7 ms per collision step of 64 cells).
+// 56.7 ms per collision step of 64 cells).  The operands are loaded in batches (see batched): left to itself
+// the compiler used one register pair for them, each load waited for before the next, and the step of 64 cells
+// took 56.8 ms, 38.1 with the batches (complex grids 122 and 74; batches of 8 and 16 operand pairs 38.8 and 42.9).
 #pragma once
 #include "qbf_device.hpp"
 #include "qbf_kernels.hpp"
@@ -221,19 +223,17 @@ __global__ __launch_bounds__(mf::T) void k_i3acc_mfma(I3Args a)
 			const float2* Fh = Fq + (size_t)(PAIR ? hs >> 1 : hs) * (P * P);
 			const float2* Ff = Fq + (size_t)a.instF[out][in] * (P * P);
 			// X = S .* H in the rows-pass order
-#pragma unroll
-			for (int r = 0; r < 4; r++)
-#pragma unroll
-				for (int t = 0; t < 8; t++) {
-					const float2 sv = at(Sg, go(r, t), gb);
-					const float2 h = at(Fh, go(r, t), gb);
+			batched<32, 4>(
+				[&](int u) { return Two<float2, float2>{at(Sg, go(u >> 3, u & 7), gb), at(Fh, go(u >> 3, u & 7), gb)}; },
+				[&](int u, const Two<float2, float2>& x) {
+					float2& y = d[u & 7][u >> 3];
 					if constexpr (PAIR) {
-						const float hv = (hs & 1) ? h.y : h.x;
-						d[t][r] = make_float2(sv.x * hv, sv.y * hv);
+						const float hv = (hs & 1) ? x.b.y : x.b.x;
+						y = make_float2(x.a.x * hv, x.a.y * hv);
 					} else {
-						d[t][r] = cmul<float>(sv, h);
+						y = cmul<float>(x.a, x.b);
 					}
-				}
+				});
 			// IFFT along k (rows pass), out: columns 4 kq + r + 16 t
 			__builtin_amdgcn_sched_barrier(0);
 			line_bwd128(d, mb, tw, kq);
@@ -277,23 +277,17 @@ __global__ __launch_bounds__(mf::T) void k_i3acc_mfma(I3Args a)
 			__builtin_amdgcn_sched_barrier(0);
 			if constexpr (PAIR) {
 				const float wa = (float)a.instW[out][2 * in], wb = (float)a.instW[out][2 * in + 1];
-#pragma unroll
-				for (int r = 0; r < 4; r++)
-#pragma unroll
-					for (int t = 0; t < 8; t++) {
-						const float2 f = at(Ff, go(r, t), gb);
-						acc[t][r][0] += (wa * f.x) * d[t][r].x + (wb * f.y) * d[t][r].y;
-					}
+				batched<32, 8>([&](int u) { return at(Ff, go(u >> 3, u & 7), gb); }, [&](int u, float2 f) {
+					const float2 y = d[u & 7][u >> 3];
+					acc[u & 7][u >> 3][0] += (wa * f.x) * y.x + (wb * f.y) * y.y;
+				});
 			} else {
 				const float wt = (float)a.instW[out][in];
-#pragma unroll
-				for (int r = 0; r < 4; r++)
-#pragma unroll
-					for (int t = 0; t < 8; t++) {
-						const float2 y = cmul<float>(at(Ff, go(r, t), gb), d[t][r]);
-						acc[t][r][0] += wt * y.x;
-						acc[t][r][PAIR ? 0 : 1] += wt * y.y;
-					}
+				batched<32, 8>([&](int u) { return at(Ff, go(u >> 3, u & 7), gb); }, [&](int u, float2 f) {
+					const float2 y = cmul<float>(f, d[u & 7][u >> 3]);
+					acc[u & 7][u >> 3][0] += wt * y.x;
+					acc[u & 7][u >> 3][PAIR ? 0 : 1] += wt * y.y;
+				});
 			}
 		}
 	}
