@@ -292,7 +292,7 @@ void on_threads(unsigned n, int nel, F fn)
 	std::vector<std::thread> th;
 	try {
 		const unsigned want = std::min({8u, std::max(1u, std::thread::hardware_concurrency()),
-			(unsigned)((unsigned long long)n * nel >> 19)});
+			(unsigned)((unsigned long long)n * nel >> 17)});
 		for (unsigned t = 1; t < want; t++) th.emplace_back(work);
 	} catch (const std::exception&) {
 	}
