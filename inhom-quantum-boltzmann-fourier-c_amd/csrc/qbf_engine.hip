@@ -339,7 +339,7 @@ struct EngineT final : public qbf_engine {
 	bool mfmaI3 = false;
 	DevBuf i3p2m;
 
-	DevBuf What, Ahat, Bhat, Sbuf, acc3, Dmir, Dsum, Vsum, Fscr, xscr;
+	DevBuf What, Ahat, Bhat, Sbuf, acc3, Dmir, Dsum, Fscr, xscr;
 	// Combination-term tables: each distinct table is uploaded once and its device copy reused, so
 	// that evaluations after the first of a configuration issue no host copy and no synchronisation
 	// (which makes the step capturable in a HIP graph).  At most TERM_CACHE tables are kept.
@@ -359,7 +359,7 @@ struct EngineT final : public qbf_engine {
 	int init()
 	{
 		for (DevBuf* b : {&i1[0].phi, &i1[0].psi1n, &i1[1].phi, &i1[1].psi1n, &i2p1, &i2p2, &i2pc, &i3p1, &i3p2n, &i3ph, &i3n, &i3p2m,
-			     &What, &Ahat, &Bhat, &Sbuf, &acc3, &Dmir, &Dsum, &Vsum, &Fscr, &xscr, &Wmid, &WF, &WF2, &Wt1, &Wt2, &src3, &Wpk,
+			     &What, &Ahat, &Bhat, &Sbuf, &acc3, &Dmir, &Dsum, &Fscr, &xscr, &Wmid, &WF, &WF2, &Wt1, &Wt2, &src3, &Wpk,
 			     &WhatP, &reim, &Cf})
 			b->lock = &liveGraphs;
 		return ensure_twiddles();
@@ -732,7 +732,7 @@ struct EngineT final : public qbf_engine {
 		qr = Fscr.fit((size_t)ncell * nF * GB, qr);
 		if (nchunk > qr) nchunk = qr;
 		nchunk = fit_ranges(ncell * nout, nchunk);
-		int r = Fscr.ensure((size_t)ncell * nF * GB * qr);
+		int r = Fscr.ensure((size_t)ncell * GB * std::max(nF * qr, 4));
 		if (!r) r = acc3.ensure((size_t)ncell * nout * nchunk * GB);
 		if (r) return r;
 		for (int q0 = 0; q0 < nq; q0 += qr) {
@@ -905,7 +905,7 @@ struct EngineT final : public qbf_engine {
 		while (qr > DBLOCK<R> && !Dmir.holds(blkB * nchunk * blocks())) qr = (blocks() - 1) * DBLOCK<R>;
 		const int nblk = blocks();
 		const int group = nblk > 1 ? 1 : DBLOCK<R> / ((qr + nchunk - 1) / nchunk);
-		int r = Fscr.ensure((size_t)ncell * NO * GB * qr);
+		int r = Fscr.ensure((size_t)ncell * GB * std::max(NO * qr, 4));
 		// (four grids a cell, as run_i3 takes, also where the pair kernel at N = 128 has two)
 		if (!r) r = acc3.ensure((size_t)ncell * GB * std::max(NO * NI * nchunk, 4));
 		if (!r) r = Dmir.ensure(blkB * nchunk * nblk);
@@ -1057,10 +1057,11 @@ struct EngineT final : public qbf_engine {
 
 	int assemble(AssembleArgs& a, int ncell)
 	{
-		int r = Vsum.ensure((size_t)ncell * 4 * GB);
+		// the sums take the place of the F grids, which the I3 kernels have read
+		int r = Fscr.ensure((size_t)ncell * 4 * GB);
 		if (r) return r;
 		const double p2 = 1.0 / ((double)P * P);
-		a.c2 = p2; a.c4 = p2 * p2; a.V = Vsum.p; a.PP = PP; a.n = (long long)ncell * PP;
+		a.c2 = p2; a.c4 = p2 * p2; a.V = Fscr.p; a.PP = PP; a.n = (long long)ncell * PP;
 		int most = 1;
 		for (int n : {a.A ? a.nchA : 1, a.B ? a.nchB : 1, a.B ? a.nchS : 1, a.B ? a.nchAcc : 1}) most = n > most ? n : most;
 		// parts shared by 8 threads where there are more than 4 of them (few cells)
@@ -1166,7 +1167,7 @@ struct EngineT final : public qbf_engine {
 		double Dcoef[4];
 		const double p2 = 1.0 / ((double)P * P), eta2[4] = {2, -2, -2, -2};
 		for (int j = 0; j < 4; j++) {
-			tl[j].push_back(term(nullptr, 0, Vsum.template as<C>() + (size_t)j * PP, 4LL * PP, 1.0));
+			tl[j].push_back(term(nullptr, 0, Fscr.template as<C>() + (size_t)j * PP, 4LL * PP, 1.0));
 			Dcoef[j] = -eta2[j] * p2 * p2;
 		}
 		return launch_combine(tl, 4, all4, ncell, out, base, Wcb, Bext, cf, fold ? Dsum.template as<double2>() : nullptr,

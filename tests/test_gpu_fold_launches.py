@@ -86,3 +86,25 @@ def test_unpaired_terms_at_n128(prec, tol):
     e.set_real_pairs(0, 0.0)
     assert l1rel(e.collision(torch.from_numpy(WF).cuda(), mode=qbf.CD).cpu().numpy()[0], ref) < tol
     e.close()
+
+
+def test_memory_of_a_benchmark_step():
+    """512 cells at N = 64, FP32, packed pairs: 8 GiB of F grids, 21 padded grids a cell (1.3 GiB), the states (0.6), the
+    tables (0.1), the mirror sums (0.2), in all 10.2; the sums that k_combine transforms have no grids of their own
+    (0.25 more)."""
+    from qbf import workloads as wl
+    N, n = 64, 512
+    W = torch.from_numpy(wl.periodic(N, n, seed=1)).cuda()
+    q = qbf.quadrature(N, 32, L, R, 16)
+    out = torch.empty_like(W)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    e = qbf.Engine(N, qbf.FP32, max_cells=n)
+    e.set_quadrature(*q)
+    e.set_real_pairs(2, 0.0)
+    e.inhom_step_periodic(W, L, 1 / n, wl.cfl_dt(N, n), out=out)
+    torch.cuda.synchronize()
+    used = (free - torch.cuda.mem_get_info()[0]) / 2 ** 30
+    e.close()
+    print(f"{used:.2f} GiB", flush=True)
+    assert used < 10.4
