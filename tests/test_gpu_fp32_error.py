@@ -31,3 +31,25 @@ def test_fp32_step_error(N, n, J, M, Nx, pairs, kmax, bound):
         err.append(l1rel(out[1], out[0]))
     print(f"N = {N}, {n} cells, pairs {pairs}: {np.mean(err):.3e} (bound {bound:.3e})", flush=True)
     assert np.mean(err) < bound
+
+
+@pytest.mark.parametrize("N,n,J,M,Nx,kmax,bound", [(64, 300, 20, 10, 512, 4, 1.912e-10), (32, 400, 32, 16, 512, 4, 2.072e-10),
+                                                   (128, 48, 16, 8, 2048, 8, 4.248e-11)])
+def test_fp32_strang_step_error(N, n, J, M, Nx, kmax, bound):
+    """L2 error of conserved Strang steps with one term range per cell (many cells), six states."""
+    q = qbf.quadrature(N, J, wl.L_BOX, wl.R_BALL, M)
+    h, dt = 1 / Nx, wl.cfl_dt(64, Nx)
+    es = []
+    for prec in (qbf.FP64, qbf.FP32):
+        es.append(qbf.Engine(N, prec, max_cells=n))
+        es[-1].set_quadrature(*q)
+        es[-1].set_moment_correction(qbf.CONS_ALL)
+    err = []
+    for seed in range(5, 11):
+        W = torch.from_numpy(wl.periodic(N, n, seed=seed, kmax=kmax)).cuda()
+        a, b = (e.inhom_step_periodic(W, wl.L_BOX, h, dt) for e in es)
+        err.append(float((a - b).norm() / a.norm()))
+    for e in es:
+        e.close()
+    print(f"N = {N}, {n} cells: {np.mean(err):.3e} (bound {bound:.3e})", flush=True)
+    assert np.mean(err) < bound
