@@ -46,16 +46,13 @@ REF_FILE = os.path.join(ROOT, "tests", "golden", "periodic64_fp64_ref.npz")
 # (FETCH_SIZE, then WRITE_SIZE), each counter scaled by its reading for the 256 MiB device copy of the
 # same run (FETCH_SIZE x 2.000, WRITE_SIZE x 1.000); the line's `traffic` is this times the average
 # number of applications per launch in the timed region.
-# N=64 (k_i3acc<float, 64, 1024>), `bench.py --no-cpu-baseline --paths mixed,bf16x3,fp64 --mixed-steps 1
-# --fp64-steps 1 --warmup 0 --c3-steps 0 --copy-calibration`: paired launches of 64 quadrature terms x 512
-# cells x 8 applications, FETCH_SIZE 8.97e6 KiB + WRITE_SIZE 2.62e5 KiB = 18.65 GB per launch (algorithmic
-# bytes 8.7 GB: F grids 8 GiB, transformed state 128 MiB, accumulator read + write 512 MiB); the complex
-# kernel was measured with launches of 8 terms x 512 cells x 16 applications (10.34 GB).
-I3_TRAFFIC_PER_APP = {False: 10.34e9 / 65536, True: 18.65e9 / 262144}
-# N=128 (k_i3acc_big<float>), `bench.py --N 128 --Nx 64 --kmax 8 --no-cpu-baseline --paths mixed,fp64
-# --mixed-steps 1 --fp64-steps 1 --warmup 0 --c3-steps 0 --copy-calibration`: 8192 applications per launch
-# (the scratch grids of the line passes go through HBM): complex 30.9 GB, paired 29.9 GB per launch
-I3_TRAFFIC_PER_APP_N128 = {False: 3.77e6, True: 3.65e6}
+# N=64, two collision evaluations each: paired (k_i3fold_pair<float, 64, 1024>), 512 cells, J=32, M=16: launches of
+# 64 folded terms x 512 cells x 8 applications, FETCH_SIZE 2.087e7 KiB + WRITE_SIZE 4.77e6 KiB = 47.6 GB; complex
+# (k_i3fold<float, 64, 1024>), 128 cells: 128 folded terms x 128 cells x 16, 4.246e7 + 8.72e6 KiB = 95.9 GB.
+I3_TRAFFIC_PER_APP = {False: 95.9e9 / 262144, True: 47.6e9 / 262144}
+# N=128 (k_i3fold_big<float>), 64 cells, launches of 32,768 applications (the scratch grids of the line passes go
+# through HBM): complex 133.1 GB, paired 117.4 GB
+I3_TRAFFIC_PER_APP_N128 = {False: 133.1e9 / 32768, True: 117.4e9 / 32768}
 
 
 def cpu_baseline(N, J, M, cores, seed):

@@ -673,8 +673,10 @@ struct EngineT final : public qbf_engine {
 		if (r) return r;
 		if constexpr (BIG)
 			hipLaunchKernelGGL((k_i1acc_big<R>), dim3(ncell * ninst * nch), dim3(T), 0, stream, a);
+		else if ((i1[slot].n + nch - 1) / nch > I1_F32)
+			hipLaunchKernelGGL((k_i1acc<R, N, T, SP, double>), dim3(ncell * ninst * nch), dim3(T), 0, stream, a);
 		else
-			hipLaunchKernelGGL((k_i1acc<R, N, T, SP>), dim3(ncell * ninst * nch), dim3(T), 0, stream, a);
+			hipLaunchKernelGGL((k_i1acc<R, N, T, SP, R>), dim3(ncell * ninst * nch), dim3(T), 0, stream, a);
 		HIPCHK(hipGetLastError());
 		*nchunk = nch;
 		return 0;

@@ -162,7 +162,12 @@ __global__ __launch_bounds__(T) void k_padfft(PadFFTArgs a)
 }
 
 // ---------------------------------------------------------------------------------------------
-template <typename R, int N, int T, bool SP>
+// A: type of the sums over the terms.  Their low frequencies are sums over the whole grid: 32 terms added in FP32
+// there were the largest part of an FP32 step's error with one range per cell (N = 64, 512 cells: 3.2e-10 with, 2.2e-10
+// without), so FP32 grids are summed in 64 bits where a range has more than I1_F32 terms.  It takes registers
+// (10 cells, N = 64, ranges of 4 terms: 101 us a launch, 85 with FP32 sums, and the step's error is 1.67e-10 or 1.71e-10).
+constexpr int I1_F32 = 4;
+template <typename R, int N, int T, bool SP, typename A>
 __global__ __launch_bounds__(T) void k_i1acc(I1Args a)
 {
 	using GE = Geo<2 * N, T>;
@@ -182,12 +187,10 @@ __global__ __launch_bounds__(T) void k_i1acc(I1Args a)
 	const cx<R>* Fh = (const cx<R>*)a.Fhat + ((size_t)cell * a.nFh + a.instFh[inst]) * (P * P);
 	const R fa = (R)a.fa, fb = (R)a.fb;
 	XP X{lds};
-	// 64-bit sums: the low frequencies of the terms are sums over the whole grid.  32 terms added in FP32 there
-	// were the largest part of an FP32 step's error with one range per cell (N = 64, 512 cells: 3.2e-10 -> 2.2e-10)
-	double2 acc[E];
+	cx<A> acc[E];
 	cx<R> v[E];
 #pragma unroll
-	for (int s = 0; s < E; s++) acc[s].x = acc[s].y = 0;
+	for (int s = 0; s < E; s++) acc[s] = czero<A>();
 	__syncthreads();
 	for (int q = qa; q < qb; q++) {
 		padfft_reg<R, N, GE>(v, g, a.phi + (size_t)q * (N * N), 1, X, tw, line, p);
@@ -202,8 +205,8 @@ __global__ __launch_bounds__(T) void k_i1acc(I1Args a)
 #pragma unroll
 		for (int s = 0; s < E; s++) {
 			const R w = uni(ps, (long long)s * T)[threadIdx.x];
-			acc[s].x += (double)w * v[s].x;
-			acc[s].y += (double)w * v[s].y;
+			acc[s].x += (A)w * v[s].x;
+			acc[s].y += (A)w * v[s].y;
 		}
 	}
 #pragma unroll
