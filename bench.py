@@ -47,12 +47,12 @@ REF_FILE = os.path.join(ROOT, "tests", "golden", "periodic64_fp64_ref.npz")
 # same run (FETCH_SIZE x 2.000, WRITE_SIZE x 1.000); the line's `traffic` is this times the average
 # number of applications per launch in the timed region.
 # N=64, two collision evaluations each: paired (k_i3fold_pair<float, 64, 1024>), 512 cells, J=32, M=16: launches of
-# 64 folded terms x 512 cells x 8 applications, FETCH_SIZE 2.087e7 KiB + WRITE_SIZE 4.77e6 KiB = 47.6 GB; complex
-# (k_i3fold<float, 64, 1024>), 128 cells: 128 folded terms x 128 cells x 16, 4.246e7 + 8.72e6 KiB = 95.9 GB.
-I3_TRAFFIC_PER_APP = {False: 95.9e9 / 262144, True: 47.6e9 / 262144}
+# 64 folded terms x 512 cells x 8 applications, FETCH_SIZE 2.047e7 KiB + WRITE_SIZE 4.94e6 KiB = 47.0 GB; complex
+# (k_i3fold<float, 64, 1024>), 128 cells: 128 folded terms x 128 cells x 16, 4.330e7 + 8.98e6 KiB = 97.9 GB.
+I3_TRAFFIC_PER_APP = {False: 97.9e9 / 262144, True: 47.0e9 / 262144}
 # N=128 (k_i3fold_big<float>), 64 cells, launches of 32,768 applications (the scratch grids of the line passes go
-# through HBM): complex 133.1 GB, paired 117.4 GB
-I3_TRAFFIC_PER_APP_N128 = {False: 133.1e9 / 32768, True: 117.4e9 / 32768}
+# through HBM): complex 132.9 GB, paired 116.8 GB
+I3_TRAFFIC_PER_APP_N128 = {False: 132.9e9 / 32768, True: 116.8e9 / 32768}
 
 
 def cpu_baseline(N, J, M, cores, seed):

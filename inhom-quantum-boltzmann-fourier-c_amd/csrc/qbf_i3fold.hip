@@ -13,11 +13,13 @@
 // the 2N grid).  One pass over the 16 products K_q[S_i .* F_j,q] therefore serves both terms, with
 // one IFFT2 per mirror output more and the N x N box of the sum over q kept in frequency space (D).
 //
-// What bounds it: the line FFTs of the K applications on the VALU (82% busy at FP32 N = 64, 63% at
-// FP64 N = 32), at FP64 N = 64 the exchange and the accumulators' traffic.  A term pair costs 16
-// applications and 16 pruned IFFT2 of three quarters of a transform (packed pairs: 8 and 4) instead of
-// 32 (16) applications.  Strang steps before -> after: FP32 N = 64, 512 cells 327 -> 206 ms; FP64 N = 32,
-// 128 cells 58.9 -> 42.3 ms; FP64 N = 64, 16 cells 62.5 -> 41.8 ms; FP32 N = 128, 32 cells 76.5 -> 48.5 ms.
+// What bounds it: in FP32 at N = 64 the line FFTs of the K applications on the VALU (72% busy with packed pairs,
+// 80% with complex grids) and a barrier phase per exchange; in FP64 the operands' traffic (N = 32: 78,000 L2
+// requests per us, 27% of them misses, 3.2 TB/s of HBM, VALU 47%; N = 64: 1.45 MB of HBM a product, 5.8 TB/s, VALU
+// 36%).  A term pair costs 16 applications and 16 pruned IFFT2 of three quarters of a transform (packed pairs: 8
+// and 4) instead of 32 (16) applications.  Strang steps term by term -> in pairs, with k_assemble and the batched
+// loads that came with them: FP32 N = 64, 512 cells 327.9 -> 204.2 ms; FP64 N = 32, 128 cells 59.9 -> 44.4 ms; FP64
+// N = 64, 16 cells 62.5 -> 43.1 ms; FP32 N = 128, 32 cells 76.6 -> 49.5 ms.
 #pragma once
 #include "qbf_kernels.hip"
 
@@ -264,7 +266,7 @@ __global__ __launch_bounds__(T, (FOLD_WPE<R, N>)) void k_i3fold(I3FoldArgs a)
 // acc [cell][2][2 nchunk], D [cell][2][2 nchunk nblk] (partial sums over p, over J, the term ranges and
 // blocks).
 // Four workgroups share a cell's S and F grids, as many cells as an XCD's L2 holds (with both p in one
-// workgroup: 457 KB of HBM traffic per product instead of 115, FP32, N = 64).
+// workgroup: 457 KB of HBM traffic per product instead of 115 when the split was chosen, FP32, N = 64; 179 now).
 template <typename R, int N, int T, bool SP>
 __global__ __launch_bounds__(T, (FOLD_WPE<R, N>)) void k_i3fold_pair(I3FoldArgs a)
 {
