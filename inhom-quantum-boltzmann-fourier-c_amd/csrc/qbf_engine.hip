@@ -6,8 +6,11 @@
 //   What_c = FFT2(pad W_c)                                   k_padfft
 //   Ahat_g = FFT2(sum_i psi1_i .* IFFT2(Fhat .* FFT2(pad(Phi_i .* W_g))))   k_i1acc  (Cc, I4)
 //   S_i    = sum_q FFT2(pad(psi1_q W_i)) .* FFT2(pad(psi2_q W_i))           k_i2acc  (I2)
-//   acc_j  = sum_q sum_i eta_i F_iq .* K_q[What_i .* F_jq]                   k_padfft + k_i3acc (I3)
-//   C_j    = Extract(IFFT2( linear combination ))                           k_combine
+//   acc_j  = sum_q sum_i eta_i F_iq .* K_q[What_i .* F_jq]                   k_padfft + k_i3fold (I3; k_i3acc
+//            for tables without mirrored terms, single integrals and the BF16 split engine)
+//   D_j    = the mirrored terms' part of it, on the N x N box in frequency space       k_i3fold, k_sum_mirror
+//   V_j    = linear combination of What, Ahat, S and acc                     k_assemble
+//   C_j    = Extract(IFFT2(V_j)) - eta2_j D_j / P^4                          k_combine
 // The reassociation is exact: the I1 weights of the reference are duplicated over
 // one angle (src/quadrature.c:192-195, 213-234) so the J^2 terms are summed into J
 // groups with Phi_i = sum_j psiR2_ij; the final convolution and Extract of every
@@ -352,8 +355,8 @@ struct EngineT final : public qbf_engine {
 	DevBuf Wmid, WF, WF2, Wt1, Wt2, src3;
 	DevBuf Wpk, WhatP, reim;          // paired path: packed spectra, their padded transforms, realness
 	// device memory for the F grids of one I3 launch (it sets the quadrature terms per launch; the
-	// accumulators cross HBM once per launch).  Measured at N = 64 on 512 cells: FP32 8 GiB (64 terms
-	// per launch) 329 ms per step against 336 ms with 2 GiB; FP64 16 GiB no faster than 2 GiB.
+	// accumulators cross HBM once per launch).  Measured at N = 64 on 512 cells, term by term: FP32 8 GiB (64
+	// terms per launch) 329 ms per step against 336 ms with 2 GiB; FP64 16 GiB no faster than 2 GiB.
 	size_t fBudget = std::is_same<R, float>::value ? ((size_t)8 << 30) : ((size_t)2 << 30);
 
 	int init()

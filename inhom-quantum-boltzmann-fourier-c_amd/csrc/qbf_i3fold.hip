@@ -112,8 +112,8 @@ __device__ __forceinline__ void k_apply(cx<R>* v, const R* ps, const XP& X, cons
 // The mirror sums of FP32 grids are kept per block of DBLOCK terms (added in FP64 afterwards,
 // k_sum_mirror): their low frequencies are sums over the whole grid, and 256 terms added in FP32 there
 // tripled the error of a step.  Error of a step with its conservation correction, N = 64, 512 and 300 cells (term
-// by term 2.20e-10, 1.91e-10): blocks of 32: 2.11e-10, 1.93e-10; 16: 2.08e-10, 1.85e-10; 8: 2.07e-10, 1.81e-10.  The
-// step of 512 cells takes 189.0, 189.6 and 190.3 ms (complex grids, 256 cells: 203.6, 203.9 and 211.4).
+// by term 2.20e-10, 1.91e-10): blocks of 32: 2.11e-10, 1.94e-10; 16: 2.08e-10, 1.85e-10; 8: 2.07e-10, 1.81e-10.  The
+// step of 512 cells takes 189.2, 189.8 and 190.5 ms (complex grids, 256 cells: 203.6, 203.9 and 211.4).
 template <typename R> constexpr int DBLOCK = sizeof(R) == 4 ? 16 : 1 << 30;
 
 // Workgroup -> (cell, group, term range) of the fold kernels; nmir: see I3FoldArgs::terms.  none: the launch
